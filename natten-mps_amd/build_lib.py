@@ -28,7 +28,7 @@ BIND = os.path.join(HERE, "natten_mps_amd", BIND_NAME + ".so")
 CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["na_generic.hip", "na_mfma.hip", "na_lean.hip", "na_global.hip", "na_rpb.hip", "na_profile.hip", "na_capi.hip"]
+SOURCES = ["na_generic.hip", "na_mfma.hip", "na_lean.hip", "na_band.hip", "na_global.hip", "na_rpb.hip", "na_profile.hip", "na_capi.hip"]
 
 FLAGS = [
     "--offload-arch=gfx950",

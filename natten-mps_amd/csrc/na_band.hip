@@ -1,0 +1,855 @@
+// Band kernels (gfx950, bf16 / fp16, head dim 32 / 64 / 128, stride 1):
+// fused forward, backward dQ and backward dK/dV for windows whose staged
+// union is too large for the other tile kernels to hold at once.
+//
+// The 8x8 tile kernels (na_lean.hip) stop at kernel 9, and the general tile
+// kernels (na_mfma.hip) stage a whole plane of the union: at kernel 13 x 13
+// and head dim 64 only a 16-query tile fits, which stages 23 rows of K and V
+// per query and runs one wave per workgroup.  Here a workgroup of 8 waves
+// owns 128 queries (keys) of one class triple and one (batch, head) -- a box
+// of 128 / T2 rows of T2 = 8 or 16 columns, 16 items per wave -- and walks
+// the union a band of NC chunks (32 slots each) at a time, so that LDS holds
+// two bands whatever the kernel size:
+//
+// * The next band's rows are requested into registers before the current
+//   band is computed, and stored to the other LDS buffer after it: loads
+//   overlap the products, with one barrier per band.  (Loads straight to
+//   LDS cannot be used that way: the compiler waits for all of them before
+//   any LDS read.)
+// * A union row takes SL slots: 32 (kernels over 9 in-plane: a 16-column
+//   tile's union spans up to 15 + K columns), one row per chunk.
+// * A wave computes only the chunks that its own items' windows reach; its
+//   online softmax rescales once per band.
+//
+// What bounds it: LDS reads (a chunk's 8 KB of K and V rows per 16 queries)
+// and the latency of a wave's score -> maximum -> exponential -> product
+// chain; 8 waves and bands of 4 rows measured as fast as 4 waves or bands of
+// 2 (16 waves: 28 % slower).  Measured, general tile (or vector) kernels ->
+// these: 13 x 13, head dim 64, fp16, 4 x 135 x 241, 8 heads, forward 2350 ->
+// 334 us; bf16 4 x 64 x 64, 8 heads, forward 275 -> 49, dQ 981 -> 124, dK/dV
+// 968 -> 105 us; head dim 128, 4 heads 501 / 1043 / 998 -> 53 / 139 / 107 us;
+// 11 x 11, head dim 32, 4 x 61 x 130, 8 heads 103 / 139 / 128 -> 57 / 128 /
+// 91 us.
+//
+// The geometry is computed in the kernel (no tables): every call, captured
+// or not, runs the same code.  MFMA lane layouts, the swizzle and the masks
+// are those of na_mfma.hip.
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+
+#include "na_tile.h"
+
+namespace na {
+
+namespace {
+
+constexpr int kBandWaves = 8;
+constexpr int kBandThreads = 64 * kBandWaves;
+constexpr uint32_t kBandOOR = 0x40000000u;  // past every staged plane (planes < 2^30 bytes)
+
+// Chunks per band: two 16-byte pieces per thread and operand at head dims
+// 64 and 128, one at 32.
+template <int D>
+constexpr int kBandChunks = D == 128 ? 2 : 4;
+
+// LDS bytes of one operand's band, and of one buffer of two operands.
+template <int D>
+constexpr int kBandOp = kBandChunks<D> * 32 * D * 2;
+
+// Tile shape: log2 of the box's columns and rows, tiles per class and axis,
+// and the divisors that decode a workgroup's index.
+struct BandGeo {
+    int sh1, sh2;
+    int lenmod[3];
+    FastDiv heads, tiles, rep, nt[3], dil[3];
+};
+
+template <typename T>
+struct BandArgs {
+    Prob p;
+    BandGeo g;
+    const T *q, *k, *v, *o, *dout;
+    const float *lse, *dlse, *delta;
+    T *out, *dq, *dk, *dv;
+    float *lse_out, *delta_out;
+    LayK lq, lk, lv, lo, ldo, ldq, ldk, ldv, ll, lde, ldl;
+    uint32_t ab, bb;  // byte ranges of one plane of the two staged operands
+};
+
+// A workgroup's tile: batch, head (kv head on the key side), the tile's
+// geometry per axis (with this wave's box), residues.
+struct BandTile {
+    int b, h, r[3];
+    AxisGeo a[3];
+};
+
+template <bool KEY>
+__device__ __forceinline__ BandTile band_tile(const Prob& p, const BandGeo& g, int wave) {
+    BandTile t;
+    const int x = xcd_block(blockIdx.x, gridDim.x);
+    const int bt = fdiv(x, g.heads);
+    t.h = x - bt * static_cast<int>(g.heads.d);
+    t.b = fdiv(bt, g.tiles);
+    int s = bt - t.b * static_cast<int>(g.tiles.d);
+    int tt[3];
+#pragma unroll
+    for (int a = 2; a >= 0; --a) {
+        int q = fdiv(s, g.nt[a]);
+        tt[a] = s - q * static_cast<int>(g.nt[a].d);
+        s = q;
+        q = fdiv(s, g.dil[a]);
+        t.r[a] = s - q * static_cast<int>(g.dil[a].d);
+        s = q;
+    }
+    const int T[3] = {(kBandWaves * 16) >> (g.sh1 + g.sh2), 1 << g.sh1, 1 << g.sh2};
+    // the wave's items 16 w .. 16 w + 15 in row-major order: whole rows of
+    // one depth (T2 <= 16)
+    const int f0 = wave * 16;
+    const int e0 = f0 >> (g.sh1 + g.sh2), e1 = (f0 >> g.sh2) & (T[1] - 1);
+    const int wl[3] = {e0, e1, 0}, wh[3] = {e0, e1 + (16 >> g.sh2) - 1, T[2] - 1};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const Axis& A = p.ax[a];
+        t.a[a] = axis_geometry(A.len, A.k, A.dil, A.causal, g.lenmod[a], 1, A.len, T[a], tt[a], t.r[a], wl[a], wh[a],
+                               KEY, g.dil[a]);
+    }
+    return t;
+}
+
+__device__ __forceinline__ ClassAxis band_class(const Axis& A, const AxisGeo& g) {
+    return ClassAxis{g.n, A.k, A.k >> 1, g.B, A.causal, 1};
+}
+
+// The lane's item: validity, position, and its window (key side: attending
+// queries) relative to the union -- rows [rlo, rlo + rn) and columns [clo,
+// clo + cn); rn = 0 for lanes past the tile.
+struct BandLane {
+    bool valid;
+    int pos[3], rlo, rn, clo, cn;
+};
+
+template <bool KEY>
+__device__ __forceinline__ BandLane band_lane(const Prob& p, const BandGeo& g, const BandTile& t, int wave, int col) {
+    const int f = wave * 16 + col;
+    const int e[3] = {f >> (g.sh1 + g.sh2), (f >> g.sh2) & ((1 << g.sh1) - 1), f & ((1 << g.sh2) - 1)};
+    BandLane l;
+    l.valid = e[0] < t.a[0].E && e[1] < t.a[1].E && e[2] < t.a[2].E;
+    int lo[3], hi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int j = t.a[a].J + (l.valid ? e[a] : 0);
+        l.pos[a] = t.r[a] + j * p.ax[a].dil;
+        item_box(band_class(p.ax[a], t.a[a]), j, KEY, lo[a], hi[a]);
+    }
+    l.rlo = lo[1] - t.a[1].lo;
+    l.rn = l.valid ? imax(hi[1] - lo[1] + 1, 0) : 0;
+    l.clo = lo[2] - t.a[2].lo;
+    l.cn = imax(hi[2] - lo[2] + 1, 0);
+    return l;
+}
+
+// Column mask of the lane's 8 slots of a chunk, as the score product's
+// accumulator input.
+template <int SL>
+__device__ __forceinline__ void band_colbias(const BandLane& l, int grp, f32x4_t (&bias)[2]) {
+    const int c0 = 8 * (grp & (SL / 8 - 1)) - l.clo;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        bias[e >> 2][e & 3] = static_cast<unsigned>(c0 + e) < static_cast<unsigned>(l.cn) ? 0.f : -INFINITY;
+}
+
+template <typename T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t band_rsrc(const T* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), static_cast<short>(0), static_cast<int>(bytes),
+                                             0x00020000);
+}
+
+// Staging of two operands' bands: thread t moves 16-byte piece t % P of
+// slots t / P + j * SPT, j < NP, of each operand (SPT slots per round of the
+// workgroup).  Columns past the union and rows past it load from outside the
+// buffer (zeros).  A round covers whole union rows, or 1 / CPR of one.
+template <typename T, int D, int SL>
+struct BandStage {
+    static constexpr int P = D / 8, NP = kBandChunks<D> * 32 * P / kBandThreads, SPT = kBandThreads / P;
+    static constexpr int CPR = SPT >= SL ? 1 : SL / SPT;            // rounds per union row
+    static constexpr int RB = kBandChunks<D> * 32 / SL;             // union rows per band
+    static_assert(SPT % SL == 0 || SL % SPT == 0, "rounds of whole rows or equal parts of one");
+    static_assert((P * (SPT < SL ? SPT : SL)) % 64 == 0, "a wave stays in one union row");
+    static_assert(SPT % 16 == 0 && (SPT % 32 == 0 || CPR == 2), "the swizzle repeats every 32 slots");
+    int row0, dst[CPR];           // first union row (wave-uniform); LDS byte offset of rounds 0 .. CPR - 1
+    uint32_t ca[CPR], cb[CPR];    // lane part of the global offsets
+    int base_a, base_b, step_a, step_b;
+    uint4 ra[NP], rb[NP];
+
+    __device__ __forceinline__ void init(const Prob& p, const BandTile& t, const LayK& la, const LayK& lb) {
+        const int tid = threadIdx.x, pp = tid % P, slot0 = tid / P;
+        row0 = __builtin_amdgcn_readfirstlane(slot0 / SL);
+        const int d1 = p.ax[1].dil, d2 = p.ax[2].dil;
+#pragma unroll
+        for (int r = 0; r < CPR; ++r) {
+            const int slot = slot0 + r * SPT, c = slot % SL;
+            dst[r] = slot * D * 2 + ((pp ^ swz<D>(slot)) << 4);
+            const bool in = c < t.a[2].U;
+            ca[r] = in ? static_cast<uint32_t>(c * d2 * la.s2 * 2 + pp * 16) : kBandOOR;
+            cb[r] = in ? static_cast<uint32_t>(c * d2 * lb.s2 * 2 + pp * 16) : kBandOOR;
+        }
+        const int p1 = t.r[1] + t.a[1].lo * d1, p2 = t.r[2] + t.a[2].lo * d2;
+        base_a = (p1 * la.s1 + p2 * la.s2) * 2;
+        base_b = (p1 * lb.s1 + p2 * lb.s2) * 2;
+        step_a = d1 * la.s1 * 2;
+        step_b = d1 * lb.s1 * 2;
+    }
+
+    // request band `bi` of the planes at pa / pb
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t pa, __amdgpu_buffer_rsrc_t pb, int bi, int U1) {
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const int row = bi * RB + row0 + j * SPT / SL, r = j % CPR;
+            const uint32_t oa = row < U1 ? static_cast<uint32_t>(base_a + row * step_a) : kBandOOR;
+            const uint32_t ob = row < U1 ? static_cast<uint32_t>(base_b + row * step_b) : kBandOOR;
+            ra[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(pa, ca[r] + oa, 0, 0));
+            rb[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(pb, cb[r] + ob, 0, 0));
+        }
+    }
+
+    // store the requested band into the buffer at `buf`
+    __device__ __forceinline__ void store(unsigned char* buf) const {
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            unsigned char* x = buf + dst[j % CPR] + j / CPR * (CPR * kBandThreads * 16);
+            *reinterpret_cast<uint4*>(x) = ra[j];
+            *reinterpret_cast<uint4*>(x + kBandOp<D>) = rb[j];
+        }
+    }
+};
+
+// LDS byte offsets (from an operand's band) of the lane's A operands of
+// chunk 0: the score product's (rows = slots) and, transposed, the product's
+// over slots (na_tile.h, score_chunk and accumulate_chunk).
+template <int D>
+struct BandOff {
+    int a[2][D / 32], t[2][D / 16];
+    __device__ __forceinline__ void init(int lane) {
+        const int col = lane & 15, grp = lane >> 4;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int slot = 8 * (col >> 2) + 4 * b + (col & 3);
+#pragma unroll
+            for (int ks = 0; ks < D / 32; ++ks) a[b][ks] = slot * D * 2 + (((ks * 4 + grp) ^ swz<D>(slot)) << 4);
+        }
+#pragma unroll
+        for (int hi = 0; hi < 2; ++hi) {
+            const int r = 8 * grp + (col >> 2) + 4 * hi;
+#pragma unroll
+            for (int db = 0; db < D / 16; ++db)
+                t[hi][db] = r * D * 2 + (((2 * db + ((col & 3) >> 1)) ^ swz<D>(r)) << 4) + (col & 1) * 8;
+        }
+    }
+};
+
+template <typename T, int D>
+__device__ __forceinline__ void band_score(const unsigned char* X, const BandOff<D>& o, int c,
+                                           const uint4 (&frag)[D / 32], const f32x4_t (&bias)[2], f32x4_t (&out)[2]) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        f32x4_t acc = bias[b];
+#pragma unroll
+        for (int ks = 0; ks < D / 32; ++ks)
+            acc = Mma<T>::run(*reinterpret_cast<const uint4*>(X + o.a[b][ks] + c * 32 * D * 2), frag[ks], acc);
+        out[b] = acc;
+    }
+}
+
+template <typename T, int D>
+__device__ __forceinline__ void band_accumulate(const unsigned char* X, const BandOff<D>& o, int c, uint4 packed,
+                                                f32x4_t (&acc)[D / 16]) {
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db) {
+        const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(X + o.t[0][db] + c * 32 * D * 2));
+        const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(X + o.t[1][db] + c * 32 * D * 2));
+        const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+        acc[db] = Mma<T>::run(make_uint4(l2.x, l2.y, h2.x, h2.y), packed, acc[db]);
+    }
+}
+
+// Walk over the union: bands of a plane, then the next plane (and, key
+// side, the next q head).
+struct BandWalk {
+    int bi, u0, h;
+};
+
+// Waves per SIMD the kernels are built for: two workgroups of 8 waves fit a
+// CU's LDS; at head dim 128 the backward kernels need the registers of one.
+constexpr int band_waves(int D, bool backward) { return D == 128 && backward ? 2 : 4; }
+#define NA_BAND_OCC(D, BWD) __attribute__((amdgpu_waves_per_eu(band_waves(D, BWD))))
+
+template <typename T, int D>
+__device__ __forceinline__ void band_redo_fwd(const void* kargs, int b, int h, int hk, int p0, int p1, int p2, int grp) {
+    const BandArgs<T>& A = *static_cast<const BandArgs<T>*>(kargs);
+    const int pos[3] = {p0, p1, p2};
+    ExactAxis x[3];
+    for (int a = 0; a < 3; ++a) x[a] = exact_axis(A.p.ax[a], pos[a]);
+    f32x4_t acc[D / 16];
+    float lse_v;
+    exact_forward<T, D>(A.p.scale, x, bh_ptr(A.q, A.lq, b, h) + vol_off(A.lq, pos), bh_ptr(A.k, A.lk, b, hk),
+                        strides3(A.lk), bh_ptr(A.v, A.lv, b, hk), strides3(A.lv), grp, acc, lse_v);
+    store_rows<T, D>(bh_ptr(A.out, A.lo, b, h), vol_off(A.lo, pos), grp, acc, 1.f);
+    if (grp == 0) bh_ptr(A.lse_out, A.ll, b, h)[vol_off(A.ll, pos)] = lse_v;
+}
+
+template <typename T, int D, int SL>
+__global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd(BandArgs<T> args) {
+    constexpr int NC = kBandChunks<D>, RPC = 32 / SL, BUF = 2 * kBandOp<D>;
+    const Prob& p = args.p;
+    unsigned char* smem = lds_base();
+    const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const BandTile t = band_tile<false>(p, args.g, wave);
+    if (!(t.a[0].tile_ok && t.a[1].tile_ok && t.a[2].tile_ok)) return;
+    const int hk = args.g.rep.d == 1 ? t.h : fdiv(t.h, args.g.rep);
+    const T* kb = bh_ptr(args.k, args.lk, t.b, hk);
+    const T* vb = bh_ptr(args.v, args.lv, t.b, hk);
+    BandStage<T, D, SL> st;
+    st.init(p, t, args.lk, args.lv);
+    const int U0 = t.a[0].U, U1 = t.a[1].U, nb = (U1 + st.RB - 1) / st.RB;
+    const auto load = [&](int u0, int bi) {
+        const int p0 = t.r[0] + (t.a[0].lo + u0) * p.ax[0].dil;
+        st.load(band_rsrc(kb + p0 * args.lk.s0, args.ab), band_rsrc(vb + p0 * args.lv.s0, args.bb), bi, U1);
+    };
+    load(0, 0);
+
+    const BandLane ln = band_lane<false>(p, args.g, t, wave, col);
+    uint4 qf[D / 32];
+    load_frags<T, D>(bh_ptr(args.q, args.lq, t.b, t.h), vol_off(args.lq, ln.pos), ln.valid, grp, qf);
+    f32x4_t cb[2];
+    band_colbias<SL>(ln, grp, cb);
+    BandOff<D> off;
+    off.init(lane);
+    const float sc2 = p.scale * kLog2e;
+    const bool wave_ok = t.a[0].wave_ok && t.a[1].wave_ok && t.a[2].wave_ok;
+    // the wave's chunks of a plane, and its planes
+    const int wc0 = t.a[1].glo / RPC, wc1 = wave_ok ? t.a[1].ghi / RPC : -1;
+    const int w0 = t.a[0].glo, w1 = t.a[0].ghi;
+    const uint4 ones = make_uint4(Mma<T>::kOnes, Mma<T>::kOnes, Mma<T>::kOnes, Mma<T>::kOnes);
+
+    f32x4_t acc[D / 16], lacc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY;
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    int u0 = 0, bi = 0;
+    // one band: publish it in buffer B, request the next one, compute
+    const auto step = [&](auto BC) {
+        constexpr int B = decltype(BC)::value;
+        st.store(smem + B * BUF);
+        lds_publish_barrier();
+        const int cu = u0, cbi = bi;
+        if (++bi == nb) {
+            bi = 0;
+            ++u0;
+        }
+        const bool more = u0 < U0;
+        if (more) load(u0, bi);
+        const int c0 = cbi * NC;
+        if (cu >= w0 && cu <= w1 && c0 + NC - 1 >= wc0 && c0 <= wc1) {
+            const unsigned char* Kb = smem + B * BUF;
+            const unsigned char* Vb = Kb + kBandOp<D>;
+            f32x4_t s[NC][2];
+            bool rv[NC];
+            float cm = -INFINITY;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                if (c0 + c >= wc0 && c0 + c <= wc1) {
+                    const int row = (c0 + c) * RPC + (RPC == 2 ? grp >> 1 : 0) - ln.rlo;
+                    rv[c] = static_cast<unsigned>(row) < static_cast<unsigned>(ln.rn);
+                    band_score<T, D>(Kb, off, c, qf, cb, s[c]);
+                    cm = fmaxp(cm, rv[c] ? max8(s[c]) : -INFINITY);
+                }
+            }
+            const float mnew = fmaxp(m, max_rows(cm) * sc2);
+            const float mref = mnew == -INFINITY ? 0.f : mnew;
+            const float corr = __builtin_amdgcn_exp2f(m - mref);
+            m = mnew;
+            lacc *= corr;
+#pragma unroll
+            for (int db = 0; db < D / 16; ++db) acc[db] *= corr;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                if (c0 + c >= wc0 && c0 + c <= wc1) {
+                    const float o = rv[c] ? -mref : -INFINITY;
+#pragma unroll
+                    for (int bb = 0; bb < 2; ++bb)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) s[c][bb][i] = __builtin_amdgcn_exp2f(fmaf(s[c][bb][i], sc2, o));
+                    const uint4 pk = pack8<T>(s[c]);
+                    band_accumulate<T, D>(Vb, off, c, pk, acc);
+                    lacc = Mma<T>::run(ones, pk, lacc);
+                }
+            }
+        }
+        return more;
+    };
+#pragma unroll 1
+    while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{})) {
+    }
+    const float lsum = lacc[0];
+    const bool redo = ln.valid && item_nonfinite(lane_sum(acc, lsum));
+    if (ln.valid) {
+        store_rows<T, D>(bh_ptr(args.out, args.lo, t.b, t.h), vol_off(args.lo, ln.pos), grp, acc, 1.f / lsum);
+        if (grp == 0) bh_ptr(args.lse_out, args.ll, t.b, t.h)[vol_off(args.ll, ln.pos)] = (m + __log2f(lsum)) * kLn2;
+    }
+    if (redo)
+        band_redo_fwd<T, D>(kernargs(), t.b, t.h, hk, opaque(ln.pos[0]), opaque(ln.pos[1]), opaque(ln.pos[2]), grp);
+}
+
+// Backward, query side: as k_bwd_q_mfma.  2-D: a first walk takes delta =
+// sum over the window of P dP (= dO . O) from the kernel's own products
+// (where that is not finite, dO . O from the rows), a second one forms dS =
+// P (dP - delta) and dq.
+template <typename T, int D>
+__device__ __forceinline__ void band_redo_bwd_q(const void* kargs, int b, int h, int hk, int p0, int p1, int p2,
+                                                int grp) {
+    const BandArgs<T>& A = *static_cast<const BandArgs<T>*>(kargs);
+    const int pos[3] = {p0, p1, p2};
+    ExactAxis x[3];
+    for (int a = 0; a < 3; ++a) x[a] = exact_axis(A.p.ax[a], pos[a]);
+    const T* do_row = bh_ptr(A.dout, A.ldo, b, h) + vol_off(A.ldo, pos);
+    float di = exact_dot<T, D>(do_row, bh_ptr(A.o, A.lo, b, h) + vol_off(A.lo, pos));
+    if (A.dlse) di -= bh_ptr(A.dlse, A.ldl, b, h)[vol_off(A.ldl, pos)];
+    f32x4_t acc[D / 16];
+    exact_backward_q<T, D>(A.p.scale, x, bh_ptr(A.q, A.lq, b, h) + vol_off(A.lq, pos), do_row,
+                           bh_ptr(A.lse, A.ll, b, h)[vol_off(A.ll, pos)], di, bh_ptr(A.k, A.lk, b, hk),
+                           strides3(A.lk), bh_ptr(A.v, A.lv, b, hk), strides3(A.lv), grp, acc);
+    store_rows<T, D>(bh_ptr(A.dq, A.ldq, b, h), vol_off(A.ldq, pos), grp, acc, A.p.scale);
+}
+
+template <typename T, int D, int SL>
+__global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_q(BandArgs<T> args) {
+    constexpr int NC = kBandChunks<D>, RPC = 32 / SL, BUF = 2 * kBandOp<D>;
+    const Prob& p = args.p;
+    unsigned char* smem = lds_base();
+    const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const BandTile t = band_tile<false>(p, args.g, wave);
+    if (!(t.a[0].tile_ok && t.a[1].tile_ok && t.a[2].tile_ok)) return;
+    const int hk = args.g.rep.d == 1 ? t.h : fdiv(t.h, args.g.rep);
+    const T* kb = bh_ptr(args.k, args.lk, t.b, hk);
+    const T* vb = bh_ptr(args.v, args.lv, t.b, hk);
+    BandStage<T, D, SL> st;
+    st.init(p, t, args.lk, args.lv);
+    const int U1 = t.a[1].U, nb = (U1 + st.RB - 1) / st.RB;
+    const int p0 = t.r[0] + t.a[0].lo * p.ax[0].dil;
+    const auto load = [&](int bi) {
+        st.load(band_rsrc(kb + p0 * args.lk.s0, args.ab), band_rsrc(vb + p0 * args.lv.s0, args.bb), bi, U1);
+    };
+    load(0);
+
+    const BandLane ln = band_lane<false>(p, args.g, t, wave, col);
+    uint4 qf[D / 32], gf[D / 32];
+    load_frags<T, D>(bh_ptr(args.q, args.lq, t.b, t.h), vol_off(args.lq, ln.pos), ln.valid, grp, qf);
+    load_frags<T, D>(bh_ptr(args.dout, args.ldo, t.b, t.h), vol_off(args.ldo, ln.pos), ln.valid, grp, gf);
+    const float L2 = ln.valid ? bh_ptr(args.lse, args.ll, t.b, t.h)[vol_off(args.ll, ln.pos)] * kLog2e : 0.f;
+    const float dl = ln.valid && args.dlse ? bh_ptr(args.dlse, args.ldl, t.b, t.h)[vol_off(args.ldl, ln.pos)] : 0.f;
+    f32x4_t cb[2];
+    band_colbias<SL>(ln, grp, cb);
+    BandOff<D> off;
+    off.init(lane);
+    const float sc2 = p.scale * kLog2e;
+    const bool wave_ok = t.a[0].wave_ok && t.a[1].wave_ok && t.a[2].wave_ok;
+    const int wc0 = t.a[1].glo / RPC, wc1 = wave_ok ? t.a[1].ghi / RPC : -1;
+    const f32x4_t zero[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+
+    f32x4_t acc[D / 16];
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float part = 0.f, di = 0.f;
+    int bi = 0, pass = 0;
+    const auto step = [&](auto BC) {
+        constexpr int B = decltype(BC)::value;
+        st.store(smem + B * BUF);
+        lds_publish_barrier();
+        const int c0 = bi * NC, cpass = pass;
+        if (++bi == nb) {
+            bi = 0;
+            ++pass;
+        }
+        const bool more = pass < 2;
+        if (more) load(bi);
+        const unsigned char* Kb = smem + B * BUF;
+        const unsigned char* Vb = Kb + kBandOp<D>;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if (c0 + c < wc0 || c0 + c > wc1) continue;
+            const int row = (c0 + c) * RPC + (RPC == 2 ? grp >> 1 : 0) - ln.rlo;
+            const float o = static_cast<unsigned>(row) < static_cast<unsigned>(ln.rn) ? -L2 : -INFINITY;
+            f32x4_t s[2], dp[2];
+            band_score<T, D>(Kb, off, c, qf, cb, s);
+            band_score<T, D>(Vb, off, c, gf, zero, dp);
+            if (cpass == 0) {
+                part = delta_part(s, dp, sc2, o, part);
+            } else {
+#pragma unroll
+                for (int bb = 0; bb < 2; ++bb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        s[bb][i] = __builtin_amdgcn_exp2f(fmaf(s[bb][i], sc2, o)) * (dp[bb][i] - di);
+                band_accumulate<T, D>(Kb, off, c, pack8<T>(s), acc);
+            }
+        }
+        if (pass == 1 && cpass == 0) {
+            di = sum_rows(part) - dl;
+            if (ln.valid && !(__builtin_fabsf(di) <= __FLT_MAX__))
+                di = exact_dot<T, D>(bh_ptr(args.dout, args.ldo, t.b, t.h) + vol_off(args.ldo, ln.pos),
+                                     bh_ptr(args.o, args.lo, t.b, t.h) + vol_off(args.lo, ln.pos)) -
+                     dl;
+            if (ln.valid && grp == 0) bh_ptr(args.delta_out, args.lde, t.b, t.h)[vol_off(args.lde, ln.pos)] = di;
+        }
+        return more;
+    };
+#pragma unroll 1
+    while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{})) {
+    }
+    const bool redo = ln.valid && item_nonfinite(lane_sum(acc, 0.f));
+    if (ln.valid) store_rows<T, D>(bh_ptr(args.dq, args.ldq, t.b, t.h), vol_off(args.ldq, ln.pos), grp, acc, p.scale);
+    if (redo)
+        band_redo_bwd_q<T, D>(kernargs(), t.b, t.h, hk, opaque(ln.pos[0]), opaque(ln.pos[1]), opaque(ln.pos[2]), grp);
+}
+
+// Backward, key side: as k_bwd_kv_mfma; the walk covers every q head of the
+// kv head's group.  Per slot of a band: -lse log2 e and -delta in LDS, and 8
+// -inf entries that lanes failing the row test read instead.
+template <typename T, int D>
+__device__ __forceinline__ void band_redo_bwd_kv(const void* kargs, int b, int hk, int p0, int p1, int p2, int grp) {
+    const BandArgs<T>& A = *static_cast<const BandArgs<T>*>(kargs);
+    const int pos[3] = {p0, p1, p2};
+    ExactAxis x[3];
+    for (int a = 0; a < 3; ++a) x[a] = exact_axis(A.p.ax[a], pos[a]);
+    const T* kr = bh_ptr(A.k, A.lk, b, hk) + vol_off(A.lk, pos);
+    const T* vr = bh_ptr(A.v, A.lv, b, hk) + vol_off(A.lv, pos);
+    const int rep = A.p.rep;
+    f32x4_t g[D / 16];
+    exact_zero(g);
+#pragma unroll 1
+    for (int h = hk * rep; h < (hk + 1) * rep; ++h)
+        exact_backward_kv<T, D, true>(A.p.scale, x, kr, vr, bh_ptr(A.q, A.lq, b, h), strides3(A.lq),
+                                      bh_ptr(A.dout, A.ldo, b, h), strides3(A.ldo), bh_ptr(A.lse, A.ll, b, h),
+                                      strides3(A.ll), bh_ptr(A.delta, A.lde, b, h), strides3(A.lde), grp, g);
+    store_rows<T, D>(bh_ptr(A.dv, A.ldv, b, hk), vol_off(A.ldv, pos), grp, g, 1.f);
+    exact_zero(g);
+#pragma unroll 1
+    for (int h = hk * rep; h < (hk + 1) * rep; ++h)
+        exact_backward_kv<T, D, false>(A.p.scale, x, kr, vr, bh_ptr(A.q, A.lq, b, h), strides3(A.lq),
+                                       bh_ptr(A.dout, A.ldo, b, h), strides3(A.ldo), bh_ptr(A.lse, A.ll, b, h),
+                                       strides3(A.ll), bh_ptr(A.delta, A.lde, b, h), strides3(A.lde), grp, g);
+    store_rows<T, D>(bh_ptr(A.dk, A.ldk, b, hk), vol_off(A.ldk, pos), grp, g, A.p.scale);
+}
+
+template <typename T, int D, int SL>
+__global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_kv(BandArgs<T> args) {
+    constexpr int NC = kBandChunks<D>, RPC = 32 / SL, BUF = 2 * kBandOp<D>, NS = NC * 32;
+    const Prob& p = args.p;
+    unsigned char* smem = lds_base();
+    float* scal = reinterpret_cast<float*>(smem + 2 * BUF);  // per buffer NS (-lse), NS (-delta); then 8 x -inf
+    const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const BandTile t = band_tile<true>(p, args.g, wave);
+    if (!(t.a[0].tile_ok && t.a[1].tile_ok && t.a[2].tile_ok)) return;
+    const BandLane ln = band_lane<true>(p, args.g, t, wave, col);
+    const int U0 = t.a[0].U, U1 = t.a[1].U, U2 = t.a[2].U;
+    f32x4_t gk[D / 16], gv[D / 16];
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db) gk[db] = gv[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const auto store = [&]() {
+        store_rows<T, D>(bh_ptr(args.dk, args.ldk, t.b, t.h), vol_off(args.ldk, ln.pos), grp, gk, p.scale);
+        store_rows<T, D>(bh_ptr(args.dv, args.ldv, t.b, t.h), vol_off(args.ldv, ln.pos), grp, gv, 1.f);
+    };
+    if (U0 == 0 || U1 == 0 || U2 == 0) {  // no query attends these keys
+        if (ln.valid) store();
+        return;
+    }
+    const int rep = static_cast<int>(args.g.rep.d);
+    BandStage<T, D, SL> st;
+    st.init(p, t, args.lq, args.ldo);
+    const int nb = (U1 + st.RB - 1) / st.RB;
+    // the thread's slot of a band (threads past NS load slot 0's scalars and drop them)
+    const int sslot = threadIdx.x < NS ? static_cast<int>(threadIdx.x) : 0;
+    const int srow = sslot / SL, scol = sslot % SL;
+    const bool sin = scol < U2;
+    const int q2 = t.r[2] + (t.a[2].lo + (sin ? scol : 0)) * p.ax[2].dil;
+    const int sl2 = q2 * args.ll.s2, sd2 = q2 * args.lde.s2;
+    float pl, pd;
+    bool pin;
+    int h = t.h * rep, u0 = 0, bi = 0;
+    const auto load = [&]() {
+        const int p0 = t.r[0] + (t.a[0].lo + u0) * p.ax[0].dil;
+        const int row = bi * st.RB + srow;
+        pin = sin && row < U1;
+        const int p1 = t.r[1] + (t.a[1].lo + (pin ? row : 0)) * p.ax[1].dil;
+        pl = (bh_ptr(args.lse, args.ll, t.b, h) + p0 * args.ll.s0)[p1 * args.ll.s1 + sl2];
+        pd = (bh_ptr(args.delta, args.lde, t.b, h) + p0 * args.lde.s0)[p1 * args.lde.s1 + sd2];
+        st.load(band_rsrc(bh_ptr(args.q, args.lq, t.b, h) + p0 * args.lq.s0, args.ab),
+                band_rsrc(bh_ptr(args.dout, args.ldo, t.b, h) + p0 * args.ldo.s0, args.bb), bi, U1);
+    };
+    load();
+
+    uint4 kf[D / 32], vf[D / 32];
+    load_frags<T, D>(bh_ptr(args.k, args.lk, t.b, t.h), vol_off(args.lk, ln.pos), ln.valid, grp, kf);
+    load_frags<T, D>(bh_ptr(args.v, args.lv, t.b, t.h), vol_off(args.lv, ln.pos), ln.valid, grp, vf);
+    if (threadIdx.x < 8) scal[4 * NS + threadIdx.x] = -INFINITY;
+    f32x4_t cb[2];
+    band_colbias<SL>(ln, grp, cb);
+    BandOff<D> off;
+    off.init(lane);
+    const float sc2 = p.scale * kLog2e;
+    const bool wave_ok = t.a[0].wave_ok && t.a[1].wave_ok && t.a[2].wave_ok;
+    const int wc0 = t.a[1].glo / RPC, wc1 = wave_ok ? t.a[1].ghi / RPC : -1;
+    const int w0 = t.a[0].glo, w1 = t.a[0].ghi;
+    const int hend = (t.h + 1) * rep;
+    const float* ninf = scal + 4 * NS;
+    const auto step = [&](auto BC) {
+        constexpr int B = decltype(BC)::value;
+        st.store(smem + B * BUF);
+        if (threadIdx.x < NS) {
+            scal[B * 2 * NS + threadIdx.x] = pin ? -pl * kLog2e : 0.f;
+            scal[B * 2 * NS + NS + threadIdx.x] = pin ? -pd : 0.f;
+        }
+        lds_publish_barrier();
+        const int c0 = bi * NC, cu = u0;
+        if (++bi == nb) {
+            bi = 0;
+            if (++u0 == U0) {
+                u0 = 0;
+                ++h;
+            }
+        }
+        const bool more = h < hend;
+        if (more) load();
+        const unsigned char* Qb = smem + B * BUF;
+        const unsigned char* Gb = Qb + kBandOp<D>;
+        if (cu >= w0 && cu <= w1) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                if (c0 + c < wc0 || c0 + c > wc1) continue;
+                const int row = (c0 + c) * RPC + (RPC == 2 ? grp >> 1 : 0) - ln.rlo;
+                const float* sc = scal + B * 2 * NS + 32 * c + 8 * grp;
+                const float* nlc = static_cast<unsigned>(row) < static_cast<unsigned>(ln.rn) ? sc : ninf;
+                const f32x4_t nl[2] = {*reinterpret_cast<const f32x4_t*>(nlc),
+                                       *reinterpret_cast<const f32x4_t*>(nlc + 4)};
+                const f32x4_t nd[2] = {*reinterpret_cast<const f32x4_t*>(sc + NS),
+                                       *reinterpret_cast<const f32x4_t*>(sc + NS + 4)};
+                f32x4_t s[2], dp[2];
+                band_score<T, D>(Qb, off, c, kf, cb, s);
+                band_score<T, D>(Gb, off, c, vf, nd, dp);
+#pragma unroll
+                for (int bb = 0; bb < 2; ++bb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        s[bb][i] = __builtin_amdgcn_exp2f(fmaf(s[bb][i], sc2, nl[bb][i]));
+                        dp[bb][i] *= s[bb][i];
+                    }
+                band_accumulate<T, D>(Gb, off, c, pack8<T>(s), gv);
+                band_accumulate<T, D>(Qb, off, c, pack8<T>(dp), gk);
+            }
+        }
+        return more;
+    };
+#pragma unroll 1
+    while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{})) {
+    }
+    const bool redo = ln.valid && item_nonfinite(lane_sum(gk, lane_sum(gv, 0.f)));
+    if (ln.valid) store();
+    if (redo)
+        band_redo_bwd_kv<T, D>(kernargs(), t.b, t.h, opaque(ln.pos[0]), opaque(ln.pos[1]), opaque(ln.pos[2]), grp);
+}
+
+// ---------------------------------------------------------------------------
+// Host side.
+// ---------------------------------------------------------------------------
+
+BandGeo band_geo(const Prob& p, int sh2, int heads) {
+    BandGeo g{};
+    g.sh2 = sh2;
+    g.sh1 = log2_of(kBandWaves * 16) - sh2;
+    const int T[3] = {1, 1 << g.sh1, 1 << g.sh2};
+    long long tiles = 1;
+    for (int a = 0; a < 3; ++a) {
+        const int n = (n_class_h(p.ax[a], 0) + T[a] - 1) / T[a];
+        g.lenmod[a] = p.ax[a].len % p.ax[a].dil;
+        g.nt[a] = make_fastdiv(static_cast<uint32_t>(n));
+        g.dil[a] = make_fastdiv(static_cast<uint32_t>(p.ax[a].dil));
+        tiles *= static_cast<long long>(n) * p.ax[a].dil;
+    }
+    g.tiles = make_fastdiv(static_cast<uint32_t>(tiles));
+    g.heads = make_fastdiv(static_cast<uint32_t>(heads));
+    g.rep = make_fastdiv(static_cast<uint32_t>(p.rep));
+    return g;
+}
+
+long long band_blocks(const Prob& p, const BandGeo& g) {
+    return static_cast<long long>(p.B) * g.heads.d * g.tiles.d;
+}
+
+uint32_t band_plane(const Prob& p, const Lay& l, int D) {
+    return static_cast<uint32_t>(((static_cast<long long>(p.ax[1].len) - 1) * l.s1 +
+                                  (static_cast<long long>(p.ax[2].len) - 1) * l.s2 + D) * 2);
+}
+
+template <typename T, int D>
+constexpr size_t kBandLds = kLdsPad + 4 * kBandOp<D>;
+template <typename T, int D>
+constexpr size_t kBandLdsKv = kBandLds<T, D> + (4 * kBandChunks<D> * 32 + 8) * sizeof(float);
+
+template <typename T, int D>
+void band_audit_dim(LdsAudit& a) {
+    audit_one(k_band_fwd<T, D, 32>, "k_band_fwd", a);
+    audit_one(k_band_bwd_q<T, D, 32>, "k_band_bwd_q", a);
+    audit_one(k_band_bwd_kv<T, D, 32>, "k_band_bwd_kv", a);
+}
+
+// No static LDS in any instance (see lds_base): checked once per process.
+bool band_static_lds_ok() {
+    static const bool ok = [] {
+        LdsAudit a;
+        band_audit_dim<bf16, 32>(a);
+        band_audit_dim<bf16, 64>(a);
+        band_audit_dim<bf16, 128>(a);
+        band_audit_dim<f16, 32>(a);
+        band_audit_dim<f16, 64>(a);
+        band_audit_dim<f16, 128>(a);
+        return a.bad == 0;
+    }();
+    return ok;
+}
+
+bool band_switch() {
+    static const bool on = [] {
+        const char* e = std::getenv("NATTEN_HIP_BAND");
+        return !(e && std::strcmp(e, "0") == 0);
+    }();
+    return on;
+}
+
+template <typename T, int D>
+hipError_t band_fwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,
+                        Lay lo, float* lse, Lay ll, hipStream_t s) {
+    BandArgs<T> a{};
+    a.p = p;
+    a.g = band_geo(p, band_columns(p.ax[2].k, false), p.Hq);
+    a.q = static_cast<const T*>(q);
+    a.k = static_cast<const T*>(k);
+    a.v = static_cast<const T*>(v);
+    a.out = static_cast<T*>(o);
+    a.lse_out = lse;
+    a.lq = to_k(lq);
+    a.lk = to_k(lk);
+    a.lv = to_k(lv);
+    a.lo = to_k(lo);
+    a.ll = to_k(ll);
+    a.ab = band_plane(p, lk, D);
+    a.bb = band_plane(p, lv, D);
+    auto kern = k_band_fwd<T, D, 32>;
+    const hipError_t e = allow_lds(kern, kBandLds<T, D>);
+    if (e != hipSuccess) return e;
+    NA_LAUNCH("na_fwd_band", kern, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
+              (kBandLds<T, D>), s, a);
+    return hipGetLastError();
+}
+
+template <typename T, int D>
+hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
+                        const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll, const float* dlse,
+                        Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv, float* delta, Lay lde,
+                        hipStream_t s) {
+    BandArgs<T> a{};
+    a.p = p;
+    a.g = band_geo(p, band_columns(p.ax[2].k, false), p.Hq);
+    a.q = static_cast<const T*>(q);
+    a.k = static_cast<const T*>(k);
+    a.v = static_cast<const T*>(v);
+    a.o = static_cast<const T*>(o);
+    a.dout = static_cast<const T*>(dout);
+    a.lse = lse;
+    a.dlse = dlse;
+    a.delta = delta;
+    a.delta_out = delta;
+    a.dq = static_cast<T*>(dq);
+    a.dk = static_cast<T*>(dk);
+    a.dv = static_cast<T*>(dv);
+    a.lq = to_k(lq);
+    a.lk = to_k(lk);
+    a.lv = to_k(lv);
+    a.lo = to_k(lo);
+    a.ldo = to_k(ldo);
+    a.ldq = to_k(ldq);
+    a.ldk = to_k(ldk);
+    a.ldv = to_k(ldv);
+    a.ll = to_k(ll);
+    a.lde = to_k(lde);
+    a.ldl = to_k(ldl);
+    a.ab = band_plane(p, lk, D);
+    a.bb = band_plane(p, lv, D);
+    auto kq = k_band_bwd_q<T, D, 32>;
+    hipError_t e = allow_lds(kq, kBandLds<T, D>);
+    if (e != hipSuccess) return e;
+    NA_LAUNCH("na_bwd_q_band", kq, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
+              (kBandLds<T, D>), s, a);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    a.g = band_geo(p, band_columns(p.ax[2].k, true), p.Hkv);
+    a.ab = band_plane(p, lq, D);
+    a.bb = band_plane(p, ldo, D);
+    auto kk = k_band_bwd_kv<T, D, 32>;
+    if ((e = allow_lds(kk, kBandLdsKv<T, D>)) != hipSuccess) return e;
+    NA_LAUNCH("na_bwd_kv_band", kk, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
+              (kBandLdsKv<T, D>), s, a);
+    return hipGetLastError();
+}
+
+#define NA_BAND_DISPATCH(RUN, ...)                              \
+    if (dtype == NATTEN_BF16) {                                 \
+        if (p.Dqk == 32) return RUN<bf16, 32>(__VA_ARGS__);     \
+        if (p.Dqk == 64) return RUN<bf16, 64>(__VA_ARGS__);     \
+        return RUN<bf16, 128>(__VA_ARGS__);                     \
+    }                                                           \
+    if (p.Dqk == 32) return RUN<f16, 32>(__VA_ARGS__);          \
+    if (p.Dqk == 64) return RUN<f16, 64>(__VA_ARGS__);          \
+    return RUN<f16, 128>(__VA_ARGS__)
+
+}  // namespace
+
+// 2-D problems (axis 0 of extent 1) at stride 1, 16-bit, head dim 32 / 64 /
+// 128 for q, k and v, whose windows span 10 to 16 columns (so that a tile's
+// union fits 32): the range past the 8x8 tile kernels.  `lays`: every 16-bit
+// operand and fp32 row operand of the call.
+bool band_eligible(const Prob& p, int dtype, bool aligned, std::initializer_list<Lay> lays) {
+    if (!band_switch() || !aligned || dtype == NATTEN_F32 || !(p.scale > 0.f)) return false;
+    if (p.Dqk != p.Dv || (p.Dqk != 32 && p.Dqk != 64 && p.Dqk != 128)) return false;
+    if (p.ax[0].len != 1 || p.ax[0].k != 1) return false;
+    for (int a = 0; a < 3; ++a)
+        if (p.ax[a].st != 1 || p.ax[a].len >= (1 << 24)) return false;
+    if (p.ax[2].k < 10 || band_columns(p.ax[2].k, true) < 0) return false;
+    // a tile has at least 8 rows: fewer would leave its waves idle
+    if (n_class_h(p.ax[1], 0) < 8) return false;
+    if (!offsets_fit(p, lays)) return false;
+    for (const Lay& l : lays)
+        if (band_plane(p, l, p.Dqk) >= kBandOOR) return false;
+    const long long tiles = ((static_cast<long long>(p.ax[1].len) + 7) / 8 + p.ax[1].dil) *
+                            ((static_cast<long long>(p.ax[2].len) + 7) / 8 + p.ax[2].dil);
+    if (tiles * p.B * p.Hq >= (1LL << 31)) return false;
+    return band_static_lds_ok();
+}
+
+hipError_t band_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,
+                        Lay lo, float* lse, Lay ll, int dtype, hipStream_t s) {
+    NA_BAND_DISPATCH(band_fwd_run, p, q, lq, k, lk, v, lv, o, lo, lse, ll, s);
+}
+
+hipError_t band_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
+                         const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll, const float* dlse,
+                         Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv, float* delta, Lay lde,
+                         int dtype, hipStream_t s) {
+    NA_BAND_DISPATCH(band_bwd_run, p, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
+                     ldv, delta, lde, s);
+}
+
+}  // namespace na

@@ -169,6 +169,11 @@ int natten_hip_forward(const natten_problem_t* p, const void* q, const natten_la
                                               to_lay(llse), p->dtype, s);
         if (e != hipErrorNotSupported) return launch_status(e, "forward");
     }
+    if (use_mfma() && na::band_eligible(P, p->dtype, vec != 0,
+                                        {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)}))
+        return launch_status(na::band_forward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), lse,
+                                              to_lay(llse), p->dtype, s),
+                             "forward");
     if (use_mfma() && na::mfma_eligible(P, p->dtype, D, vec != 0, false) &&
         na::mfma_offsets_fit(P, {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)})) {
         return launch_status(na::mfma_forward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), lse,
@@ -208,6 +213,16 @@ int backward_impl(const natten_problem_t* p, const na::Prob& P, const void* q, c
             dlse, to_lay(ldlse), dq, to_lay(ldq), dk, to_lay(ldk), dv, to_lay(ldv), delta, to_lay(ldelta), p->dtype,
             static_cast<hipStream_t>(stream));
         if (e != hipErrorNotSupported) return launch_status(e, "backward");
+    }
+    if (use_mfma() &&
+        na::band_eligible(P, p->dtype, vec != 0,
+                          {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(ldo), to_lay(llse), to_lay(ldq),
+                           to_lay(ldk), to_lay(ldv), to_lay(ldelta), dlse ? to_lay(ldlse) : to_lay(llse)})) {
+        return launch_status(na::band_backward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), dout,
+                                               to_lay(ldo), lse, to_lay(llse), dlse, to_lay(ldlse), dq, to_lay(ldq),
+                                               dk, to_lay(ldk), dv, to_lay(ldv), delta, to_lay(ldelta), p->dtype,
+                                               static_cast<hipStream_t>(stream)),
+                             "backward");
     }
     if (use_mfma() && na::mfma_eligible(P, p->dtype, D, vec != 0, true) &&
         na::mfma_offsets_fit(P, {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(ldo), to_lay(llse),

@@ -257,6 +257,17 @@ __host__ __device__ inline AxisGeo axis_geometry(int len, int K, int dil, int ca
     return o;
 }
 
+// Band kernels (na_band.hip): columns of a tile's box (log2) for in-plane
+// kernel K, 16 where every tile's union fits a row of 32 slots, else 8; -1
+// where neither does.  A query tile's union spans at most
+// T - 1 + K columns.  A key tile's (the queries attending its keys) reaches
+// further where the border holds windows back, up to 31 columns for K = 11
+// at T = 16 and 32 for K = 16 at T = 8, over every class size.
+inline int band_columns(int K, bool key) {
+    if (!key) return K <= 17 ? 4 : -1;
+    return K <= 11 ? 4 : K <= 16 ? 3 : -1;
+}
+
 // f(j0, j1, j2, e, valid) for each neighbour e (row-major over the kernel) of
 // the query at (i0, i1, i2).  Invalid (causal) neighbours have j < 0 on some
 // axis and must not be dereferenced.

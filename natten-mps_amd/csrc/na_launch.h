@@ -156,6 +156,17 @@ hipError_t lean_backward(const Prob& p, const void* q, Lay lq, const void* k, La
                          const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
                          float* delta, Lay lde, int dtype, hipStream_t s);
 
+// Band kernels (na_band.hip): 2-D problems at stride 1, 16-bit, head dim 32,
+// 64 or 128, in-plane kernels of 10 to 16 columns; no tables, so every
+// eligible call has a launch.
+bool band_eligible(const Prob& p, int dtype, bool aligned, std::initializer_list<Lay> lays);
+hipError_t band_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,
+                        Lay lo, float* lse, Lay ll, int dtype, hipStream_t s);
+hipError_t band_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
+                         const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll,
+                         const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
+                         float* delta, Lay lde, int dtype, hipStream_t s);
+
 // Key side of the global keys' backward (na_global.hip): dk and dv of the
 // global keys (summed over every query of each q head of the group), from the
 // forward's lse and the backward's delta.  Partial sums over slices of the

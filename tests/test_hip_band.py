@@ -1,0 +1,99 @@
+"""The band kernels (csrc/na_band.hip): in-plane windows of 10 to 16 columns,
+staged a band of union rows at a time.  Sizes at the edges of their tiles
+(128 items in rows of 8 or 16 columns; bands of 2 or 4 rows), on every head
+dim, against the CPU oracle."""
+
+import pytest
+import torch
+
+import oracle.pure as P
+from _parity import assert_parity
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+@pytest.fixture(autouse=True)
+def _hip():
+    import natten_mps_amd
+
+    natten_mps_amd.set_backend("hip")
+    yield
+
+
+CASES = [
+    # spatial, heads q / kv, dim, kernel, dilation, causal, packed
+    ((17, 33), 2, 2, 64, (13, 13), (1, 1), (False, False), False),
+    ((16, 13), 1, 1, 32, (3, 13), (1, 1), (False, False), False),   # one column of windows
+    ((8, 40), 2, 2, 64, (1, 11), (1, 1), (False, False), False),    # no window rows to walk
+    ((29, 45), 2, 2, 32, (13, 13), (1, 1), (True, False), False),
+    ((23, 44), 4, 2, 64, (7, 11), (1, 1), (False, True), False),    # GQA
+    ((50, 31), 2, 2, 128, (15, 15), (2, 2), (False, False), False),
+    ((21, 36), 2, 1, 128, (5, 16), (1, 2), (False, False), False),  # even kernel
+    ((40, 20), 2, 2, 64, (33, 10), (1, 1), (False, False), True),   # packed q/k/v views
+    ((27, 49), 3, 3, 32, (11, 11), (2, 3), (True, True), True),
+]
+
+
+def _inputs(seed, shapes, dtype):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(s, generator=g, dtype=torch.float32).to(dtype) for s in shapes]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", CASES)
+def test_band_kernels_match_oracle(case, dtype):
+    """Output, log-sum-exp and the gradients through both."""
+    from natten_mps_amd import functional as F
+    from natten_mps_amd._core import _lib
+
+    sp, hq, hkv, dim, ks, dil, causal, packed = case
+    print(case, dtype, flush=True)
+    q, k, v, do = _inputs(31, [(2, *sp, hq, dim), (2, *sp, hkv, dim), (2, *sp, hkv, dim), (2, *sp, hq, dim)], dtype)
+    (dl,) = _inputs(32, [(2, *sp, hq)], dtype)
+    dev = [t.to(DEV) for t in (q, k, v)]
+    if packed:
+        dev = list(torch.stack(dev, dim=3).unbind(3))
+    leaves = [t.requires_grad_(True) for t in dev]
+    _lib.profile_read(reset=True)
+    _lib.profile_enable(True)
+    try:
+        out, lse = F.na2d(*leaves, kernel_size=ks, dilation=dil, is_causal=causal, return_lse=True)
+        grads = torch.autograd.grad((out, lse), leaves, (do.to(DEV), dl.to(DEV)))
+        torch.cuda.synchronize()
+    finally:
+        _lib.profile_enable(False)
+    launched = set(_lib.profile_read(reset=True))
+    assert {"na_fwd_band", "na_bwd_q_band", "na_bwd_kv_band"} <= launched, launched
+
+    rq, rk, rv = (t.float().requires_grad_(True) for t in (q, k, v))
+    n = hq // hkv
+    ke, ve = (t.repeat_interleave(n, dim=-2) for t in (rk, rv))
+    logits = P.na2d_qk_forward(rq, ke, ks, dil, (1, 1), causal, dim ** -0.5)
+    ref_lse = torch.logsumexp(logits, dim=-1)
+    ref = P.na2d_av_forward(torch.softmax(logits, dim=-1), ve, ks, dil, (1, 1), causal)
+    rgrads = torch.autograd.grad((ref, ref_lse), (rq, rk, rv), (do.float(), dl.float()))
+    for name, a, b in zip(("out", "lse", "dq", "dk", "dv"), (out, lse, *grads), (ref, ref_lse, *rgrads)):
+        assert_parity(a.detach().cpu(), b.detach(), dtype, name)
+
+
+def test_band_kernels_recompute_non_finite_operands():
+    """A non-finite key outside a query's window does not reach it, and one
+    inside does, as in the oracle (the finite elements agree)."""
+    from natten_mps_amd import functional as F
+
+    ks = (13, 13)
+    q, k, v, do = _inputs(33, [(1, 20, 34, 1, 64)] * 4, torch.bfloat16)
+    k[0, 3, 5, 0, 7] = float("inf")
+    v[0, 15, 30, 0, 9] = float("nan")
+    leaves = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+    out = F.na2d(*leaves, kernel_size=ks)
+    grads = torch.autograd.grad(out, leaves, do.to(DEV))
+    ref_leaves = [t.float().requires_grad_(True) for t in (q, k, v)]
+    ref = P.na2d_forward(*ref_leaves, ks, (1, 1), (1, 1), (False, False), None)
+    rgrads = torch.autograd.grad(ref, ref_leaves, do.float())
+    for name, a, b in zip(("out", "dq", "dk", "dv"), (out, *grads), (ref, *rgrads)):
+        a, b = a.detach().float().cpu(), b.detach()
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b)), name
+        fin = torch.isfinite(b)
+        assert_parity(a[fin], b[fin], torch.bfloat16, name)
