@@ -1410,6 +1410,15 @@ int split_chunks(const Axis& A, int r, const LeanAxisTile& a, int K2) {
 // items along axis 2.
 bool lean_1d(const Prob& p) { return p.ax[0].len == 1 && p.ax[1].len == 1 && p.ax[1].k == 1; }
 
+// Chunks per wave of the widest key-side instance.  A wave's two key rows
+// are attended from at most K1 + 1 + K1 / 2 rows near one border, which the
+// instance for NCH (NCH + 2 chunks) holds; in a class of about 2 K1 rows both
+// borders meet in one wave and the span reaches the whole class (7 x 7 on
+// classes of 14 rows: 14), which the widest one holds: backward of 64 x 14 x
+// 14 x 12 heads, head dim 32, 21.1 + 22.4 us on the general tiles, 15.3 +
+// 20.0 us here; split key side of 16 x 28 x 28 x 8, dilation 2, 22.8 -> 20.
+constexpr int kLeanMaxKeyChunks = 7;
+
 // Chunks of 32 slots a wave of a 1-D query tile reads: its 16 windows from
 // the staged row holding the first of them (up to 15 slots in).
 int lean_nch_1d(int K) { return std::max(1, (K + 30 + 31) / 32); }
@@ -1420,7 +1429,7 @@ int lean_nch_1d(int K) { return std::max(1, (K + 30 + 31) / 32); }
 // class size and border start, the union's size; key tiles also each
 // wave's first staged row (bytes of [9]) and chunk count (bytes of [10]),
 // and [14] = 1 where no query attends the tile.  False when a wave's
-// windows (attending spans) do not fit nch (key tiles: nch + 2) chunks.
+// windows (attending spans) do not fit nch (key tiles: kLeanMaxKeyChunks) chunks.
 bool lean_records_1d(const Prob& p, bool key, int nch, std::vector<int>& h, int& nst_max, int& rows_max) {
     const Axis& A = p.ax[2];
     for (int r = 0; r < A.dil; ++r) {
@@ -1477,7 +1486,7 @@ bool lean_records_1d(const Prob& p, bool key, int nch, std::vector<int>& h, int&
                     end = whi - U0 - 16 * first + 1;
                 }
                 const int need = (end + 31) / 32;
-                if (need > (key ? nch + 2 : nch)) return false;
+                if (need > (key ? kLeanMaxKeyChunks : nch)) return false;
                 fb[w] = first;
                 nb[w] = need;
                 nst = std::max(nst, first + 2 * (key ? need : nch));
@@ -1919,7 +1928,8 @@ hipError_t lean_bwd_run(const Prob& p, const LeanGeo* gq, const LeanGeo* gk, con
     NA_LAUNCH("na_bwd_q_lean", kq, dim3(static_cast<unsigned>(tasks)), dim3(64 * kLeanWaves * HP), shm_q, s, a);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    auto kern = k_lean_bwd_kv<T, D, NCH + 2, D3, ONE_D>;
+    auto kern = gk->rows_max <= 2 * (NCH + 2) ? k_lean_bwd_kv<T, D, NCH + 2, D3, ONE_D>
+                                              : k_lean_bwd_kv<T, D, kLeanMaxKeyChunks, D3, ONE_D>;
     if ((e = allow_lds(kern, shm_k)) != hipSuccess) return e;
     // key tiles over the kv heads, each walking the q heads of its group
     LeanBwdArgs<T> ak = a;
@@ -1944,7 +1954,7 @@ hipError_t lean_backward(const Prob& p, const void* q, Lay lq, const void* k, La
     const int nch = d1 ? lean_nch_1d(p.ax[2].k) : lean_nch(p.ax[1].k);
     const LeanGeo* gq = lean_geometry(p, 0, nch, s);
     const LeanGeo* gk = gq ? lean_geometry(p, 1, nch, s) : nullptr;
-    if (!gq || !gk || gq->ntiles != gk->ntiles || gk->rows_max > 2 * (nch + 2)) return hipErrorNotSupported;
+    if (!gq || !gk || gq->ntiles != gk->ntiles || gk->rows_max > 2 * kLeanMaxKeyChunks) return hipErrorNotSupported;
 #define NA_LB_A(T, DD) \
     lean_bwd_args<T, DD>(p, q, lq, k, lk, v, o, lo, dout, ldo, lse, ll, dlse, dq, ldq, dk, ldk, dv, delta)
     // GQA with an even group: two q heads per dQ workgroup share the staged K/V
@@ -2061,9 +2071,12 @@ hipError_t lean_wsum_key(const char* name, const Prob& p, int D, const void* w, 
     const int nch = lean_nch(p.ax[1].k);
     if (static_cast<long long>(p.B) * p.Hq * 8192 >= (1LL << 31)) return hipErrorNotSupported;
     const LeanGeo* g = lean_geometry(p, 2, nch, s);
-    if (!g || g->rows_max > 2 * (nch + 2)) return hipErrorNotSupported;
+    if (!g || g->rows_max > 2 * kLeanMaxKeyChunks) return hipErrorNotSupported;
     name = lean_key_name(name);
-#define NA_LW(T, DD, N) return lean_wsum_key_run<T, DD, N + 2>(name, p, g, w, lw, x, lx, o, lo, mul, s)
+#define NA_LW(T, DD, N)                                                                              \
+    return g->rows_max <= 2 * (N + 2)                                                                \
+               ? lean_wsum_key_run<T, DD, N + 2>(name, p, g, w, lw, x, lx, o, lo, mul, s)             \
+               : lean_wsum_key_run<T, DD, kLeanMaxKeyChunks>(name, p, g, w, lw, x, lx, o, lo, mul, s)
 #define NA_LW_N(T, DD)          \
     switch (nch) {              \
         case 1: NA_LW(T, DD, 1); \
