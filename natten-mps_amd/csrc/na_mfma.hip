@@ -1347,7 +1347,12 @@ bool choose_tile(const Prob& p, Kind kind, int D, TileShape& ts, size_t extra_ld
         const int u2 = varlen ? union_extent_upto(p.ax[2], T[2], key_tile) : union_extent(p.ax[2], T[2], key_tile);
         ts.rowshift = std::max(3, log2_of(u2));
         ts.slots = ((u1 * (1 << ts.rowshift) + 31) / 32) * 32;
-        return lds_bytes(kind, ts.slots, D) + extra_lds <= budget;
+        // extra_lds (global keys, at most 16 KB) comes on top of the smaller
+        // budget: two workgroups of up to 80 KB still fit a CU.  Inside it, a
+        // 7 x 7 head-dim-64 union (57 KB) fell to 32-query tiles: 8 x 48 x 48
+        // x 8 heads, 16 tokens, forward 52 -> 44 us, dQ 54 -> 44 us
+        const size_t lds = lds_bytes(kind, ts.slots, D);
+        return lds + (budget == kLdsBudgetLarge ? extra_lds : 0) <= budget;
     };
     const auto finish = [&]() {
         ts.nheads = key_tile ? p.Hkv : p.Hq;
