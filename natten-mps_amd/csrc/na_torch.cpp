@@ -14,6 +14,10 @@
 // the ctypes path: invalid input -> ValueError, unsupported ->
 // NotImplementedError, launch failure -> RuntimeError.
 //
+// A FusedCall also serves the variable-length calls (varlen_fwd /
+// varlen_bwd, with the samples' extents as one more operand), and GlobalCall
+// the calls with global keys (gfwd / gbwd).
+//
 // SplitCall does the same for the four split ops (qk, av, qk_bwd, av_bwd)
 // and the four relative-position-bias ops (rpb_qk, rpb_av, rpb_qk_bwd,
 // rpb_av_bwd).
@@ -129,8 +133,10 @@ struct FusedCall {
         std::memcpy(lay.data(), l.data(), l.size());
     }
 
-    std::tuple<at::Tensor, at::Tensor> forward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
-                                               int64_t stream) const {
+    // lens: per-sample extents of a variable-length call (device int32
+    // [batch][3]), or null
+    std::tuple<at::Tensor, at::Tensor> run_forward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                                                   int64_t stream, const int32_t* lens) const {
         if (lay.size() != kFwdLays) throw pybind11::value_error("FusedCall.forward: not a forward signature");
         c10::OptionalDeviceGuard guard;
         if (current_index() != q.get_device()) guard.reset_device(q.device());
@@ -141,18 +147,26 @@ struct FusedCall {
         blk.allocate(q.device());
         at::Tensor out = blk.part(0, out_shape, q.scalar_type());
         at::Tensor lse = blk.part(1, lse_shape, at::kFloat);
-        const int rc = natten_hip_forward(&prob, q.data_ptr(), &lay[0], k.data_ptr(), &lay[1], v.data_ptr(), &lay[2],
-                                          out.data_ptr(), &lay[3], lse.data_ptr<float>(), &lay[4],
-                                          reinterpret_cast<void*>(stream));
-        if (rc != NATTEN_OK) raise_status(rc, "forward");
+        void* const s = reinterpret_cast<void*>(stream);
+        const int rc =
+            lens ? natten_hip_varlen_forward(&prob, lens, q.data_ptr(), &lay[0], k.data_ptr(), &lay[1], v.data_ptr(),
+                                             &lay[2], out.data_ptr(), &lay[3], lse.data_ptr<float>(), &lay[4], s)
+                 : natten_hip_forward(&prob, q.data_ptr(), &lay[0], k.data_ptr(), &lay[1], v.data_ptr(), &lay[2],
+                                      out.data_ptr(), &lay[3], lse.data_ptr<float>(), &lay[4], s);
+        if (rc != NATTEN_OK) raise_status(rc, lens ? "varlen_forward" : "forward");
         return {out, lse};
     }
 
-    std::tuple<at::Tensor, at::Tensor, at::Tensor> backward(const at::Tensor& q, const at::Tensor& k,
-                                                            const at::Tensor& v, const at::Tensor& out,
-                                                            const at::Tensor& d_out, const at::Tensor& lse,
-                                                            const std::optional<at::Tensor>& d_lse,
-                                                            int64_t stream) const {
+    std::tuple<at::Tensor, at::Tensor> forward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                                               int64_t stream) const {
+        return run_forward(q, k, v, stream, nullptr);
+    }
+
+    std::tuple<at::Tensor, at::Tensor, at::Tensor> run_backward(const at::Tensor& q, const at::Tensor& k,
+                                                                const at::Tensor& v, const at::Tensor& out,
+                                                                const at::Tensor& d_out, const at::Tensor& lse,
+                                                                const std::optional<at::Tensor>& d_lse,
+                                                                int64_t stream, const int32_t* lens) const {
         if (lay.size() != kBwdLays) throw pybind11::value_error("FusedCall.backward: not a backward signature");
         c10::OptionalDeviceGuard guard;
         if (current_index() != q.get_device()) guard.reset_device(q.device());
@@ -174,17 +188,91 @@ struct FusedCall {
         at::Tensor dv = blk.part(2, v.sizes(), v.scalar_type());
         float* const delta = static_cast<float*>(blk.st.mutable_data()) + blk.off[3] / sizeof(float);
         const float* dl = d_lse.has_value() ? d_lse->data_ptr<float>() : nullptr;
-        const int rc = natten_hip_backward(
-            &prob, q.data_ptr(), &lay[0], k.data_ptr(), &lay[1], v.data_ptr(), &lay[2], out.data_ptr(), &lay[3],
-            d_out.data_ptr(), &lay[4], lse.data_ptr<float>(), &lay[5], dl, dl ? &lay[6] : nullptr, dq.data_ptr(),
-            &lay[7], dk.data_ptr(), &lay[8], dv.data_ptr(), &lay[9], delta, &lay[10],
-            reinterpret_cast<void*>(stream));
-        if (rc != NATTEN_OK) raise_status(rc, "backward");
+        void* const s = reinterpret_cast<void*>(stream);
+        const int rc =
+            lens ? natten_hip_varlen_backward(&prob, lens, q.data_ptr(), &lay[0], k.data_ptr(), &lay[1], v.data_ptr(),
+                                              &lay[2], out.data_ptr(), &lay[3], d_out.data_ptr(), &lay[4],
+                                              lse.data_ptr<float>(), &lay[5], dq.data_ptr(), &lay[7], dk.data_ptr(),
+                                              &lay[8], dv.data_ptr(), &lay[9], delta, &lay[10], s)
+                 : natten_hip_backward(&prob, q.data_ptr(), &lay[0], k.data_ptr(), &lay[1], v.data_ptr(), &lay[2],
+                                       out.data_ptr(), &lay[3], d_out.data_ptr(), &lay[4], lse.data_ptr<float>(),
+                                       &lay[5], dl, dl ? &lay[6] : nullptr, dq.data_ptr(), &lay[7], dk.data_ptr(),
+                                       &lay[8], dv.data_ptr(), &lay[9], delta, &lay[10], s);
+        if (rc != NATTEN_OK) raise_status(rc, lens ? "varlen_backward" : "backward");
         return {dq, dk, dv};
+    }
+
+    std::tuple<at::Tensor, at::Tensor, at::Tensor> backward(const at::Tensor& q, const at::Tensor& k,
+                                                            const at::Tensor& v, const at::Tensor& out,
+                                                            const at::Tensor& d_out, const at::Tensor& lse,
+                                                            const std::optional<at::Tensor>& d_lse,
+                                                            int64_t stream) const {
+        return run_backward(q, k, v, out, d_out, lse, d_lse, stream, nullptr);
     }
 
     static int current_index() {
         return c10::impl::getDeviceGuardImpl(c10::DeviceType::CUDA)->getDevice().index();
+    }
+};
+
+// Fused calls with global keys: FusedCall's layouts followed by those of the
+// global keys and values (backward: and of their gradients).
+struct GlobalCall : FusedCall {
+    int64_t work_floats;  // backward: the global keys' partial sums
+
+    GlobalCall(const pybind11::bytes& prob_bytes, const pybind11::bytes& lay_bytes, std::vector<int64_t> out_shape_,
+               std::vector<int64_t> lse_shape_, int64_t work_floats_)
+        : FusedCall(prob_bytes, lay_bytes, std::move(out_shape_), std::move(lse_shape_), false),
+          work_floats(work_floats_) {
+        if (work_floats < 0) throw pybind11::value_error("GlobalCall: negative workspace");
+    }
+
+    std::tuple<at::Tensor, at::Tensor> forward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                                               const at::Tensor& gk, const at::Tensor& gv, int64_t stream) const {
+        if (lay.size() != kFwdLays + 2) throw pybind11::value_error("GlobalCall.forward: not a forward signature");
+        c10::OptionalDeviceGuard guard;
+        if (current_index() != q.get_device()) guard.reset_device(q.device());
+        Block blk;
+        blk.add(numel(out_shape) * static_cast<int64_t>(c10::elementSize(q.scalar_type())));
+        blk.add(numel(lse_shape) * static_cast<int64_t>(sizeof(float)));
+        blk.allocate(q.device());
+        at::Tensor out = blk.part(0, out_shape, q.scalar_type());
+        at::Tensor lse = blk.part(1, lse_shape, at::kFloat);
+        const int rc = natten_hip_forward_global(
+            &prob, q.data_ptr(), &lay[0], k.data_ptr(), &lay[1], v.data_ptr(), &lay[2], gk.data_ptr(), &lay[5],
+            gv.data_ptr(), &lay[6], static_cast<int32_t>(gk.size(1)), out.data_ptr(), &lay[3], lse.data_ptr<float>(),
+            &lay[4], reinterpret_cast<void*>(stream));
+        if (rc != NATTEN_OK) raise_status(rc, "forward_global");
+        return {out, lse};
+    }
+
+    std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor> backward(
+        const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& gk, const at::Tensor& gv,
+        const at::Tensor& out, const at::Tensor& d_out, const at::Tensor& lse,
+        const std::optional<at::Tensor>& d_lse, int64_t stream) const {
+        if (lay.size() != kBwdLays + 4) throw pybind11::value_error("GlobalCall.backward: not a backward signature");
+        c10::OptionalDeviceGuard guard;
+        if (current_index() != q.get_device()) guard.reset_device(q.device());
+        Block blk;
+        const at::Tensor* like[5] = {&q, &k, &v, &gk, &gv};
+        for (const at::Tensor* t : like) blk.add(t->numel() * static_cast<int64_t>(c10::elementSize(t->scalar_type())));
+        blk.allocate(q.device());
+        at::Tensor g[5];
+        for (int i = 0; i < 5; ++i) g[i] = blk.part(i, like[i]->sizes(), like[i]->scalar_type());
+        // delta rows and the partial sums: only this call's kernels use them
+        const int64_t rows = (numel(lse_shape) + 63) & ~int64_t(63);
+        const Workspace work(static_cast<size_t>(rows + work_floats) * sizeof(float),
+                             reinterpret_cast<hipStream_t>(stream));
+        float* const delta = static_cast<float*>(work.ptr);
+        const float* dl = d_lse.has_value() ? d_lse->data_ptr<float>() : nullptr;
+        const int rc = natten_hip_backward_global(
+            &prob, q.data_ptr(), &lay[0], k.data_ptr(), &lay[1], v.data_ptr(), &lay[2], gk.data_ptr(), &lay[11],
+            gv.data_ptr(), &lay[12], static_cast<int32_t>(gk.size(1)), out.data_ptr(), &lay[3], d_out.data_ptr(),
+            &lay[4], lse.data_ptr<float>(), &lay[5], dl, dl ? &lay[6] : nullptr, g[0].data_ptr(), &lay[7],
+            g[1].data_ptr(), &lay[8], g[2].data_ptr(), &lay[9], g[3].data_ptr(), &lay[13], g[4].data_ptr(), &lay[14],
+            delta, &lay[10], delta + rows, work_floats, reinterpret_cast<void*>(stream));
+        if (rc != NATTEN_OK) raise_status(rc, "backward_global");
+        return {g[0], g[1], g[2], g[3], g[4]};
     }
 };
 
@@ -418,7 +506,8 @@ struct Entry {
 };
 
 constexpr size_t kCacheMax = 64;
-std::vector<Entry<FusedCall>> g_fwd, g_bwd;
+std::vector<Entry<FusedCall>> g_fwd, g_bwd, g_vfwd, g_vbwd;
+std::vector<Entry<GlobalCall>> g_gfwd, g_gbwd;
 std::vector<Entry<SplitCall>> g_split[kSplitOps];
 
 template <typename C>
@@ -438,8 +527,9 @@ bool remember(std::vector<Entry<C>>& cache, const Key& k, pybind11::object call)
 }
 
 void clear_all() {
-    g_fwd.clear();
-    g_bwd.clear();
+    for (auto* c : {&g_fwd, &g_bwd, &g_vfwd, &g_vbwd}) c->clear();
+    g_gfwd.clear();
+    g_gbwd.clear();
     for (auto& c : g_split) c.clear();
 }
 
@@ -511,6 +601,93 @@ bool bwd_register(int64_t rank, const at::Tensor& dout, const at::Tensor& q, con
                   pybind11::handle dil, pybind11::handle st, pybind11::handle causal, pybind11::handle scale,
                   const std::optional<at::Tensor>& dlse, pybind11::object call) {
     return remember(g_bwd, bwd_key(rank, dout, q, k, v, out, lse, ks, dil, st, causal, scale, dlse),
+                    std::move(call));
+}
+
+// Variable-length calls: lens is the device int32 [batch][3] of the samples'
+// extents (its values are not part of the key).
+Key varlen_key(int64_t rank, std::initializer_list<const at::Tensor*> ts, const at::Tensor* lse,
+               const at::Tensor& lens, pybind11::handle ks, pybind11::handle dil, pybind11::handle scale) {
+    Key key;
+    key.put(rank);
+    for (const at::Tensor* t : ts) key.tensor(*t, true);
+    if (lse) key.tensor(*lse, false, true);
+    key.tensor(lens, true);
+    if (lens.defined() && (lens.scalar_type() != at::kInt || lens.dim() != 2 || lens.size(1) != 3 || !lens.is_contiguous()))
+        key.ok = false;
+    key.ints(ks);
+    key.ints(dil);
+    key.scale(scale);
+    return key;
+}
+
+pybind11::object varlen_fwd(int64_t rank, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                            const at::Tensor& lens, pybind11::handle ks, pybind11::handle dil,
+                            pybind11::handle scale) {
+    const FusedCall* c = find(g_vfwd, varlen_key(rank, {&q, &k, &v}, nullptr, lens, ks, dil, scale));
+    if (!c) return pybind11::none();
+    return pybind11::cast(c->run_forward(q, k, v, current_stream(q), lens.data_ptr<int32_t>()));
+}
+
+bool varlen_fwd_register(int64_t rank, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                         const at::Tensor& lens, pybind11::handle ks, pybind11::handle dil, pybind11::handle scale,
+                         pybind11::object call) {
+    return remember(g_vfwd, varlen_key(rank, {&q, &k, &v}, nullptr, lens, ks, dil, scale), std::move(call));
+}
+
+pybind11::object varlen_bwd(int64_t rank, const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k,
+                            const at::Tensor& v, const at::Tensor& out, const at::Tensor& lse, const at::Tensor& lens,
+                            pybind11::handle ks, pybind11::handle dil, pybind11::handle scale) {
+    const FusedCall* c = find(g_vbwd, varlen_key(rank, {&q, &k, &v, &out, &dout}, &lse, lens, ks, dil, scale));
+    if (!c) return pybind11::none();
+    return pybind11::cast(
+        c->run_backward(q, k, v, out, dout, lse, std::nullopt, current_stream(q), lens.data_ptr<int32_t>()));
+}
+
+bool varlen_bwd_register(int64_t rank, const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k,
+                         const at::Tensor& v, const at::Tensor& out, const at::Tensor& lse, const at::Tensor& lens,
+                         pybind11::handle ks, pybind11::handle dil, pybind11::handle scale, pybind11::object call) {
+    return remember(g_vbwd, varlen_key(rank, {&q, &k, &v, &out, &dout}, &lse, lens, ks, dil, scale), std::move(call));
+}
+
+// Calls with global keys: the fused key and the two token tensors.
+Key global_key(Key key, const at::Tensor& gk, const at::Tensor& gv) {
+    key.tensor(gk, true);
+    key.tensor(gv, true);
+    return key;
+}
+
+pybind11::object gfwd(int64_t rank, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                      const at::Tensor& gk, const at::Tensor& gv, pybind11::handle ks, pybind11::handle st,
+                      pybind11::handle dil, pybind11::handle causal, pybind11::handle scale) {
+    const GlobalCall* c = find(g_gfwd, global_key(fwd_key(rank, q, k, v, ks, st, dil, causal, scale), gk, gv));
+    if (!c) return pybind11::none();
+    return pybind11::cast(c->forward(q, k, v, gk, gv, current_stream(q)));
+}
+
+bool gfwd_register(int64_t rank, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& gk,
+                   const at::Tensor& gv, pybind11::handle ks, pybind11::handle st, pybind11::handle dil,
+                   pybind11::handle causal, pybind11::handle scale, pybind11::object call) {
+    return remember(g_gfwd, global_key(fwd_key(rank, q, k, v, ks, st, dil, causal, scale), gk, gv), std::move(call));
+}
+
+pybind11::object gbwd(int64_t rank, const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k,
+                      const at::Tensor& v, const at::Tensor& gk, const at::Tensor& gv, const at::Tensor& out,
+                      const at::Tensor& lse, pybind11::handle ks, pybind11::handle st, pybind11::handle dil,
+                      pybind11::handle causal, pybind11::handle scale, const std::optional<at::Tensor>& dlse) {
+    const GlobalCall* c =
+        find(g_gbwd, global_key(bwd_key(rank, dout, q, k, v, out, lse, ks, dil, st, causal, scale, dlse), gk, gv));
+    if (!c) return pybind11::none();
+    return pybind11::cast(c->backward(q, k, v, gk, gv, out, dout, lse, dlse, current_stream(q)));
+}
+
+bool gbwd_register(int64_t rank, const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k,
+                   const at::Tensor& v, const at::Tensor& gk, const at::Tensor& gv, const at::Tensor& out,
+                   const at::Tensor& lse, pybind11::handle ks, pybind11::handle st, pybind11::handle dil,
+                   pybind11::handle causal, pybind11::handle scale, const std::optional<at::Tensor>& dlse,
+                   pybind11::object call) {
+    return remember(g_gbwd,
+                    global_key(bwd_key(rank, dout, q, k, v, out, lse, ks, dil, st, causal, scale, dlse), gk, gv),
                     std::move(call));
 }
 
@@ -650,6 +827,17 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                             std::vector<int64_t>, bool>())
         .def("forward", &FusedCall::forward)
         .def("backward", &FusedCall::backward);
+    pybind11::class_<GlobalCall>(m, "GlobalCall")
+        .def(pybind11::init<const pybind11::bytes&, const pybind11::bytes&, std::vector<int64_t>,
+                            std::vector<int64_t>, int64_t>());
+    m.def("varlen_fwd", &varlen_fwd, "cached variable-length forward: (out, lse), or None");
+    m.def("varlen_fwd_register", &varlen_fwd_register, "register the FusedCall of a variable-length forward");
+    m.def("varlen_bwd", &varlen_bwd, "cached variable-length backward: (dq, dk, dv), or None");
+    m.def("varlen_bwd_register", &varlen_bwd_register, "register the FusedCall of a variable-length backward");
+    m.def("gfwd", &gfwd, "cached forward with global keys: (out, lse), or None");
+    m.def("gfwd_register", &gfwd_register, "register the GlobalCall of a forward with global keys");
+    m.def("gbwd", &gbwd, "cached backward with global keys: (dq, dk, dv, dgk, dgv), or None");
+    m.def("gbwd_register", &gbwd_register, "register the GlobalCall of a backward with global keys");
     m.def("fwd", &fwd, "cached fused forward: (out, lse), or None when the signature is not registered");
     m.def("fwd_register", &fwd_register, "register the FusedCall of a forward signature");
     m.def("bwd", &bwd, "cached fused backward: (dq, dk, dv), or None when the signature is not registered");

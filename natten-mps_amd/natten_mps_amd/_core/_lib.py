@@ -40,6 +40,7 @@ ENTRY_POINTS = (
     "natten_hip_qk_backward",
     "natten_hip_av_backward",
     "natten_hip_neighborhood_map",
+    "natten_hip_varlen_extents",
     "natten_hip_varlen_forward",
     "natten_hip_varlen_backward",
     "natten_hip_rpb_qk_forward",
@@ -103,6 +104,7 @@ _SIGNATURES = {
     "natten_hip_qk_backward": ([_P(Problem)] + [_VP, _LP] * 5 + [_VP], ctypes.c_int),
     "natten_hip_av_backward": ([_P(Problem)] + [_VP, _LP] * 5 + [_VP], ctypes.c_int),
     "natten_hip_neighborhood_map": ([_P(Problem), _VP, _VP, _VP], ctypes.c_int),
+    "natten_hip_varlen_extents": ([_VP, ctypes.c_int32, ctypes.c_int32, _VP, _VP], ctypes.c_int),
     "natten_hip_varlen_forward": ([_P(Problem), _VP] + [_VP, _LP] * 5 + [_VP], ctypes.c_int),
     "natten_hip_varlen_backward": ([_P(Problem), _VP] + [_VP, _LP] * 10 + [_VP], ctypes.c_int),
     "natten_hip_rpb_qk_forward": ([_P(Problem)] + [_VP, _LP] * 2 + [_VP] + [_VP, _LP] + [_VP], ctypes.c_int),

@@ -488,13 +488,25 @@ def neighborhood_map(rank: int, spatial: Sequence[int], kernel_size, dilation, s
 # ---------------------------------------------------------------------------
 
 
-def _varlen_lens(rank: int, sizes: torch.Tensor, device) -> torch.Tensor:
+def varlen_extents(rank: int, sizes: torch.Tensor, device) -> torch.Tensor:
     """Per-sample extents ``[B, rank]`` -> int32 ``[B, 3]`` on the device,
-    padded (leading) axes set to 1."""
-    s = sizes.reshape(sizes.shape[0], rank).to(device=device, dtype=torch.int32)
-    if rank < 3:
-        s = torch.cat([torch.ones((s.shape[0], 3 - rank), dtype=torch.int32, device=device), s], dim=1)
-    return s.contiguous()
+    padded (leading) axes set to 1; a tensor already in that form is returned
+    as it is.  Host extents travel as kernel arguments (no copy that would
+    wait for the stream)."""
+    B = sizes.shape[0]
+    if sizes.device.type == "cuda":
+        if sizes.device == device and sizes.dtype == torch.int32 and sizes.shape == (B, 3) and sizes.is_contiguous():
+            return sizes
+        s = sizes.reshape(B, rank).to(device=device, dtype=torch.int32)
+        if rank < 3:
+            s = torch.cat([torch.ones((B, 3 - rank), dtype=torch.int32, device=device), s], dim=1)
+        return s.contiguous()
+    host = sizes.reshape(B, rank).to(torch.int32).contiguous()
+    lens = torch.empty((B, 3), dtype=torch.int32, device=device)
+    rc = _launch(lens.device, _lib.load().natten_hip_varlen_extents, host.data_ptr(), B, rank, lens.data_ptr(),
+                 _raw_stream(lens.device))
+    _lib.check(rc, "varlen_extents")
+    return lens
 
 
 def _varlen_problem(rank, q, k, v, kernel_size, dilation, scale_value):
@@ -507,10 +519,17 @@ def _varlen_problem(rank, q, k, v, kernel_size, dilation, scale_value):
 def varlen_forward_with_lse(rank: int, q, k, v, sizes, kernel_size, dilation, scale):
     """Fused forward of a padded batch whose sample b has spatial extent
     ``sizes[b]`` (``[B, rank]`` ints): ``(out, lse)``, zero at padding."""
+    _on_device(q, k, v)
+    lens = varlen_extents(rank, sizes, q.device)
+    b = _lib.binding()
+    if b is not None:
+        r = b.varlen_fwd(rank, q, k, v, lens, kernel_size, dilation, scale)
+        if r is not None:
+            return r
+    given = (q, k, v)
     q, k, v = _inner(q), _inner(k), _inner(v)
     scale_value = float(q.shape[-1] ** -0.5 if scale is None else scale)
     prob = _varlen_problem(rank, q, k, v, kernel_size, dilation, scale_value)
-    lens = _varlen_lens(rank, sizes, q.device)
     B, Hq = q.shape[0], q.shape[-2]
     sp = tuple(q.shape[1:1 + rank])
     out = torch.empty((B, *sp, Hq, v.shape[-1]), dtype=q.dtype, device=q.device)
@@ -521,17 +540,27 @@ def varlen_forward_with_lse(rank: int, q, k, v, sizes, kernel_size, dilation, sc
                  q.data_ptr(), L(q), k.data_ptr(), L(k), v.data_ptr(), L(v), out.data_ptr(), L(out),
                  lse.data_ptr(), L(lse, 0), _raw_stream(q.device))
     _lib.check(rc, "varlen_forward")
+    if b is not None and all(a is u for a, u in zip(given, (q, k, v))):
+        lays = [_lib.layout(t, rank, 1) for t in (q, k, v, out)] + [_lib.layout(lse, rank, 0)]
+        call = b.FusedCall(bytes(prob), b"".join(bytes(x) for x in lays), list(out.shape), list(lse.shape), False)
+        b.varlen_fwd_register(rank, q, k, v, lens, kernel_size, dilation, scale, call)
     return out, lse
 
 
 def varlen_backward(rank: int, d_out, q, k, v, out, lse, sizes, kernel_size, dilation, scale):
     """``(dq, dk, dv)`` of :func:`varlen_forward_with_lse`, zero at padding."""
+    _on_device(q, k, v, d_out, out, lse)
+    lens = varlen_extents(rank, sizes, q.device)
+    b = _lib.binding()
+    if b is not None:
+        r = b.varlen_bwd(rank, d_out, q, k, v, out, lse, lens, kernel_size, dilation, scale)
+        if r is not None:
+            return r
+    given = (q, k, v, out, d_out, lse)
     q, k, v, out, d_out = _inner(q), _inner(k), _inner(v), _inner(out), _inner(d_out.to(q.dtype))
     lse = lse.to(torch.float32).contiguous()
     scale_value = float(q.shape[-1] ** -0.5 if scale is None else scale)
     prob = _varlen_problem(rank, q, k, v, kernel_size, dilation, scale_value)
-    _on_device(d_out, out, lse)
-    lens = _varlen_lens(rank, sizes, q.device)
     dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     dk = torch.empty(k.shape, dtype=k.dtype, device=k.device)
     dv = torch.empty(v.shape, dtype=v.dtype, device=v.device)
@@ -544,6 +573,11 @@ def varlen_backward(rank: int, d_out, q, k, v, out, lse, sizes, kernel_size, dil
                  dk.data_ptr(), L(dk), dv.data_ptr(), L(dv), delta.data_ptr(), L(delta, 0),
                  _raw_stream(q.device))
     _lib.check(rc, "varlen_backward")
+    if b is not None and all(a is u for a, u in zip(given, (q, k, v, out, d_out, lse))):
+        lays = [_lib.layout(t, rank, 1) for t in (q, k, v, out, d_out)] + [_lib.layout(lse, rank, 0), _lib.Layout()]
+        lays += [_lib.layout(t, rank, 1) for t in (dq, dk, dv)] + [_lib.layout(delta, rank, 0)]
+        call = b.FusedCall(bytes(prob), b"".join(bytes(x) for x in lays), [], list(lse.shape), False)
+        b.varlen_bwd_register(rank, d_out, q, k, v, out, lse, lens, kernel_size, dilation, scale, call)
     return dq, dk, dv
 
 
@@ -744,6 +778,12 @@ def _check_global(q, k, gk, gv):
 def forward_with_lse_global(rank: int, q, k, v, gk, gv, kernel_size, stride, dilation, is_causal, scale):
     """(out, lse) of neighbourhood attention plus global keys: one softmax
     over each query's window and the N global keys (lse fp32)."""
+    b = _lib.binding()
+    if b is not None:
+        r = b.gfwd(rank, q, k, v, gk, gv, kernel_size, stride, dilation, is_causal, scale)
+        if r is not None:
+            return r
+    given = (q, k, v, gk, gv)
     q, k, v, gk, gv = _inner(q), _inner(k), _inner(v), _inner(gk), _inner(gv)
     _check_global(q, k, gk, gv)
     scale_value = float(q.shape[-1] ** -0.5 if scale is None else scale)
@@ -757,12 +797,22 @@ def forward_with_lse_global(rank: int, q, k, v, gk, gv, kernel_size, stride, dil
                  gv.data_ptr(), _byref(lgv), int(gk.shape[1]), out.data_ptr(), r[3], lse.data_ptr(), r[4],
                  _raw_stream(q.device))
     _lib.check(rc, "forward_global")
+    if b is not None and all(a is u for a, u in zip(given, (q, k, v, gk, gv))):
+        blob = b"".join(bytes(x) for x in (*sig.refs[0], lgk, lgv))
+        call = b.GlobalCall(bytes(sig.prob), blob, list(sig.out_shape), list(sig.lse_shape), 0)
+        b.gfwd_register(rank, q, k, v, gk, gv, kernel_size, stride, dilation, is_causal, scale, call)
     return out, lse
 
 
 def fused_backward_global(rank: int, d_out, q, k, v, gk, gv, out, lse, kernel_size, dilation, stride, is_causal,
                           scale, d_lse=None):
     """(dq, dk, dv, dgk, dgv) of forward_with_lse_global."""
+    b = _lib.binding()
+    if b is not None:
+        r = b.gbwd(rank, d_out, q, k, v, gk, gv, out, lse, kernel_size, stride, dilation, is_causal, scale, d_lse)
+        if r is not None:
+            return r
+    given = (d_out, q, k, v, gk, gv, out, lse, d_lse)
     q, k, v, out, d_out, gk, gv = (_inner(t) for t in (q, k, v, out, d_out, gk, gv))
     _check_global(q, k, gk, gv)
     if lse.dtype != torch.float32 or not lse.is_contiguous():
@@ -792,6 +842,12 @@ def fused_backward_global(rank: int, d_out, q, k, v, gk, gv, out, lse, kernel_si
                  dv.data_ptr(), r[9], dgk.data_ptr(), T(dgk), dgv.data_ptr(), T(dgv), delta.data_ptr(), r[10],
                  work.data_ptr(), work_floats, _raw_stream(q.device))
     _lib.check(rc, "backward_global")
+    if b is not None and all(a is u for a, u in zip(given, (d_out, q, k, v, gk, gv, out, lse, d_lse))):
+        lays = [x if x is not None else _lib.Layout() for x in sig.refs[0]]
+        blob = b"".join(bytes(x) for x in (*lays, *(_lib.token_layout(t) for t in (gk, gv, dgk, dgv))))
+        call = b.GlobalCall(bytes(sig.prob), blob, [], list(sig.lse_shape), work_floats)
+        b.gbwd_register(rank, d_out, q, k, v, gk, gv, out, lse, kernel_size, stride, dilation, is_causal, scale,
+                        d_lse, call)
     return dq, dk, dv, dgk, dgv
 
 

@@ -145,6 +145,8 @@ def create_na_lse_autograd_fn(rank: int) -> type:
             out, lse = getattr(mod, f"na{rank}d_forward_with_lse")(q, k, v, kernel_size, stride, dilation,
                                                                    is_causal, scale)
             ctx.save_for_backward(q, k, v, lse, out)
+            # an output that nothing uses comes back as None, not as zeros
+            ctx.set_materialize_grads(False)
             return out, lse
 
         @staticmethod
@@ -182,6 +184,8 @@ def create_na_global_autograd_fn(rank: int) -> type:
             out, lse = getattr(mod, f"na{rank}d_forward_with_lse_global")(q, k, v, gk, gv, kernel_size, stride,
                                                                           dilation, is_causal, scale)
             ctx.save_for_backward(q, k, v, gk, gv, lse, out)
+            # an output that nothing uses comes back as None, not as zeros
+            ctx.set_materialize_grads(False)
             return out, lse
 
         @staticmethod

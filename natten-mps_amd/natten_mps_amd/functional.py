@@ -425,6 +425,10 @@ class _NAVarlenFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, rank, mod, query, key, value, sizes, ks, dil, scale):
+        # the backend's own form of the extents, made once for both directions
+        extents = getattr(mod, "varlen_extents", None)
+        if extents is not None and query.is_cuda:
+            sizes = extents(rank, sizes, query.device)
         out, lse = getattr(mod, f"na{rank}d_varlen_forward_with_lse")(query, key, value, sizes, ks, dil, scale)
         ctx.rank, ctx.mod, ctx.ks, ctx.dil, ctx.scale = rank, mod, ks, dil, scale
         ctx.save_for_backward(query, key, value, out, lse, sizes)
@@ -468,8 +472,9 @@ def _varlen(rank, query, key, value, sizes, kernel_size, dilation, scale):
         _validate_seq_lens(sizes, B, max_sp[0], ks[0], rows=host)
     else:
         _validate_spatial_sizes(sizes, B, max_sp, ks, rank, rows=host)
-    sizes2 = sizes.reshape(B, rank)
     rows = [[int(x)] for x in host] if rank == 1 else [[int(x) for x in r] for r in host]
+    # sizes that live on the device continue as their host copy
+    sizes2 = sizes.reshape(B, rank) if sizes.device.type == "cpu" else torch.tensor(rows, dtype=torch.int32)
     # a sample's extent must hold the dilated kernel, as na*d on its slice requires
     for ext in {tuple(row) for row in rows}:
         check_dilation_kernel_vs_input(dil, ks, ext)
