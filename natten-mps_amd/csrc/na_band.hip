@@ -782,7 +782,7 @@ template <typename T, int D>
 hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                         const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll, const float* dlse,
                         Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv, float* delta, Lay lde,
-                        hipStream_t s) {
+                        int sides, hipStream_t s) {
     BandArgs<T> a{};
     a.p = p;
     a.g = band_geo(p, band_columns(p.ax[2].k, false), p.Hq);
@@ -811,12 +811,15 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
     a.ldl = to_k(ldl);
     a.ab = band_plane(p, lk, D);
     a.bb = band_plane(p, lv, D);
-    auto kq = k_band_bwd_q<T, D, 32>;
-    hipError_t e = allow_lds(kq, kBandLds<T, D>);
-    if (e != hipSuccess) return e;
-    NA_LAUNCH("na_bwd_q_band", kq, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
-              (kBandLds<T, D>), s, a);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipError_t e;
+    if (sides & kQuerySide) {
+        auto kq = k_band_bwd_q<T, D, 32>;
+        if ((e = allow_lds(kq, kBandLds<T, D>)) != hipSuccess) return e;
+        NA_LAUNCH("na_bwd_q_band", kq, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
+                  (kBandLds<T, D>), s, a);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    if (!(sides & kKeySide)) return hipSuccess;
     a.g = band_geo(p, band_columns(p.ax[2].k, true), p.Hkv);
     a.ab = band_plane(p, lq, D);
     a.bb = band_plane(p, ldo, D);
@@ -839,26 +842,38 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
 
 }  // namespace
 
-// 2-D problems (axis 0 of extent 1) at stride 1, 16-bit, head dim 32 / 64 /
-// 128 for q, k and v, whose windows span 10 to 16 columns (so that a tile's
-// union fits 32): the range past the 8x8 tile kernels.  `lays`: every 16-bit
-// operand and fp32 row operand of the call.
-bool band_eligible(const Prob& p, int dtype, bool aligned, std::initializer_list<Lay> lays) {
-    if (!band_switch() || !aligned || dtype == NATTEN_F32 || !(p.scale > 0.f)) return false;
-    if (p.Dqk != p.Dv || (p.Dqk != 32 && p.Dqk != 64 && p.Dqk != 128)) return false;
-    if (p.ax[0].len != 1 || p.ax[0].k != 1) return false;
+// The sides of a problem that run on these kernels: 2-D (axis 0 of extent 1)
+// at stride 1, 16-bit, head dim 32 / 64 / 128 for q, k and v, in-plane
+// kernel of 2 to 16 columns (so that a tile's union fits 32), and
+// * both sides for 10 to 16 columns (past the 8x8 tile kernels), and at head
+//   dim 128 from 8: there the general tiles' border unions cross 16 columns
+//   and their rows double (9 x 9, 8 x 64 x 64 x 4 heads: forward 97 -> 61
+//   us, the backward left the tiles, 995 + 950 -> 110 + 94 us; at 7 x 7 both
+//   are level, 57 + 76 + 90 against 58 + 99 + 87);
+// * the key side alone where the 8x8 tiles serve the query side but some key
+//   tile's union does not fit them (`lean`: they take the problem; 9 x 9, 8 x
+//   64 x 64 x 8: dK/dV 222 -> 56 us at head dim 32, 613 -> 111 at 64; 7 x 7
+//   on 32 x 22 x 22 x 8: 57 -> 37).
+// `lays`: every 16-bit operand and fp32 row operand of the call.  The answer
+// depends on the problem alone, never on which tables exist.
+int band_sides(const Prob& p, int dtype, bool aligned, bool lean, std::initializer_list<Lay> lays) {
+    if (!band_switch() || !aligned || dtype == NATTEN_F32 || !(p.scale > 0.f)) return 0;
+    if (p.Dqk != p.Dv || (p.Dqk != 32 && p.Dqk != 64 && p.Dqk != 128)) return 0;
+    if (p.ax[0].len != 1 || p.ax[0].k != 1) return 0;
     for (int a = 0; a < 3; ++a)
-        if (p.ax[a].st != 1 || p.ax[a].len >= (1 << 24)) return false;
-    if (p.ax[2].k < 10 || band_columns(p.ax[2].k, true) < 0) return false;
+        if (p.ax[a].st != 1 || p.ax[a].len >= (1 << 24)) return 0;
+    if (band_columns(p.ax[2].k, true) < 0) return 0;
     // a tile has at least 8 rows: fewer would leave its waves idle
-    if (n_class_h(p.ax[1], 0) < 8) return false;
-    if (!offsets_fit(p, lays)) return false;
+    if (n_class_h(p.ax[1], 0) < 8) return 0;
+    const bool both = p.ax[2].k >= (p.Dqk == 128 ? 8 : 10);
+    if (!both && !(lean && !lean_key_tiles_fit(p))) return 0;
+    if (!offsets_fit(p, lays)) return 0;
     for (const Lay& l : lays)
-        if (band_plane(p, l, p.Dqk) >= kBandOOR) return false;
+        if (band_plane(p, l, p.Dqk) >= kBandOOR) return 0;
     const long long tiles = ((static_cast<long long>(p.ax[1].len) + 7) / 8 + p.ax[1].dil) *
                             ((static_cast<long long>(p.ax[2].len) + 7) / 8 + p.ax[2].dil);
-    if (tiles * p.B * p.Hq >= (1LL << 31)) return false;
-    return band_static_lds_ok();
+    if (tiles * p.B * p.Hq >= (1LL << 31) || !band_static_lds_ok()) return 0;
+    return both ? kQuerySide | kKeySide : kKeySide;
 }
 
 hipError_t band_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,
@@ -869,9 +884,9 @@ hipError_t band_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay
 hipError_t band_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                          const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll, const float* dlse,
                          Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv, float* delta, Lay lde,
-                         int dtype, hipStream_t s) {
+                         int dtype, hipStream_t s, int sides) {
     NA_BAND_DISPATCH(band_bwd_run, p, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
-                     ldv, delta, lde, s);
+                     ldv, delta, lde, sides, s);
 }
 
 }  // namespace na

@@ -186,8 +186,9 @@ int natten_hip_forward(const natten_problem_t* p, const void* q, const natten_la
                                               to_lay(llse), p->dtype, s);
         if (e != hipErrorNotSupported) return launch_status(e, "forward");
     }
-    if (use_mfma() && na::band_eligible(P, p->dtype, vec != 0,
-                                        {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)}))
+    if (use_mfma() && (na::band_sides(P, p->dtype, vec != 0, false,
+                                      {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)}) &
+                       na::kQuerySide))
         return launch_status(na::band_forward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), lse,
                                               to_lay(llse), p->dtype, s),
                              "forward");
@@ -204,6 +205,54 @@ int natten_hip_forward(const natten_problem_t* p, const void* q, const natten_la
 
 namespace {
 
+// Operands of a backward call, for the launchers of the tile kernels.
+struct BackwardCall {
+    const na::Prob& P;
+    int dtype, vec;
+    const void *q, *k, *v, *o, *dout;
+    na::Lay lq, lk, lv, lo, ldo;
+    const float* lse;
+    na::Lay ll;
+    const float* dlse;
+    na::Lay ldl;
+    void *dq, *dk, *dv;
+    na::Lay ldq, ldk, ldv;
+    float* delta;
+    na::Lay lde;
+    hipStream_t s;
+
+    bool lean_ok() const {
+        return use_mfma() &&
+               na::lean_eligible(P, dtype, vec != 0, {lq, lo, ldo, ldq}, {lk, lv, ldk, ldv},
+                                 dlse ? std::initializer_list<na::Lay>{ll, lde, ldl}
+                                      : std::initializer_list<na::Lay>{ll, lde});
+    }
+    int band_sides(bool lean) const {
+        return use_mfma() ? na::band_sides(P, dtype, vec != 0, lean,
+                                           {lq, lk, lv, lo, ldo, ll, ldq, ldk, ldv, lde, dlse ? ldl : ll})
+                          : 0;
+    }
+    bool mfma_ok(int sides) const {
+        return use_mfma() && na::mfma_eligible(P, dtype, P.Dqk > P.Dv ? P.Dqk : P.Dv, vec != 0, true, false, sides) &&
+               na::mfma_offsets_fit(P, {lq, lk, lv, lo, ldo, ll, ldq, ldk, ldv, lde}) &&
+               (!dlse || na::mfma_offsets_fit(P, {ldl}));
+    }
+    hipError_t lean(int sides) const {
+        return na::lean_backward(P, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
+                                 ldv, delta, lde, dtype, s, sides);
+    }
+    hipError_t band(int sides) const {
+        return na::band_backward(P, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
+                                 ldv, delta, lde, dtype, s, sides);
+    }
+    hipError_t mfma(int sides, const na::GlobalSet* g = nullptr) const {
+        return na::mfma_backward(P, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
+                                 ldv, delta, lde, dtype, s, g, sides);
+    }
+};
+
+constexpr int kBothSides = na::kQuerySide | na::kKeySide;
+
 // Shared body of the two backward entry points (the problem already checked).
 int backward_impl(const natten_problem_t* p, const na::Prob& P, const void* q, const natten_layout_t* lq,
                   const void* k, const natten_layout_t* lk, const void* v, const natten_layout_t* lv,
@@ -219,43 +268,29 @@ int backward_impl(const natten_problem_t* p, const na::Prob& P, const void* q, c
                                               {dout, ldo, P.Dv}, {dq, ldq, P.Dqk}, {dk, ldk, P.Dqk}, {dv, ldv, P.Dv}})
                         ? 1
                         : 0;
-    // the lean 2-D tiles first (their checks are cheap), then the general tiles
-    if (use_mfma() &&
-        na::lean_eligible(P, p->dtype, vec != 0, {to_lay(lq), to_lay(lo), to_lay(ldo), to_lay(ldq)},
-                          {to_lay(lk), to_lay(lv), to_lay(ldk), to_lay(ldv)},
-                          dlse ? std::initializer_list<na::Lay>{to_lay(llse), to_lay(ldelta), to_lay(ldlse)}
-                               : std::initializer_list<na::Lay>{to_lay(llse), to_lay(ldelta)})) {
-        const hipError_t e = na::lean_backward(
-            P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), dout, to_lay(ldo), lse, to_lay(llse),
-            dlse, to_lay(ldlse), dq, to_lay(ldq), dk, to_lay(ldk), dv, to_lay(ldv), delta, to_lay(ldelta), p->dtype,
-            static_cast<hipStream_t>(stream));
+    const BackwardCall c{P, p->dtype, vec, q, k, v, out, dout, to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo),
+                         to_lay(ldo), lse, to_lay(llse), dlse, to_lay(ldlse), dq, dk, dv, to_lay(ldq), to_lay(ldk),
+                         to_lay(ldv), delta, to_lay(ldelta), static_cast<hipStream_t>(stream)};
+    // the lean tiles first, the band kernels for what their unions cannot
+    // hold, then the general tiles
+    const bool lean = c.lean_ok();
+    const int band = c.band_sides(lean);
+    if (band == kBothSides) return launch_status(c.band(kBothSides), "backward");
+    if (band == na::kKeySide) {
+        // the query side as without the band kernels (the general tiles give
+        // the lean ones' bits where no table of those exists)
+        hipError_t e = c.lean(na::kQuerySide);
+        if (e == hipErrorNotSupported) e = c.mfma_ok(na::kQuerySide) ? c.mfma(na::kQuerySide) : c.band(na::kQuerySide);
+        return launch_status(e == hipSuccess ? c.band(na::kKeySide) : e, "backward");
+    }
+    if (lean) {
+        const hipError_t e = c.lean(kBothSides);
         if (e != hipErrorNotSupported) return launch_status(e, "backward");
     }
-    if (use_mfma() &&
-        na::band_eligible(P, p->dtype, vec != 0,
-                          {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(ldo), to_lay(llse), to_lay(ldq),
-                           to_lay(ldk), to_lay(ldv), to_lay(ldelta), dlse ? to_lay(ldlse) : to_lay(llse)})) {
-        return launch_status(na::band_backward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), dout,
-                                               to_lay(ldo), lse, to_lay(llse), dlse, to_lay(ldlse), dq, to_lay(ldq),
-                                               dk, to_lay(ldk), dv, to_lay(ldv), delta, to_lay(ldelta), p->dtype,
-                                               static_cast<hipStream_t>(stream)),
-                             "backward");
-    }
-    if (use_mfma() && na::mfma_eligible(P, p->dtype, D, vec != 0, true) &&
-        na::mfma_offsets_fit(P, {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(ldo), to_lay(llse),
-                                 to_lay(ldq), to_lay(ldk), to_lay(ldv), to_lay(ldelta)}) &&
-        (!dlse || na::mfma_offsets_fit(P, {to_lay(ldlse)}))) {
-        return launch_status(na::mfma_backward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), dout,
-                                               to_lay(ldo), lse,
-                                               to_lay(llse), dlse, to_lay(ldlse), dq, to_lay(ldq), dk, to_lay(ldk), dv,
-                                               to_lay(ldv), delta, to_lay(ldelta), p->dtype,
-                                               static_cast<hipStream_t>(stream)),
-                             "backward");
-    }
+    if (c.mfma_ok(kBothSides)) return launch_status(c.mfma(kBothSides), "backward");
     return launch_status(
-        na::generic_backward(P, vec, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), dout, to_lay(ldo),
-                             lse, to_lay(llse), dlse, to_lay(ldlse), dq, to_lay(ldq), dk, to_lay(ldk), dv,
-                             to_lay(ldv), delta, to_lay(ldelta), p->dtype, static_cast<hipStream_t>(stream)),
+        na::generic_backward(P, vec, q, c.lq, k, c.lk, v, c.lv, out, c.lo, dout, c.ldo, lse, c.ll, dlse, c.ldl, dq,
+                             c.ldq, dk, c.ldk, dv, c.ldv, delta, c.lde, p->dtype, c.s),
         "backward");
 }
 
@@ -445,10 +480,22 @@ int natten_hip_backward_global(const natten_problem_t* p, const void* q, const n
                     "global keys run on the MFMA tile kernels only (bf16/fp16, head dim 32/64/96/128, stride 1, "
                     "aligned operands)");
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    rc = launch_status(na::mfma_backward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), dout,
-                                         to_lay(ldo), lse, to_lay(llse), dlse, to_lay(ldlse), dq, to_lay(ldq), dk,
-                                         to_lay(ldk), dv, to_lay(ldv), delta, to_lay(ldelta), p->dtype, s, &g),
-                       "backward_global");
+    const BackwardCall c{P, p->dtype, vec, q, k, v, out, dout, to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo),
+                         to_lay(ldo), lse, to_lay(llse), dlse, to_lay(ldlse), dq, dk, dv, to_lay(ldq), to_lay(ldk),
+                         to_lay(ldv), delta, to_lay(ldelta), s};
+    // the window's key side knows nothing of the global keys: it runs where
+    // it would without them
+    hipError_t e = c.mfma(na::kQuerySide, &g);
+    if (e == hipSuccess) {
+        const bool lean = c.lean_ok();
+        if (c.band_sides(lean) & na::kKeySide) {
+            e = c.band(na::kKeySide);
+        } else {
+            e = lean ? c.lean(na::kKeySide) : hipErrorNotSupported;
+            if (e == hipErrorNotSupported) e = c.mfma(na::kKeySide);
+        }
+    }
+    rc = launch_status(e, "backward_global");
     if (rc) return rc;
     return launch_status(na::mfma_global_key_backward(P, q, to_lay(lq), dout, to_lay(ldo), lse, to_lay(llse), delta,
                                                       to_lay(ldelta), g, dgk, to_lay(ldgk), dgv, to_lay(ldgv), work,

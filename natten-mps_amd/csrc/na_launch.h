@@ -110,8 +110,10 @@ struct GlobalSet {
 // number of instances whose attributes were read.
 bool mfma_static_lds_ok();
 int mfma_lds_audit(int* checked);
-// `global`: with global keys (their LDS on top of the tiles').
-bool mfma_eligible(const Prob& p, int dtype, int D, bool aligned, bool backward, bool global = false);
+// `global`: with global keys (their LDS on top of the tiles'); `sides`: of
+// the backward.
+bool mfma_eligible(const Prob& p, int dtype, int D, bool aligned, bool backward, bool global = false,
+                   int sides = kQuerySide | kKeySide);
 bool mfma_offsets_fit(const Prob& p, std::initializer_list<Lay> lays);
 
 // Variable-length fused forward / backward on the MFMA tile kernels: the
@@ -131,7 +133,8 @@ hipError_t mfma_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay
 hipError_t mfma_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                          const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll,
                          const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
-                         float* delta, Lay lde, int dtype, hipStream_t s, const GlobalSet* g = nullptr);
+                         float* delta, Lay lde, int dtype, hipStream_t s, const GlobalSet* g = nullptr,
+                         int sides = kQuerySide | kKeySide);
 
 // Lean 2-D tile kernels (na_lean.hip): 2-D problems at stride 1, bf16/fp16,
 // head dim 32 or 64, kernel sizes up to 9, q-side and k-side operands each
@@ -154,18 +157,21 @@ hipError_t lean_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay
 hipError_t lean_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                          const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll,
                          const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
-                         float* delta, Lay lde, int dtype, hipStream_t s);
+                         float* delta, Lay lde, int dtype, hipStream_t s, int sides = kQuerySide | kKeySide);
+// A 2-D problem's key tiles fit the key-side kernels (lean_eligible aside).
+bool lean_key_tiles_fit(const Prob& p);
 
 // Band kernels (na_band.hip): 2-D problems at stride 1, 16-bit, head dim 32,
-// 64 or 128, in-plane kernels of 10 to 16 columns; no tables, so every
-// eligible call has a launch.
-bool band_eligible(const Prob& p, int dtype, bool aligned, std::initializer_list<Lay> lays);
+// 64 or 128.  band_sides: the sides (kQuerySide, kKeySide) of a problem that
+// run on them; no tables, so each has a launch in every call.  `lean`: the
+// 8x8 tile kernels take the problem's query side.
+int band_sides(const Prob& p, int dtype, bool aligned, bool lean, std::initializer_list<Lay> lays);
 hipError_t band_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,
                         Lay lo, float* lse, Lay ll, int dtype, hipStream_t s);
 hipError_t band_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                          const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll,
                          const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
-                         float* delta, Lay lde, int dtype, hipStream_t s);
+                         float* delta, Lay lde, int dtype, hipStream_t s, int sides = kQuerySide | kKeySide);
 
 // Key side of the global keys' backward (na_global.hip): dk and dv of the
 // global keys (summed over every query of each q head of the group), from the

@@ -1909,42 +1909,91 @@ LeanBwdArgs<T> lean_bwd_args(const Prob& p, const void* q, Lay lq, const void* k
     return a;
 }
 
+// sides: gq is read for the query side, gk for the key side.
 template <typename T, int D, int NCH, bool D3, bool ONE_D = false, int HP = 1>
-hipError_t lean_bwd_run(const Prob& p, const LeanGeo* gq, const LeanGeo* gk, const LeanBwdArgs<T>& base,
+hipError_t lean_bwd_run(const Prob& p, const LeanGeo* gq, const LeanGeo* gk, const LeanBwdArgs<T>& base, int sides,
                         hipStream_t s) {
-    LeanBwdArgs<T> a = base;
-    a.rec = gq->ptr;
-    a.rec_k = gk->ptr;
-    a.dec = lean_decode(p, p.Hq / HP, gq->ntiles);
-    a.nr = std::max(gk->nst_max, 1);
+    const int ntiles = (sides & kQuerySide ? gq : gk)->ntiles;
+    const long long tasks = static_cast<long long>(p.B) * (p.Hq / HP) * ntiles * p.ax[0].len;
     const size_t shm_q = kLdsPad + static_cast<size_t>(2) * lean_rows<ONE_D>(NCH) * 16 * D * sizeof(T);
+    const int nr = gk ? std::max(gk->nst_max, 1) : 1;
     const size_t shm_k =
-        kLdsPad + static_cast<size_t>(a.nr) * 16 * (2 * D * sizeof(T) + 2 * sizeof(float)) + 8 * sizeof(float);
-    const long long tasks = static_cast<long long>(p.B) * (p.Hq / HP) * gq->ntiles * p.ax[0].len;
+        kLdsPad + static_cast<size_t>(nr) * 16 * (2 * D * sizeof(T) + 2 * sizeof(float)) + 8 * sizeof(float);
     if (tasks >= (1LL << 31) || shm_q > 160 * 1024 || shm_k > 160 * 1024) return hipErrorNotSupported;
-    auto kq = k_lean_bwd_q<T, D, NCH, D3, ONE_D, HP>;
-    hipError_t e = allow_lds(kq, shm_q);
-    if (e != hipSuccess) return e;
-    NA_LAUNCH("na_bwd_q_lean", kq, dim3(static_cast<unsigned>(tasks)), dim3(64 * kLeanWaves * HP), shm_q, s, a);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    hipError_t e;
+    if (sides & kQuerySide) {
+        LeanBwdArgs<T> a = base;
+        a.rec = gq->ptr;
+        a.dec = lean_decode(p, p.Hq / HP, ntiles);
+        auto kq = k_lean_bwd_q<T, D, NCH, D3, ONE_D, HP>;
+        e = allow_lds(kq, shm_q);
+        if (e != hipSuccess) return e;
+        NA_LAUNCH("na_bwd_q_lean", kq, dim3(static_cast<unsigned>(tasks)), dim3(64 * kLeanWaves * HP), shm_q, s, a);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    if (!(sides & kKeySide)) return hipSuccess;
     auto kern = gk->rows_max <= 2 * (NCH + 2) ? k_lean_bwd_kv<T, D, NCH + 2, D3, ONE_D>
                                               : k_lean_bwd_kv<T, D, kLeanMaxKeyChunks, D3, ONE_D>;
     if ((e = allow_lds(kern, shm_k)) != hipSuccess) return e;
     // key tiles over the kv heads, each walking the q heads of its group
-    LeanBwdArgs<T> ak = a;
-    ak.dec = lean_decode(p, p.Hkv, gq->ntiles);
-    const long long ktasks = static_cast<long long>(p.B) * p.Hkv * gq->ntiles * p.ax[0].len;
+    LeanBwdArgs<T> ak = base;
+    ak.rec_k = gk->ptr;
+    ak.nr = nr;
+    ak.dec = lean_decode(p, p.Hkv, ntiles);
+    const long long ktasks = static_cast<long long>(p.B) * p.Hkv * ntiles * p.ax[0].len;
     NA_LAUNCH("na_bwd_kv_lean", kern, dim3(static_cast<unsigned>(ktasks)), dim3(64 * kLeanWaves), shm_k, s, ak);
     return hipGetLastError();
 }
 
-// Backward on the lean kernels; hipErrorNotSupported
-// when this problem has no lean launch.
+// The key tiles of a 2-D problem fit the key-side kernels: every tile's
+// union (the queries attending its keys) at most 16 columns wide and 32
+// staged rows high, a wave's own rows within the widest instance.  The
+// borders widen a union: at K = 8 and 9 a tile next to one reaches 20
+// columns, at K = 7 a class of 22 makes one of 17.  The same conditions as
+// lean_geometry's, from the extents alone; kept per axis geometry.
+bool lean_key_tiles_fit(const Prob& p) {
+    struct Entry {
+        int len, k, dil, causal, u, rows, nst;
+    };
+    static std::mutex mu;
+    static std::vector<Entry> cache;
+    const auto axis = [](const Axis& A) {
+        {
+            std::lock_guard<std::mutex> g(mu);
+            for (const Entry& e : cache)
+                if (e.len == A.len && e.k == A.k && e.dil == A.dil && e.causal == A.causal) return e;
+        }
+        Entry e{A.len, A.k, A.dil, A.causal, 0, 0, 0};
+        for (int r = 0; r < A.dil; ++r) {
+            const int n = (A.len - r + A.dil - 1) / A.dil;
+            for (int t = 0; t < (n + 7) / 8; ++t) {
+                LeanAxisTile a;
+                if (!lean_axis_tile(A, r, t, true, a)) continue;
+                e.u = std::max(e.u, a.U);
+                for (int w = 0; w < 4; ++w) {
+                    const int rows = a.we[2 * w + 1] - a.ws[2 * w] + 1;
+                    e.rows = std::max(e.rows, rows);
+                    e.nst = std::max(e.nst, a.ws[2 * w] + 2 * ((std::max(rows, 0) + 1) / 2));
+                }
+                e.nst = std::max(e.nst, a.U);
+            }
+        }
+        std::lock_guard<std::mutex> g(mu);
+        if (cache.size() >= 512) cache.clear();
+        cache.push_back(e);
+        return e;
+    };
+    const Entry a1 = axis(p.ax[1]), a2 = axis(p.ax[2]);
+    return a2.u <= 16 && a1.rows <= 2 * kLeanMaxKeyChunks && a1.nst <= 32;
+}
+
+// Backward on the lean kernels (the sides asked for); hipErrorNotSupported,
+// with nothing launched, when this problem has no lean launch.
 hipError_t lean_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                          const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll,
                          const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
-                         float* delta, Lay lde, int dtype, hipStream_t s) {
+                         float* delta, Lay lde, int dtype, hipStream_t s, int sides) {
     (void)lv;
     (void)ldv;
     if (!same_lay(ll, lde) || (dlse && !same_lay(ll, ldl))) return hipErrorNotSupported;
@@ -1952,22 +2001,24 @@ hipError_t lean_backward(const Prob& p, const void* q, Lay lq, const void* k, La
     const bool d1 = lean_1d(p), d3 = lean_3d(p);
     if (d3 && dtype != NATTEN_F32) return hipErrorNotSupported;  // 3-D instances exist for fp32 only
     const int nch = d1 ? lean_nch_1d(p.ax[2].k) : lean_nch(p.ax[1].k);
-    const LeanGeo* gq = lean_geometry(p, 0, nch, s);
-    const LeanGeo* gk = gq ? lean_geometry(p, 1, nch, s) : nullptr;
-    if (!gq || !gk || gq->ntiles != gk->ntiles || gk->rows_max > 2 * kLeanMaxKeyChunks) return hipErrorNotSupported;
+    const LeanGeo* gq = sides & kQuerySide ? lean_geometry(p, 0, nch, s) : nullptr;
+    if ((sides & kQuerySide) && !gq) return hipErrorNotSupported;
+    const LeanGeo* gk = sides & kKeySide ? lean_geometry(p, 1, nch, s) : nullptr;
+    if ((sides & kKeySide) && (!gk || gk->rows_max > 2 * kLeanMaxKeyChunks)) return hipErrorNotSupported;
+    if (gq && gk && gq->ntiles != gk->ntiles) return hipErrorNotSupported;
 #define NA_LB_A(T, DD) \
     lean_bwd_args<T, DD>(p, q, lq, k, lk, v, o, lo, dout, ldo, lse, ll, dlse, dq, ldq, dk, ldk, dv, delta)
     // GQA with an even group: two q heads per dQ workgroup share the staged K/V
     const bool pairs = p.rep % 2 == 0 && lean_head_pairs();
 #define NA_LB(T, DD, N)                                                                          \
-    return d1 ? (pairs ? lean_bwd_run<T, DD, N, false, true, 2>(p, gq, gk, NA_LB_A(T, DD), s)     \
-                       : lean_bwd_run<T, DD, N, false, true>(p, gq, gk, NA_LB_A(T, DD), s))       \
-              : (pairs ? lean_bwd_run<T, DD, N, false, false, 2>(p, gq, gk, NA_LB_A(T, DD), s)    \
-                       : lean_bwd_run<T, DD, N, false>(p, gq, gk, NA_LB_A(T, DD), s))
+    return d1 ? (pairs ? lean_bwd_run<T, DD, N, false, true, 2>(p, gq, gk, NA_LB_A(T, DD), sides, s)     \
+                       : lean_bwd_run<T, DD, N, false, true>(p, gq, gk, NA_LB_A(T, DD), sides, s))       \
+              : (pairs ? lean_bwd_run<T, DD, N, false, false, 2>(p, gq, gk, NA_LB_A(T, DD), sides, s)    \
+                       : lean_bwd_run<T, DD, N, false>(p, gq, gk, NA_LB_A(T, DD), sides, s))
 #define NA_LB3(T, DD, N)                                                              \
-    return d1 ? lean_bwd_run<T, DD, N, false, true>(p, gq, gk, NA_LB_A(T, DD), s)     \
-              : (d3 ? lean_bwd_run<T, DD, N, true>(p, gq, gk, NA_LB_A(T, DD), s)      \
-                    : lean_bwd_run<T, DD, N, false>(p, gq, gk, NA_LB_A(T, DD), s))
+    return d1 ? lean_bwd_run<T, DD, N, false, true>(p, gq, gk, NA_LB_A(T, DD), sides, s)     \
+              : (d3 ? lean_bwd_run<T, DD, N, true>(p, gq, gk, NA_LB_A(T, DD), sides, s)      \
+                    : lean_bwd_run<T, DD, N, false>(p, gq, gk, NA_LB_A(T, DD), sides, s))
 #define NA_LB_N(T, DD, F)    \
     switch (nch) {           \
         case 1: F(T, DD, 1); \

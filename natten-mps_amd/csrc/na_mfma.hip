@@ -1728,16 +1728,20 @@ template <typename T, int D, int LAY, bool GLOBAL>
 hipError_t launch_bwd(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                       const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll,
                       const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
-                      float* delta, Lay lde, const GlobalSet* g, hipStream_t s) {
+                      float* delta, Lay lde, const GlobalSet* g, int sides, hipStream_t s) {
     TileShape tq{}, tk{};
-    if (!choose_tile(p, kBackwardQ, D, tq, GLOBAL ? global_lds(D) : 0) || !choose_tile(p, kBackwardKV, D, tk))
+    if (((sides & kQuerySide) && !choose_tile(p, kBackwardQ, D, tq, GLOBAL ? global_lds(D) : 0)) ||
+        ((sides & kKeySide) && !choose_tile(p, kBackwardKV, D, tk)))
         return hipErrorInvalidValue;
-    hipError_t e = tq.rowshift > 5
-                       ? run_bwd_q<T, D, LAY, true, GLOBAL>(p, tq, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll,
-                                                            dlse, ldl, dq, ldq, delta, lde, g, s)
-                       : run_bwd_q<T, D, LAY, false, GLOBAL>(p, tq, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll,
-                                                             dlse, ldl, dq, ldq, delta, lde, g, s);
-    if (e != hipSuccess) return e;
+    if (sides & kQuerySide) {
+        const hipError_t e =
+            tq.rowshift > 5 ? run_bwd_q<T, D, LAY, true, GLOBAL>(p, tq, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll,
+                                                                 dlse, ldl, dq, ldq, delta, lde, g, s)
+                            : run_bwd_q<T, D, LAY, false, GLOBAL>(p, tq, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse,
+                                                                  ll, dlse, ldl, dq, ldq, delta, lde, g, s);
+        if (e != hipSuccess) return e;
+    }
+    if (!(sides & kKeySide)) return hipSuccess;
     if (tk.rowshift > 5)
         return run_bwd_kv<T, D, LAY, true>(p, tk, q, lq, k, lk, v, lv, dout, ldo, lse, ll, delta, lde, dk, ldk, dv,
                                            ldv, s);
@@ -1749,16 +1753,16 @@ template <typename T, int D>
 hipError_t launch_bwd(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                       const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll,
                       const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
-                      float* delta, Lay lde, const GlobalSet* gs, hipStream_t s) {
+                      float* delta, Lay lde, const GlobalSet* gs, int sides, hipStream_t s) {
     // global-key instances exist for the general layout group only
     if (gs)
         return launch_bwd<T, D, kLayGeneral, true>(p, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq,
-                                                   ldq, dk, ldk, dv, ldv, delta, lde, gs, s);
+                                                   ldq, dk, ldk, dv, ldv, delta, lde, gs, sides, s);
     // without dlse its layout is never read
     const int g = layout_group({lq, lo, ldo, ldq}, {lk, lv, ldk, ldv}, {ll, lde, dlse ? ldl : ll});
 #define NA_BWD_LAY(L)                                                                                                 \
     return launch_bwd<T, D, L, false>(p, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, \
-                                      dv, ldv, delta, lde, nullptr, s)
+                                      dv, ldv, delta, lde, nullptr, sides, s)
     switch (g) {
         case kLayOne:
             NA_BWD_LAY(kLayOne);
@@ -2188,7 +2192,7 @@ static Lay item_lay(const Prob& p, Lay l) {
     return l;
 }
 
-bool mfma_eligible(const Prob& p, int dtype, int D, bool aligned, bool backward, bool global) {
+bool mfma_eligible(const Prob& p, int dtype, int D, bool aligned, bool backward, bool global, int sides) {
     if (dtype == NATTEN_F32 || !aligned || !(p.scale > 0.f) || !mfma_static_lds_ok()) return false;
     if (p.Dqk != p.Dv || !(D == 32 || D == 64 || D == 96 || D == 128)) return false;
     // a strided axis must be one residue class (its query items then sit at
@@ -2200,8 +2204,10 @@ bool mfma_eligible(const Prob& p, int dtype, int D, bool aligned, bool backward,
     TileShape ts{};
     if (!choose_tile(p, kForward, D, ts, extra) || grid_blocks(p, ts) >= (1LL << 31)) return false;
     if (backward) {
-        if (!choose_tile(p, kBackwardQ, D, ts, extra) || grid_blocks(p, ts) >= (1LL << 31)) return false;
-        if (!choose_tile(p, kBackwardKV, D, ts) || grid_blocks(p, ts) >= (1LL << 31)) return false;
+        if ((sides & kQuerySide) && (!choose_tile(p, kBackwardQ, D, ts, extra) || grid_blocks(p, ts) >= (1LL << 31)))
+            return false;
+        if ((sides & kKeySide) && (!choose_tile(p, kBackwardKV, D, ts) || grid_blocks(p, ts) >= (1LL << 31)))
+            return false;
     }
     return true;
 }
@@ -2280,12 +2286,12 @@ hipError_t mfma_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay
 hipError_t mfma_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                          const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll,
                          const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
-                         float* delta, Lay lde, int dtype, hipStream_t s, const GlobalSet* g) {
+                         float* delta, Lay lde, int dtype, hipStream_t s, const GlobalSet* g, int sides) {
     lq = item_lay(p, lq);
     ldq = item_lay(p, ldq);
 #define NA_BWD(T, DD)                                                                                            \
     return launch_bwd<T, DD>(p, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv, \
-                             ldv, delta, lde, g, s)
+                             ldv, delta, lde, g, sides, s)
     if (dtype == NATTEN_BF16) {
         if (p.Dqk == 32) NA_BWD(bf16, 32);
         if (p.Dqk == 64) NA_BWD(bf16, 64);

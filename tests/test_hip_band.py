@@ -40,9 +40,33 @@ def _inputs(seed, shapes, dtype):
     return [torch.randn(s, generator=g, dtype=torch.float32).to(dtype) for s in shapes]
 
 
+# Windows whose query side stays on the 8 x 8 tiles: the key tiles at the
+# border, or of classes about twice the kernel, do not fit those.
+KEY_SIDE_CASES = [
+    ((40, 64), 2, 2, 64, (9, 9), (1, 1), (False, False), False),
+    ((17, 30), 4, 2, 64, (9, 9), (1, 1), (False, False), False),
+    ((40, 32), 2, 2, 32, (8, 8), (1, 1), (False, False), False),
+    ((22, 22), 2, 2, 32, (7, 7), (1, 1), (False, False), True),
+    ((48, 48), 2, 1, 32, (9, 9), (2, 2), (False, False), False),
+]
+# Head dim 128 takes both sides from 8 columns.
+WIDE_CASES = [((21, 37), 2, 1, 128, (9, 9), (1, 1), (True, False), False),
+              ((19, 40), 1, 1, 128, (5, 8), (1, 2), (False, False), True)]
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("case", CASES + WIDE_CASES)
 def test_band_kernels_match_oracle(case, dtype):
+    _check(case, dtype, {"na_fwd_band", "na_bwd_q_band", "na_bwd_kv_band"})
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", KEY_SIDE_CASES)
+def test_band_key_side_matches_oracle(case, dtype):
+    assert not any("q_band" in n for n in _check(case, dtype, {"na_bwd_kv_band"}))
+
+
+def _check(case, dtype, names):
     """Output, log-sum-exp and the gradients through both."""
     from natten_mps_amd import functional as F
     from natten_mps_amd._core import _lib
@@ -64,7 +88,7 @@ def test_band_kernels_match_oracle(case, dtype):
     finally:
         _lib.profile_enable(False)
     launched = set(_lib.profile_read(reset=True))
-    assert {"na_fwd_band", "na_bwd_q_band", "na_bwd_kv_band"} <= launched, launched
+    assert names <= launched, launched
 
     rq, rk, rv = (t.float().requires_grad_(True) for t in (q, k, v))
     n = hq // hkv
@@ -75,6 +99,31 @@ def test_band_kernels_match_oracle(case, dtype):
     rgrads = torch.autograd.grad((ref, ref_lse), (rq, rk, rv), (do.float(), dl.float()))
     for name, a, b in zip(("out", "lse", "dq", "dk", "dv"), (out, lse, *grads), (ref, ref_lse, *rgrads)):
         assert_parity(a.detach().cpu(), b.detach(), dtype, name)
+    return launched
+
+
+@pytest.mark.parametrize("tokens", [1, 7])
+@pytest.mark.parametrize("ks", [(9, 9), (7, 7)])  # key side on the band and on the lean tiles
+def test_window_key_side_under_global_keys(ks, tokens):
+    """dK / dV of the window with global keys beside it."""
+    from natten_mps_amd import functional as F
+
+    shapes = [(2, 33, 40, 2, 64)] * 3 + [(2, tokens, 2, 64)] * 2 + [(2, 33, 40, 2, 64)]
+    *ts, do = _inputs(34, shapes, torch.bfloat16)
+    leaves = [t.to(DEV).requires_grad_(True) for t in ts]
+    out = F.na2d(*leaves[:3], kernel_size=ks, additional_keys=leaves[3], additional_values=leaves[4])
+    grads = torch.autograd.grad(out, leaves, do.to(DEV))
+    q, k, v, gk, gv = (t.float().requires_grad_(True) for t in ts)
+    one = (1, 1)
+    logits = P.na2d_qk_forward(q, k, ks, one, one, (False, False), 64 ** -0.5)
+    extra = torch.einsum("bxyhd,bthd->bxyht", q, gk) * 64 ** -0.5
+    w = torch.softmax(torch.cat([logits, extra], dim=-1), dim=-1)
+    n = logits.shape[-1]
+    ref = P.na2d_av_forward(w[..., :n], v, ks, one, one, (False, False)) + torch.einsum(
+        "bxyht,bthd->bxyhd", w[..., n:], gv)
+    rgrads = torch.autograd.grad(ref, (q, k, v, gk, gv), do.float())
+    for name, a, b in zip(("out", "dq", "dk", "dv", "dgk", "dgv"), (out, *grads), (ref, *rgrads)):
+        assert_parity(a.detach().cpu(), b.detach(), torch.bfloat16, name)
 
 
 def test_band_kernels_recompute_non_finite_operands():
