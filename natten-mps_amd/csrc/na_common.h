@@ -420,60 +420,6 @@ template <> __device__ __forceinline__ bf16 from_f<bf16>(float f) {
     return r;
 }
 
-// N consecutive elements starting at p[d0], converted to float.  `vec` means
-// p + d0 is aligned to N*sizeof(T) bytes and D % N == 0 (so d0 < D implies the
-// whole run is in range).  Otherwise a guarded scalar path.
-template <typename T, int N>
-__device__ __forceinline__ void load_run(const T* __restrict__ p, int d0, int D, bool vec, float (&out)[N]) {
-    if (vec) {
-        if (d0 < D) {
-            constexpr int NW = (N * (int)sizeof(T)) / 16;
-            static_assert(NW >= 1, "run must cover at least 16 bytes");
-            uint4 raw[NW];
-            const uint4* src = reinterpret_cast<const uint4*>(p + d0);
-#pragma unroll
-            for (int w = 0; w < NW; ++w) raw[w] = src[w];
-            const T* e = reinterpret_cast<const T*>(raw);
-#pragma unroll
-            for (int j = 0; j < N; ++j) out[j] = to_f(e[j]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < N; ++j) out[j] = 0.f;
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < N; ++j) out[j] = (d0 + j < D) ? to_f(p[d0 + j]) : 0.f;
-    }
-}
-
-template <typename T, int N>
-__device__ __forceinline__ void store_run(T* __restrict__ p, int d0, int D, bool vec, const float (&in)[N]) {
-    if (vec) {
-        if (d0 < D) {
-            constexpr int NW = (N * (int)sizeof(T)) / 16;
-            T e[N];
-#pragma unroll
-            for (int j = 0; j < N; ++j) e[j] = from_f<T>(in[j]);
-            const uint4* src = reinterpret_cast<const uint4*>(e);
-            uint4* dst = reinterpret_cast<uint4*>(p + d0);
-#pragma unroll
-            for (int w = 0; w < NW; ++w) dst[w] = src[w];
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < N; ++j)
-            if (d0 + j < D) p[d0 + j] = from_f<T>(in[j]);
-    }
-}
-
-// Sum over the LPQ consecutive lanes that share one query.
-template <int LPQ>
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-    for (int m = LPQ / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, LPQ);
-    return v;
-}
-
 // Sum / max over the `split` lane groups (LPQ lanes each, consecutive) of
 // one query or key, in a fixed butterfly order.
 template <int LPQ>

@@ -1,6 +1,7 @@
 // Generic neighbourhood-attention kernels: every rank (as three padded axes),
 // dtype (fp32 / fp16 / bf16), kernel size, dilation, stride, causal mask and
-// GQA ratio.  Vector-ALU (FMA) kernels with fp32 accumulation.
+// GQA ratio.  Vector-ALU (FMA) kernels with fp32 accumulation (split gathers
+// of fp32 operands: fp64).
 //
 // Work mapping: a "group" of LPQ consecutive lanes owns one query (or one key,
 // for the key-centric gradient kernels); each lane owns DPL consecutive head
@@ -10,7 +11,18 @@
 // read straight from global memory; the overlap between neighbouring windows
 // is served by L1/L2 (blocks are remapped so each XCD walks a contiguous
 // range).
+//
+// Bound by instruction issue and the L1 (each neighbour's row is read once per
+// query).  What took the time beside the products, and was taken out: 64-bit
+// position products and divisions in every step, sums through the LDS
+// crossbar, one store per logit, selects on every element for lanes past the
+// head dim, and on the key side loads waited for one by one.  us, before ->
+// after: fp32 fused 2 x 64 x 64 x 4, dim 64, 11 x 11, dilation 2: 115 / 108 /
+// 260 -> 80 / 85 / 152 (forward / dQ / dK dV); bfloat16 2 x 12 x 20 x 24 x 4,
+// dim 48, 3 x 5 x 5: 130 / 239 / 262 -> 77 / 156 / 145; fp32 split ops 4 x 45
+// x 61 x 4, dim 32, 7 x 7: query side 25 each, key side 66 -> 22-25 and 33.
 #include <cstdlib>
+#include <type_traits>
 
 #include "na_launch.h"
 
@@ -78,13 +90,101 @@ __device__ __forceinline__ bool sample_extent(Prob& p, const int* __restrict__ l
     return true;
 }
 
-template <typename T, int DPL>
-__device__ __forceinline__ void store_zero(T* g, int d0, int D, int vec) {
-    float z[DPL];
-#pragma unroll
-    for (int j = 0; j < DPL; ++j) z[j] = 0.f;
-    store_run<T, DPL>(g, d0, D, vec, z);
+// Sum over the LPQ consecutive lanes of a group, on the vector ALU: pairs and
+// quads by quad permutes, then mirrored halves (each quad, then each half row
+// holds one value by then).  Shuffles through the LDS crossbar put two or
+// three LDS latencies into every step's chain.
+template <int LPQ>
+__device__ __forceinline__ float lane_sum(float v) {
+    const auto dpp = [&](auto ctrl) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value,
+                                                                     0xf, 0xf, true));
+    };
+    if constexpr (LPQ >= 2) v += dpp(std::integral_constant<int, 0xB1>{});    // quad_perm [1, 0, 3, 2]
+    if constexpr (LPQ >= 4) v += dpp(std::integral_constant<int, 0x4E>{});    // quad_perm [2, 3, 0, 1]
+    if constexpr (LPQ >= 8) v += dpp(std::integral_constant<int, 0x141>{});   // row_half_mirror
+    if constexpr (LPQ >= 16) v += dpp(std::integral_constant<int, 0x140>{});  // row_mirror
+    static_assert(LPQ <= 16);
+    return v;
 }
+
+// The DPL head dims of a group's lane, as registers.  On 16-byte aligned rows
+// (`vec`: D is a multiple of DPL) they are 16-byte pieces dealt to the lanes in
+// turn, so that every load of a group reads one contiguous run: with a lane's
+// dims side by side, the two loads of an fp32 row each spanned the whole row
+// and the L1 served them at half its rate.  Other rows: DPL dims side by side,
+// one element at a time.
+template <typename T, int DPL, int LPQ>
+struct Run {
+    static constexpr int EPP = 16 / static_cast<int>(sizeof(T)), NW = DPL / EPP;
+    static_assert(NW >= 1);
+    struct Raw {
+        uint4 w[NW];
+    };
+
+    static __device__ __forceinline__ int dim(int lane, int w) { return (w * LPQ + lane) * EPP; }
+
+    // Issues the loads.  Pieces past the head dim read the row start; their
+    // values meet only `dot`, which drops them, and registers never stored.
+    static __device__ __forceinline__ Raw fetch(const T* __restrict__ p, int lane, int D) {
+        Raw r;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const int d = dim(lane, w);
+            r.w[w] = *reinterpret_cast<const uint4*>(p + (d < D ? d : 0));
+        }
+        return r;
+    }
+    static __device__ __forceinline__ void unpack(const Raw& r, float (&out)[DPL]) {
+        const T* e = reinterpret_cast<const T*>(r.w);
+#pragma unroll
+        for (int j = 0; j < DPL; ++j) out[j] = to_f(e[j]);
+    }
+    static __device__ __forceinline__ void load(const T* __restrict__ p, int lane, int D, int vec, float (&out)[DPL]) {
+        if (vec) {
+            unpack(fetch(p, lane, D), out);
+        } else {
+#pragma unroll
+            for (int j = 0; j < DPL; ++j) out[j] = lane * DPL + j < D ? to_f(p[lane * DPL + j]) : 0.f;
+        }
+    }
+    static __device__ __forceinline__ void store(T* __restrict__ p, int lane, int D, int vec, const float (&in)[DPL]) {
+        if (vec) {
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const int d = dim(lane, w);
+                if (d >= D) continue;
+                T e[EPP];
+#pragma unroll
+                for (int j = 0; j < EPP; ++j) e[j] = from_f<T>(in[w * EPP + j]);
+                *reinterpret_cast<uint4*>(p + d) = *reinterpret_cast<const uint4*>(e);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < DPL; ++j)
+                if (lane * DPL + j < D) p[lane * DPL + j] = from_f<T>(in[j]);
+        }
+    }
+    // The lane's part of a . b over D dims.
+    static __device__ __forceinline__ float dot(const float (&a)[DPL], const float (&b)[DPL], int lane, int D,
+                                                int vec) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            float s = 0.f;
+#pragma unroll
+            for (int j = 0; j < EPP; ++j) s = fmaf(a[w * EPP + j], b[w * EPP + j], s);
+            sum += !vec || dim(lane, w) < D ? s : 0.f;
+        }
+        return sum;
+    }
+    static __device__ __forceinline__ void zero(T* g, int lane, int D, int vec) {
+        float z[DPL];
+#pragma unroll
+        for (int j = 0; j < DPL; ++j) z[j] = 0.f;
+        store(g, lane, D, vec, z);
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Pipelined walks.  A group's walk over its neighbours (or attending
@@ -92,43 +192,33 @@ __device__ __forceinline__ void store_zero(T* g, int d0, int D, int vec) {
 // the next U steps are already in flight.  `fetch` issues a step's loads and
 // returns the raw registers (no use of the loaded values, so no wait), `use`
 // consumes them, in the same order as the plain walk.  Only for 16-byte
-// aligned runs (`vec`): lanes past the head dim read the row start and drop
-// it when unpacking; masked (causal) neighbours load from a clamped position
+// aligned runs (`vec`); masked (causal) neighbours load from a clamped position
 // and are skipped by `use`.  fetch(j0, j1, j2, e) gets the neighbour's
-// position and index, use(step, e, valid) its registers.
+// position and index, use(step, e, valid, u) its registers (u: step within
+// its block of U).
 // ---------------------------------------------------------------------------
-template <typename T, int N>
-struct Raw {
-    static constexpr int NW = (N * static_cast<int>(sizeof(T))) / 16;
-    uint4 w[NW];
-};
-
-template <typename T, int N>
-__device__ __forceinline__ Raw<T, N> fetch_run(const T* __restrict__ p, int d0, int D) {
-    Raw<T, N> r;
-    const uint4* src = reinterpret_cast<const uint4*>(p + (d0 < D ? d0 : 0));
-#pragma unroll
-    for (int w = 0; w < Raw<T, N>::NW; ++w) r.w[w] = src[w];
-    return r;
-}
-
-template <typename T, int N>
-__device__ __forceinline__ void unpack_run(const Raw<T, N>& r, int d0, int D, float (&out)[N]) {
-    const T* e = reinterpret_cast<const T*>(r.w);
-#pragma unroll
-    for (int j = 0; j < N; ++j) out[j] = d0 < D ? to_f(e[j]) : 0.f;
-}
-
 // Steps in flight: about 8 runs of 16 bytes per lane.
 template <typename T, int DPL, int RUNS>
 constexpr int pipe_depth() {
-    constexpr int w = Raw<T, DPL>::NW * RUNS;
+    constexpr int w = DPL * static_cast<int>(sizeof(T)) / 16 * RUNS;
     return w >= 4 ? 2 : 8 / w;
 }
 
-template <int U, class Fetch, class Use>
-__device__ __forceinline__ void walk_neighbors_pipelined(const Prob& p, int i0, int i1, int i2, int sp, int split,
-                                                         Fetch&& fetch, Use&& use) {
+// Keeps what follows in a branch of its own: turned into selects, a new row's
+// products or a step's products would be paid on every step.
+__device__ __forceinline__ void keep_branch() { asm volatile(""); }
+
+// Offsets of one step in NT operands.  The walks below carry them from step
+// to step by additions: computed from the position, each was three 64-bit
+// products, which run at a quarter of the rate and took most of the time.
+template <int NT>
+struct Offsets {
+    long long o[NT];
+};
+
+template <int U, int NT, class Fetch, class Use>
+__device__ __forceinline__ void walk_neighbors_pipelined(const Prob& p, int b, int h, int i0, int i1, int i2, int sp,
+                                                         int split, const Lay (&l)[NT], Fetch&& fetch, Use&& use) {
     const Axis &A0 = p.ax[0], &A1 = p.ax[1], &A2 = p.ax[2];
     const int f0 = axis_first(A0, i0), f1 = axis_first(A1, i1), f2 = axis_first(A2, i2);
     const int sa = split_axis(p);
@@ -139,8 +229,23 @@ __device__ __forceinline__ void walk_neighbors_pipelined(const Prob& p, int i0, 
     const int ny = y0 < A1.k ? (A1.k - y0 + ys - 1) / ys : 0;
     const int nz = z0 < A2.k ? (A2.k - z0 + zs - 1) / zs : 0;
     const int total = nx * ny * nz;
-    using P = decltype(fetch(0, 0, 0, 0));
-    int x = x0, y = y0, z = z0;
+    using P = decltype(fetch(Offsets<NT>{}, 0));
+    int x = x0, y = y0, z = z0, e = 0;
+    bool ok = false;
+    Offsets<NT> row, col, dcol;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) dcol.o[t] = static_cast<long long>(zs) * A2.dil * l[t].s2;
+    const auto start_row = [&] {
+        const int j0 = f0 + x * A0.dil, j1 = f1 + y * A1.dil;
+        ok = (j0 >= 0) & (j1 >= 0);
+        e = (x * A1.k + y) * A2.k;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            row.o[t] = l[t].at(b, j0 < 0 ? 0 : j0, j1 < 0 ? 0 : j1, 0, h);
+            col.o[t] = static_cast<long long>(f2 + z0 * A2.dil) * l[t].s2;
+        }
+    };
+    start_row();
     // blocks of U steps: every fetch of a block is issued before the first
     // use, unconditionally (past the end the cursor stays on the last step),
     // so the compiler waits for each step's loads with the rest in flight
@@ -150,24 +255,108 @@ __device__ __forceinline__ void walk_neighbors_pipelined(const Prob& p, int i0, 
         bool okb[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int j0 = f0 + x * A0.dil, j1 = f1 + y * A1.dil, j2 = f2 + z * A2.dil;
-            okb[u] = (j0 >= 0) & (j1 >= 0) & (j2 >= 0);
-            eb[u] = (x * A1.k + y) * A2.k + z;
-            buf[u] = fetch(j0 < 0 ? 0 : j0, j1 < 0 ? 0 : j1, j2 < 0 ? 0 : j2, eb[u]);
+            const int j2 = f2 + z * A2.dil;
+            okb[u] = ok & (j2 >= 0);
+            eb[u] = e + z;
+            Offsets<NT> at;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) at.o[t] = row.o[t] + (j2 < 0 ? 0 : col.o[t]);
+            buf[u] = fetch(at, eb[u]);
             if (i + u + 1 < total) {
-                if ((z += zs) >= A2.k) {
+                z += zs;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) col.o[t] += dcol.o[t];
+                if (z >= A2.k) {
+                    keep_branch();
                     z = z0;
                     if ((y += ys) >= A1.k) {
                         y = y0;
                         x += xs;
                     }
+                    start_row();
                 }
             }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (i + u < total) use(buf[u], eb[u], okb[u]);
+            if (i + u < total) use(buf[u], eb[u], okb[u], u);
     }
+}
+
+// The attending queries of key (m0, m1, m2), in for_each_query_split's order:
+// fetch(offsets, e) and use(step, e).  Strides of 1 only: positions and
+// windows come from the key's residue class.
+template <int U, int NT, class Fetch, class Use>
+__device__ __forceinline__ void walk_queries_pipelined(const Prob& p, int b, int h, int m0, int m1, int m2, int sp,
+                                                       int split, const Lay (&l)[NT], Fetch&& fetch, Use&& use) {
+    int lo[3], hi[3], key[3];
+    const int m[3] = {m0, m1, m2};
+    ClassAxis c[3];
+    bool any = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const Axis& A = p.ax[a];
+        key[a] = m[a] / A.dil;
+        c[a] = class_axis(A, m[a] - key[a] * A.dil);
+        class_span(c[a], key[a], lo[a], hi[a]);
+        while (hi[a] >= lo[a] && m[a] + (hi[a] - key[a]) * A.dil >= A.out) --hi[a];
+        any = any && lo[a] <= hi[a];
+    }
+    if (!any) return;
+    const Axis &A0 = p.ax[0], &A1 = p.ax[1], &A2 = p.ax[2];
+    const int sa = split_axis(p);
+    const int s0 = sa == 0 ? split : 1, s1 = sa == 1 ? split : 1, s2 = sa == 2 ? split : 1;
+    const int b0 = lo[0] + (sa == 0 ? sp : 0), b1 = lo[1] + (sa == 1 ? sp : 0), b2 = lo[2] + (sa == 2 ? sp : 0);
+    const int n0 = hi[0] >= b0 ? (hi[0] - b0) / s0 + 1 : 0, n1 = hi[1] >= b1 ? (hi[1] - b1) / s1 + 1 : 0;
+    const int n2 = hi[2] >= b2 ? (hi[2] - b2) / s2 + 1 : 0;
+    const int total = n0 * n1 * n2;
+    if (total == 0) return;
+    using P = decltype(fetch(Offsets<NT>{}, 0));
+    int j0 = b0, j1 = b1, j2 = b2, e = 0;
+    Offsets<NT> at, dcol;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) dcol.o[t] = static_cast<long long>(s2) * A2.dil * l[t].s2;
+    const auto start_row = [&] {
+        e = ((key[0] - class_ws(c[0], j0)) * A1.k + key[1] - class_ws(c[1], j1)) * A2.k + key[2];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            at.o[t] = l[t].at(b, m0 + (j0 - key[0]) * A0.dil, m1 + (j1 - key[1]) * A1.dil,
+                              m2 + (b2 - key[2]) * A2.dil, h);
+    };
+    start_row();
+    for (int i = 0; i < total; i += U) {
+        P buf[U];
+        int eb[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            eb[u] = e - class_ws(c[2], j2);
+            buf[u] = fetch(at, eb[u]);
+            if (i + u + 1 < total) {
+                j2 += s2;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) at.o[t] += dcol.o[t];
+                if (j2 > hi[2]) {
+                    keep_branch();
+                    j2 = b2;
+                    if ((j1 += s1) > hi[1]) {
+                        j1 = b1;
+                        j0 += s0;
+                    }
+                    start_row();
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (i + u < total) {
+                keep_branch();
+                use(buf[u], eb[u]);
+            }
+    }
+}
+
+__device__ __forceinline__ bool unit_strides(const Prob& p) {
+    return p.ax[0].st == 1 && p.ax[1].st == 1 && p.ax[2].st == 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -182,27 +371,25 @@ __global__ __launch_bounds__(256) void k_forward(Prob p, int vec, int split, con
                                                  float* __restrict__ lse, Lay ll) {
     const long long qi = group_index(LPQ * split);
     if (qi >= static_cast<long long>(p.B) * p.nout * p.Hq) return;
-    const int d0 = (threadIdx.x % LPQ) * DPL;
+    using R = Run<T, DPL, LPQ>;
+    const int ln = threadIdx.x % LPQ;
     const int sp = (threadIdx.x / LPQ) % split;
     const QPos Q = decode_query(p, qi);
     const int hk = Q.h / p.rep;
     if (lens && !sample_extent(p, lens, Q.b, Q.i0, Q.i1, Q.i2)) {
-        if (sp == 0) store_zero<T, DPL>(out + lo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), d0, p.Dv, vec);
-        if (sp == 0 && d0 == 0) lse[ll.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)] = 0.f;
+        if (sp == 0) R::zero(out + lo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), ln, p.Dv, vec);
+        if (sp == 0 && ln == 0) lse[ll.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)] = 0.f;
         return;
     }
 
     float qv[DPL];
-    load_run<T, DPL>(q + lq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), d0, p.Dqk, vec, qv);
+    R::load(q + lq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), ln, p.Dqk, vec, qv);
     float m = -INFINITY, l = 0.f, acc[DPL];
 #pragma unroll
     for (int j = 0; j < DPL; ++j) acc[j] = 0.f;
 
     const auto step = [&](const float (&kv)[DPL], const float (&vv)[DPL]) {
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < DPL; ++j) s = fmaf(qv[j], kv[j], s);
-        s = group_sum<LPQ>(s) * p.scale;
+        const float s = lane_sum<LPQ>(R::dot(qv, kv, ln, p.Dqk, vec)) * p.scale;
         if (s > m) {
             const float c = expf(m - s);
             l *= c;
@@ -217,27 +404,27 @@ __global__ __launch_bounds__(256) void k_forward(Prob p, int vec, int split, con
     };
     if (vec) {
         struct Step {
-            Raw<T, DPL> k, v;
+            typename R::Raw k, v;
         };
-        walk_neighbors_pipelined<pipe_depth<T, DPL, 2>()>(
-            p, Q.i0, Q.i1, Q.i2, sp, split,
-            [&](int j0, int j1, int j2, int) {
-                return Step{fetch_run<T, DPL>(k + lk.at(Q.b, j0, j1, j2, hk), d0, p.Dqk),
-                            fetch_run<T, DPL>(v + lv.at(Q.b, j0, j1, j2, hk), d0, p.Dv)};
+        walk_neighbors_pipelined<pipe_depth<T, DPL, 2>(), 2>(
+            p, Q.b, hk, Q.i0, Q.i1, Q.i2, sp, split, {lk, lv},
+            [&](const Offsets<2>& at, int) {
+                return Step{R::fetch(k + at.o[0], ln, p.Dqk), R::fetch(v + at.o[1], ln, p.Dv)};
             },
-            [&](const Step& st, int, bool ok) {
+            [&](const Step& st, int, bool ok, int) {
                 if (!ok) return;
+                keep_branch();
                 float kv[DPL], vv[DPL];
-                unpack_run<T, DPL>(st.k, d0, p.Dqk, kv);
-                unpack_run<T, DPL>(st.v, d0, p.Dv, vv);
+                R::unpack(st.k, kv);
+                R::unpack(st.v, vv);
                 step(kv, vv);
             });
     } else {
         for_each_neighbor_split(p, Q.i0, Q.i1, Q.i2, sp, split, [&](int j0, int j1, int j2, int, bool ok) {
             if (!ok) return;
             float kv[DPL], vv[DPL];
-            load_run<T, DPL>(k + lk.at(Q.b, j0, j1, j2, hk), d0, p.Dqk, vec, kv);
-            load_run<T, DPL>(v + lv.at(Q.b, j0, j1, j2, hk), d0, p.Dv, vec, vv);
+            R::load(k + lk.at(Q.b, j0, j1, j2, hk), ln, p.Dqk, vec, kv);
+            R::load(v + lv.at(Q.b, j0, j1, j2, hk), ln, p.Dv, vec, vv);
             step(kv, vv);
         });
     }
@@ -253,53 +440,73 @@ __global__ __launch_bounds__(256) void k_forward(Prob p, int vec, int split, con
     }
 #pragma unroll
     for (int j = 0; j < DPL; ++j) acc[j] = acc[j] / l;
-    if (sp == 0) store_run<T, DPL>(out + lo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), d0, p.Dv, vec, acc);
-    if (sp == 0 && d0 == 0) lse[ll.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)] = m + logf(l);
+    if (sp == 0) R::store(out + lo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), ln, p.Dv, vec, acc);
+    if (sp == 0 && ln == 0) lse[ll.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)] = m + logf(l);
 }
+
+// Row elements of a query, one per step, collected so that the group's lanes
+// store up to LPQ of them at once (of one block of U steps).
+template <typename T, int LPQ, int U>
+struct RowPut {
+    T* row;
+    int at = -1;
+    T val{};
+    __device__ __forceinline__ void add(int lane, int u, int e, T v) {
+        if (u % LPQ == lane) {
+            at = e;
+            val = v;
+        }
+        if (u % LPQ == LPQ - 1 || u == U - 1) flush();
+    }
+    __device__ __forceinline__ void flush() {
+        if (at >= 0) row[at] = val;
+        at = -1;
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Split QK: logits per neighbour (unscaled unless has_scale), -inf if invalid.
 // ---------------------------------------------------------------------------
 template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_qk(Prob p, int vec,
+__global__ __launch_bounds__(256) void k_qk(Prob p, int vec, int split,
                                             const T* __restrict__ q, Lay lq,
                                             const T* __restrict__ k, Lay lk,
                                             T* __restrict__ attn, Lay la) {
-    const long long qi = group_index(LPQ);
+    const long long qi = group_index(LPQ * split);
     if (qi >= static_cast<long long>(p.B) * p.nout * p.Hq) return;
-    const int d0 = (threadIdx.x % LPQ) * DPL;
+    using R = Run<T, DPL, LPQ>;
+    const int ln = threadIdx.x % LPQ;
+    const int sp = (threadIdx.x / LPQ) % split;
     const QPos Q = decode_query(p, qi);
     float qv[DPL];
-    load_run<T, DPL>(q + lq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), d0, p.Dqk, vec, qv);
+    R::load(q + lq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), ln, p.Dqk, vec, qv);
     T* row = attn + la.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h);
     if (vec) {
-        walk_neighbors_pipelined<pipe_depth<T, DPL, 1>()>(
-            p, Q.i0, Q.i1, Q.i2, 0, 1,
-            [&](int j0, int j1, int j2, int) { return fetch_run<T, DPL>(k + lk.at(Q.b, j0, j1, j2, Q.h), d0, p.Dqk); },
-            [&](const Raw<T, DPL>& r, int e, bool ok) {
+        RowPut<T, LPQ, pipe_depth<T, DPL, 1>()> put{row};
+        walk_neighbors_pipelined<pipe_depth<T, DPL, 1>(), 1>(
+            p, Q.b, Q.h, Q.i0, Q.i1, Q.i2, sp, split, {lk},
+            [&](const Offsets<1>& at, int) { return R::fetch(k + at.o[0], ln, p.Dqk); },
+            [&](const typename R::Raw& r, int e, bool ok, int u) {
                 float kv[DPL];
-                unpack_run<T, DPL>(r, d0, p.Dqk, kv);
-                float acc = 0.f;
-#pragma unroll
-                for (int j = 0; j < DPL; ++j) acc = fmaf(qv[j], kv[j], acc);
-                float s = ok ? group_sum<LPQ>(acc) : -INFINITY;
+                R::unpack(r, kv);
+                const float acc = R::dot(qv, kv, ln, p.Dqk, vec);
+                float s = ok ? lane_sum<LPQ>(acc) : -INFINITY;
                 if (p.has_scale) s *= p.scale;
-                if (d0 == 0) row[e] = from_f<T>(s);
+                put.add(ln, u, e, from_f<T>(s));
             });
+        put.flush();
         return;
     }
-    for_each_neighbor(p, Q.i0, Q.i1, Q.i2, [&](int j0, int j1, int j2, int e, bool ok) {
+    for_each_neighbor_split(p, Q.i0, Q.i1, Q.i2, sp, split, [&](int j0, int j1, int j2, int e, bool ok) {
         float s = -INFINITY;
         if (ok) {
             float kv[DPL];
-            load_run<T, DPL>(k + lk.at(Q.b, j0, j1, j2, Q.h), d0, p.Dqk, vec, kv);
-            float acc = 0.f;
-#pragma unroll
-            for (int j = 0; j < DPL; ++j) acc = fmaf(qv[j], kv[j], acc);
-            s = group_sum<LPQ>(acc);
+            R::load(k + lk.at(Q.b, j0, j1, j2, Q.h), ln, p.Dqk, vec, kv);
+            const float acc = R::dot(qv, kv, ln, p.Dqk, vec);
+            s = lane_sum<LPQ>(acc);
         }
         if (p.has_scale) s *= p.scale;
-        if (d0 == 0) row[e] = from_f<T>(s);
+        if (ln == 0) row[e] = from_f<T>(s);
     });
 }
 
@@ -323,24 +530,30 @@ __device__ __forceinline__ A gather_fma(float a, float b, A acc) {
     return static_cast<A>(a) * static_cast<A>(b) + acc;
 }
 
-// acc (times mul) rounded to float for store_run.
-template <typename A, int DPL>
-__device__ __forceinline__ void gather_out(const A (&acc)[DPL], float mul, float (&out)[DPL]) {
+// The groups' sum of acc (times mul) rounded to float for store_run.
+template <int LPQ, typename A, int DPL>
+__device__ __forceinline__ void gather_out(const A (&acc)[DPL], int split, float mul, float (&out)[DPL]) {
 #pragma unroll
-    for (int j = 0; j < DPL; ++j) out[j] = static_cast<float>(acc[j] * static_cast<A>(mul));
+    for (int j = 0; j < DPL; ++j) {
+        A v = acc[j];
+        for (int m = split >> 1; m >= 1; m >>= 1) v += __shfl_xor(v, m * LPQ);
+        out[j] = static_cast<float>(v * static_cast<A>(mul));
+    }
 }
 
 // ---------------------------------------------------------------------------
 // Split AV: out = sum_valid attn * v.
 // ---------------------------------------------------------------------------
 template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_av(Prob p, int vec,
+__global__ __launch_bounds__(256) void k_av(Prob p, int vec, int split,
                                             const T* __restrict__ attn, Lay la,
                                             const T* __restrict__ v, Lay lv,
                                             T* __restrict__ out, Lay lo) {
-    const long long qi = group_index(LPQ);
+    const long long qi = group_index(LPQ * split);
     if (qi >= static_cast<long long>(p.B) * p.nout * p.Hq) return;
-    const int d0 = (threadIdx.x % LPQ) * DPL;
+    using R = Run<T, DPL, LPQ>;
+    const int ln = threadIdx.x % LPQ;
+    const int sp = (threadIdx.x / LPQ) % split;
     const QPos Q = decode_query(p, qi);
     const T* row = attn + la.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h);
     using A = typename GatherAcc<T>::type;
@@ -349,35 +562,36 @@ __global__ __launch_bounds__(256) void k_av(Prob p, int vec,
     for (int j = 0; j < DPL; ++j) acc[j] = 0;
     if (vec) {
         struct Step {
-            Raw<T, DPL> v;
+            typename R::Raw v;
             T a;
         };
-        walk_neighbors_pipelined<pipe_depth<T, DPL, 1>()>(
-            p, Q.i0, Q.i1, Q.i2, 0, 1,
-            [&](int j0, int j1, int j2, int e) {
-                return Step{fetch_run<T, DPL>(v + lv.at(Q.b, j0, j1, j2, Q.h), d0, p.Dv), row[e]};
+        walk_neighbors_pipelined<pipe_depth<T, DPL, 1>(), 1>(
+            p, Q.b, Q.h, Q.i0, Q.i1, Q.i2, sp, split, {lv},
+            [&](const Offsets<1>& at, int e) {
+                return Step{R::fetch(v + at.o[0], ln, p.Dv), row[e]};
             },
-            [&](Step& st, int, bool ok) {
+            [&](const Step& st, int, bool ok, int) {
                 if (!ok) return;
+                keep_branch();
                 const float a = to_f(st.a);
                 float vv[DPL];
-                unpack_run<T, DPL>(st.v, d0, p.Dv, vv);
+                R::unpack(st.v, vv);
 #pragma unroll
                 for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(a, vv[j], acc[j]);
             });
     } else {
-        for_each_neighbor(p, Q.i0, Q.i1, Q.i2, [&](int j0, int j1, int j2, int e, bool ok) {
+        for_each_neighbor_split(p, Q.i0, Q.i1, Q.i2, sp, split, [&](int j0, int j1, int j2, int e, bool ok) {
             if (!ok) return;
             const float a = to_f(row[e]);
             float vv[DPL];
-            load_run<T, DPL>(v + lv.at(Q.b, j0, j1, j2, Q.h), d0, p.Dv, vec, vv);
+            R::load(v + lv.at(Q.b, j0, j1, j2, Q.h), ln, p.Dv, vec, vv);
 #pragma unroll
             for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(a, vv[j], acc[j]);
         });
     }
     float res[DPL];
-    gather_out(acc, 1.f, res);
-    store_run<T, DPL>(out + lo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), d0, p.Dv, vec, res);
+    gather_out<LPQ>(acc, split, 1.f, res);
+    if (sp == 0) R::store(out + lo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), ln, p.Dv, vec, res);
 }
 
 // ---------------------------------------------------------------------------
@@ -397,90 +611,83 @@ __global__ __launch_bounds__(256) void k_bwd_dq(Prob p, int vec, int split, cons
                                                 float* __restrict__ delta, Lay lde) {
     const long long qi = group_index(LPQ * split);
     if (qi >= static_cast<long long>(p.B) * p.nout * p.Hq) return;
-    const int d0 = (threadIdx.x % LPQ) * DPL;
+    using R = Run<T, DPL, LPQ>;
+    const int ln = threadIdx.x % LPQ;
     const int sp = (threadIdx.x / LPQ) % split;
     const QPos Q = decode_query(p, qi);
     const int hk = Q.h / p.rep;
     if (lens && !sample_extent(p, lens, Q.b, Q.i0, Q.i1, Q.i2)) {
-        if (sp == 0) store_zero<T, DPL>(dq + ldq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), d0, p.Dqk, vec);
-        if (sp == 0 && d0 == 0) delta[lde.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)] = 0.f;
+        if (sp == 0) R::zero(dq + ldq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), ln, p.Dqk, vec);
+        if (sp == 0 && ln == 0) delta[lde.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)] = 0.f;
         return;
     }
 
     float qv[DPL], dov[DPL];
-    load_run<T, DPL>(q + lq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), d0, p.Dqk, vec, qv);
-    load_run<T, DPL>(dout + ldo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), d0, p.Dv, vec, dov);
+    R::load(q + lq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), ln, p.Dqk, vec, qv);
+    R::load(dout + ldo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), ln, p.Dv, vec, dov);
     const float L = lse[ll.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)];
+    // use(key, value) for each valid neighbour
+    const auto walk = [&](auto&& use) {
+        if (vec) {
+            struct Step {
+                typename R::Raw k, v;
+            };
+            walk_neighbors_pipelined<pipe_depth<T, DPL, 2>(), 2>(
+                p, Q.b, hk, Q.i0, Q.i1, Q.i2, sp, split, {lk, lv},
+                [&](const Offsets<2>& at, int) {
+                    return Step{R::fetch(k + at.o[0], ln, p.Dqk), R::fetch(v + at.o[1], ln, p.Dv)};
+                },
+                [&](const Step& st, int, bool ok, int) {
+                    if (!ok) return;
+                    keep_branch();
+                    float kv[DPL], vv[DPL];
+                    R::unpack(st.k, kv);
+                    R::unpack(st.v, vv);
+                    use(kv, vv);
+                });
+        } else {
+            for_each_neighbor_split(p, Q.i0, Q.i1, Q.i2, sp, split, [&](int j0, int j1, int j2, int, bool ok) {
+                if (!ok) return;
+                float kv[DPL], vv[DPL];
+                R::load(k + lk.at(Q.b, j0, j1, j2, hk), ln, p.Dqk, vec, kv);
+                R::load(v + lv.at(Q.b, j0, j1, j2, hk), ln, p.Dv, vec, vv);
+                use(kv, vv);
+            });
+        }
+    };
     float di = 0.f;
     if constexpr (sizeof(T) == 4) {
         // delta = dO . O: exact enough when O was stored in fp32.
         float ov[DPL];
-        load_run<T, DPL>(o + lo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), d0, p.Dv, vec, ov);
-#pragma unroll
-        for (int j = 0; j < DPL; ++j) di = fmaf(dov[j], ov[j], di);
-        di = group_sum<LPQ>(di);
+        R::load(o + lo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), ln, p.Dv, vec, ov);
+        di = lane_sum<LPQ>(R::dot(dov, ov, ln, p.Dv, vec));
     } else {
         // 16-bit O carries ~2^-9 relative rounding; use the equivalent
         // delta = sum_k P_k (dO . v_k) from an extra pass instead.
-        for_each_neighbor_split(p, Q.i0, Q.i1, Q.i2, sp, split, [&](int j0, int j1, int j2, int, bool ok) {
-            if (!ok) return;
-            float kv[DPL], vv[DPL];
-            load_run<T, DPL>(k + lk.at(Q.b, j0, j1, j2, hk), d0, p.Dqk, vec, kv);
-            load_run<T, DPL>(v + lv.at(Q.b, j0, j1, j2, hk), d0, p.Dv, vec, vv);
-            float s = 0.f, dp = 0.f;
-#pragma unroll
-            for (int j = 0; j < DPL; ++j) { s = fmaf(qv[j], kv[j], s); dp = fmaf(dov[j], vv[j], dp); }
-            s = group_sum<LPQ>(s) * p.scale;
-            dp = group_sum<LPQ>(dp);
+        walk([&](const float (&kv)[DPL], const float (&vv)[DPL]) {
+            const float s = lane_sum<LPQ>(R::dot(qv, kv, ln, p.Dqk, vec)) * p.scale;
+            const float dp = lane_sum<LPQ>(R::dot(dov, vv, ln, p.Dv, vec));
             di = fmaf(expf(s - L), dp, di);
         });
         di = split_sum<LPQ>(di, split);
     }
     if (dlse) di -= dlse[ldl.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)];
-    if (sp == 0 && d0 == 0) delta[lde.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)] = di;
+    if (sp == 0 && ln == 0) delta[lde.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h)] = di;
 
     float acc[DPL];
 #pragma unroll
     for (int j = 0; j < DPL; ++j) acc[j] = 0.f;
     const auto step = [&](const float (&kv)[DPL], const float (&vv)[DPL]) {
-        float s = 0.f, dp = 0.f;
-#pragma unroll
-        for (int j = 0; j < DPL; ++j) { s = fmaf(qv[j], kv[j], s); dp = fmaf(dov[j], vv[j], dp); }
-        s = group_sum<LPQ>(s) * p.scale;
-        dp = group_sum<LPQ>(dp);
+        const float s = lane_sum<LPQ>(R::dot(qv, kv, ln, p.Dqk, vec)) * p.scale;
+        const float dp = lane_sum<LPQ>(R::dot(dov, vv, ln, p.Dv, vec));
         const float ds = expf(s - L) * (dp - di);
 #pragma unroll
         for (int j = 0; j < DPL; ++j) acc[j] = fmaf(ds, kv[j], acc[j]);
     };
-    if (vec) {
-        struct Step {
-            Raw<T, DPL> k, v;
-        };
-        walk_neighbors_pipelined<pipe_depth<T, DPL, 2>()>(
-            p, Q.i0, Q.i1, Q.i2, sp, split,
-            [&](int j0, int j1, int j2, int) {
-                return Step{fetch_run<T, DPL>(k + lk.at(Q.b, j0, j1, j2, hk), d0, p.Dqk),
-                            fetch_run<T, DPL>(v + lv.at(Q.b, j0, j1, j2, hk), d0, p.Dv)};
-            },
-            [&](const Step& st, int, bool ok) {
-                if (!ok) return;
-                float kv[DPL], vv[DPL];
-                unpack_run<T, DPL>(st.k, d0, p.Dqk, kv);
-                unpack_run<T, DPL>(st.v, d0, p.Dv, vv);
-                step(kv, vv);
-            });
-    } else {
-        for_each_neighbor_split(p, Q.i0, Q.i1, Q.i2, sp, split, [&](int j0, int j1, int j2, int, bool ok) {
-            if (!ok) return;
-            float kv[DPL], vv[DPL];
-            load_run<T, DPL>(k + lk.at(Q.b, j0, j1, j2, hk), d0, p.Dqk, vec, kv);
-            load_run<T, DPL>(v + lv.at(Q.b, j0, j1, j2, hk), d0, p.Dv, vec, vv);
-            step(kv, vv);
-        });
-    }
+    walk(step);
 #pragma unroll
     for (int j = 0; j < DPL; ++j) acc[j] = split_sum<LPQ>(acc[j], split) * p.scale;
-    if (sp == 0) store_run<T, DPL>(dq + ldq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), d0, p.Dqk, vec, acc);
+    if (sp == 0) R::store(dq + ldq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), ln, p.Dqk, vec, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -501,50 +708,70 @@ __global__ __launch_bounds__(256) void k_bwd_dkdv(Prob p, int vec, int split, co
                                                   T* __restrict__ dv, Lay ldv) {
     const long long ki = group_index(LPQ * split);
     if (ki >= static_cast<long long>(p.B) * p.nkey * p.Hkv) return;
-    const int d0 = (threadIdx.x % LPQ) * DPL;
+    using R = Run<T, DPL, LPQ>;
+    const int ln = threadIdx.x % LPQ;
     const int sp = (threadIdx.x / LPQ) % split;
     const KPos K = decode_key(p, ki, p.Hkv);
     if (lens && !sample_extent(p, lens, K.b, K.m0, K.m1, K.m2)) {
-        if (sp == 0) store_zero<T, DPL>(dk + ldk.at(K.b, K.m0, K.m1, K.m2, K.h), d0, p.Dqk, vec);
-        if (sp == 0) store_zero<T, DPL>(dv + ldv.at(K.b, K.m0, K.m1, K.m2, K.h), d0, p.Dv, vec);
+        if (sp == 0) R::zero(dk + ldk.at(K.b, K.m0, K.m1, K.m2, K.h), ln, p.Dqk, vec);
+        if (sp == 0) R::zero(dv + ldv.at(K.b, K.m0, K.m1, K.m2, K.h), ln, p.Dv, vec);
         return;
     }
 
     float kv[DPL], vv[DPL], gk[DPL], gv[DPL];
-    load_run<T, DPL>(k + lk.at(K.b, K.m0, K.m1, K.m2, K.h), d0, p.Dqk, vec, kv);
-    load_run<T, DPL>(v + lv.at(K.b, K.m0, K.m1, K.m2, K.h), d0, p.Dv, vec, vv);
+    R::load(k + lk.at(K.b, K.m0, K.m1, K.m2, K.h), ln, p.Dqk, vec, kv);
+    R::load(v + lv.at(K.b, K.m0, K.m1, K.m2, K.h), ln, p.Dv, vec, vv);
 #pragma unroll
     for (int j = 0; j < DPL; ++j) { gk[j] = 0.f; gv[j] = 0.f; }
 
-    for_each_query_split(p, K.m0, K.m1, K.m2, sp, split, [&](int o0, int o1, int o2, int i0, int i1, int i2, int) {
-        for (int r = 0; r < p.rep; ++r) {
-            const int h = K.h * p.rep + r;
-            float qv[DPL], dov[DPL];
-            load_run<T, DPL>(q + lq.at(K.b, i0, i1, i2, h), d0, p.Dqk, vec, qv);
-            load_run<T, DPL>(dout + ldo.at(K.b, o0, o1, o2, h), d0, p.Dv, vec, dov);
-            const float L = lse[ll.at(K.b, o0, o1, o2, h)];
-            const float di = delta[lde.at(K.b, o0, o1, o2, h)];
-            float s = 0.f, dp = 0.f;
+    const auto add = [&](const float (&qv)[DPL], const float (&dov)[DPL], float L, float di) {
+        const float s = lane_sum<LPQ>(R::dot(qv, kv, ln, p.Dqk, vec)) * p.scale;
+        const float dp = lane_sum<LPQ>(R::dot(dov, vv, ln, p.Dv, vec));
+        const float pr = expf(s - L);
+        const float ds = pr * (dp - di);
 #pragma unroll
-            for (int j = 0; j < DPL; ++j) { s = fmaf(qv[j], kv[j], s); dp = fmaf(dov[j], vv[j], dp); }
-            s = group_sum<LPQ>(s) * p.scale;
-            dp = group_sum<LPQ>(dp);
-            const float pr = expf(s - L);
-            const float ds = pr * (dp - di);
-#pragma unroll
-            for (int j = 0; j < DPL; ++j) {
-                gv[j] = fmaf(pr, dov[j], gv[j]);
-                gk[j] = fmaf(ds, qv[j], gk[j]);
-            }
+        for (int j = 0; j < DPL; ++j) {
+            gv[j] = fmaf(pr, dov[j], gv[j]);
+            gk[j] = fmaf(ds, qv[j], gk[j]);
         }
-    });
+    };
+    if (vec && unit_strides(p)) {
+        struct Step {
+            typename R::Raw q, g;
+            float L, di;
+        };
+        for (int r = 0; r < p.rep; ++r) {
+            walk_queries_pipelined<pipe_depth<T, DPL, 2>(), 4>(
+                p, K.b, K.h * p.rep + r, K.m0, K.m1, K.m2, sp, split, {lq, ldo, ll, lde},
+                [&](const Offsets<4>& at, int) {
+                    return Step{R::fetch(q + at.o[0], ln, p.Dqk), R::fetch(dout + at.o[1], ln, p.Dv),
+                                lse[at.o[2]], delta[at.o[3]]};
+                },
+                [&](const Step& st, int) {
+                    float qv[DPL], dov[DPL];
+                    R::unpack(st.q, qv);
+                    R::unpack(st.g, dov);
+                    add(qv, dov, st.L, st.di);
+                });
+        }
+    } else {
+        for_each_query_split(p, K.m0, K.m1, K.m2, sp, split, [&](int o0, int o1, int o2, int i0, int i1, int i2, int) {
+            for (int r = 0; r < p.rep; ++r) {
+                const int h = K.h * p.rep + r;
+                float qv[DPL], dov[DPL];
+                R::load(q + lq.at(K.b, i0, i1, i2, h), ln, p.Dqk, vec, qv);
+                R::load(dout + ldo.at(K.b, o0, o1, o2, h), ln, p.Dv, vec, dov);
+                add(qv, dov, lse[ll.at(K.b, o0, o1, o2, h)], delta[lde.at(K.b, o0, o1, o2, h)]);
+            }
+        });
+    }
 #pragma unroll
     for (int j = 0; j < DPL; ++j) {
         gk[j] = split_sum<LPQ>(gk[j], split) * p.scale;
         gv[j] = split_sum<LPQ>(gv[j], split);
     }
-    if (sp == 0) store_run<T, DPL>(dk + ldk.at(K.b, K.m0, K.m1, K.m2, K.h), d0, p.Dqk, vec, gk);
-    if (sp == 0) store_run<T, DPL>(dv + ldv.at(K.b, K.m0, K.m1, K.m2, K.h), d0, p.Dv, vec, gv);
+    if (sp == 0) R::store(dk + ldk.at(K.b, K.m0, K.m1, K.m2, K.h), ln, p.Dqk, vec, gk);
+    if (sp == 0) R::store(dv + ldv.at(K.b, K.m0, K.m1, K.m2, K.h), ln, p.Dv, vec, gv);
 }
 
 // ---------------------------------------------------------------------------
@@ -552,13 +779,15 @@ __global__ __launch_bounds__(256) void k_bwd_dkdv(Prob p, int vec, int split, co
 // entry is zero, and both carry the logit scale when has_scale.
 // ---------------------------------------------------------------------------
 template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_qk_bwd_q(Prob p, int vec,
+__global__ __launch_bounds__(256) void k_qk_bwd_q(Prob p, int vec, int split,
                                                   const T* __restrict__ da, Lay lda,
                                                   const T* __restrict__ k, Lay lk,
                                                   T* __restrict__ dq, Lay ldq) {
-    const long long qi = group_index(LPQ);
+    const long long qi = group_index(LPQ * split);
     if (qi >= static_cast<long long>(p.B) * p.nout * p.Hq) return;
-    const int d0 = (threadIdx.x % LPQ) * DPL;
+    using R = Run<T, DPL, LPQ>;
+    const int ln = threadIdx.x % LPQ;
+    const int sp = (threadIdx.x / LPQ) % split;
     const QPos Q = decode_query(p, qi);
     const T* row = da + lda.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h);
     using A = typename GatherAcc<T>::type;
@@ -567,129 +796,172 @@ __global__ __launch_bounds__(256) void k_qk_bwd_q(Prob p, int vec,
     for (int j = 0; j < DPL; ++j) acc[j] = 0;
     if (vec) {
         struct Step {
-            Raw<T, DPL> k;
+            typename R::Raw k;
             T g;
         };
-        walk_neighbors_pipelined<pipe_depth<T, DPL, 1>()>(
-            p, Q.i0, Q.i1, Q.i2, 0, 1,
-            [&](int j0, int j1, int j2, int e) {
-                return Step{fetch_run<T, DPL>(k + lk.at(Q.b, j0, j1, j2, Q.h), d0, p.Dqk), row[e]};
+        walk_neighbors_pipelined<pipe_depth<T, DPL, 1>(), 1>(
+            p, Q.b, Q.h, Q.i0, Q.i1, Q.i2, sp, split, {lk},
+            [&](const Offsets<1>& at, int e) {
+                return Step{R::fetch(k + at.o[0], ln, p.Dqk), row[e]};
             },
-            [&](Step& st, int, bool ok) {
+            [&](const Step& st, int, bool ok, int) {
                 if (!ok) return;
+                keep_branch();
                 const float g = to_f(st.g);
                 float kv[DPL];
-                unpack_run<T, DPL>(st.k, d0, p.Dqk, kv);
+                R::unpack(st.k, kv);
 #pragma unroll
                 for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(g, kv[j], acc[j]);
             });
     } else {
-        for_each_neighbor(p, Q.i0, Q.i1, Q.i2, [&](int j0, int j1, int j2, int e, bool ok) {
+        for_each_neighbor_split(p, Q.i0, Q.i1, Q.i2, sp, split, [&](int j0, int j1, int j2, int e, bool ok) {
             if (!ok) return;
             const float g = to_f(row[e]);
             float kv[DPL];
-            load_run<T, DPL>(k + lk.at(Q.b, j0, j1, j2, Q.h), d0, p.Dqk, vec, kv);
+            R::load(k + lk.at(Q.b, j0, j1, j2, Q.h), ln, p.Dqk, vec, kv);
 #pragma unroll
             for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(g, kv[j], acc[j]);
         });
     }
     float res[DPL];
-    gather_out(acc, p.has_scale ? p.scale : 1.f, res);
-    store_run<T, DPL>(dq + ldq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), d0, p.Dqk, vec, res);
+    gather_out<LPQ>(acc, split, p.has_scale ? p.scale : 1.f, res);
+    if (sp == 0) R::store(dq + ldq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), ln, p.Dqk, vec, res);
 }
 
 template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_qk_bwd_k(Prob p, int vec,
+__global__ __launch_bounds__(256) void k_qk_bwd_k(Prob p, int vec, int split,
                                                   const T* __restrict__ da, Lay lda,
                                                   const T* __restrict__ q, Lay lq,
                                                   T* __restrict__ dk, Lay ldk) {
-    const long long ki = group_index(LPQ);
+    const long long ki = group_index(LPQ * split);
     if (ki >= static_cast<long long>(p.B) * p.nkey * p.Hkv) return;
-    const int d0 = (threadIdx.x % LPQ) * DPL;
+    using R = Run<T, DPL, LPQ>;
+    const int ln = threadIdx.x % LPQ;
+    const int sp = (threadIdx.x / LPQ) % split;
     const KPos K = decode_key(p, ki, p.Hkv);
     using A = typename GatherAcc<T>::type;
     A acc[DPL];
 #pragma unroll
     for (int j = 0; j < DPL; ++j) acc[j] = 0;
-    for_each_query(p, K.m0, K.m1, K.m2, [&](int o0, int o1, int o2, int i0, int i1, int i2, int e) {
-        const float g = to_f(da[lda.at(K.b, o0, o1, o2, K.h) + e]);
-        float qv[DPL];
-        load_run<T, DPL>(q + lq.at(K.b, i0, i1, i2, K.h), d0, p.Dqk, vec, qv);
+    if (vec && unit_strides(p)) {
+        struct Step {
+            typename R::Raw x;
+            T w;
+        };
+        walk_queries_pipelined<pipe_depth<T, DPL, 1>(), 2>(
+            p, K.b, K.h, K.m0, K.m1, K.m2, sp, split, {lq, lda},
+            [&](const Offsets<2>& at, int e) {
+                return Step{R::fetch(q + at.o[0], ln, p.Dqk), da[at.o[1] + e]};
+            },
+            [&](const Step& st, int) {
+                const float w = to_f(st.w);
+                float xv[DPL];
+                R::unpack(st.x, xv);
 #pragma unroll
-        for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(g, qv[j], acc[j]);
-    });
+                for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(w, xv[j], acc[j]);
+            });
+    } else {
+        for_each_query_split(p, K.m0, K.m1, K.m2, sp, split, [&](int o0, int o1, int o2, int i0, int i1, int i2, int e) {
+            const float g = to_f(da[lda.at(K.b, o0, o1, o2, K.h) + e]);
+            float qv[DPL];
+            R::load(q + lq.at(K.b, i0, i1, i2, K.h), ln, p.Dqk, vec, qv);
+#pragma unroll
+            for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(g, qv[j], acc[j]);
+        });
+    }
     float res[DPL];
-    gather_out(acc, p.has_scale ? p.scale : 1.f, res);
-    store_run<T, DPL>(dk + ldk.at(K.b, K.m0, K.m1, K.m2, K.h), d0, p.Dqk, vec, res);
+    gather_out<LPQ>(acc, split, p.has_scale ? p.scale : 1.f, res);
+    if (sp == 0) R::store(dk + ldk.at(K.b, K.m0, K.m1, K.m2, K.h), ln, p.Dqk, vec, res);
 }
 
 // ---------------------------------------------------------------------------
 // Split AV backward: dattn (query side) and dv (key side).
 // ---------------------------------------------------------------------------
 template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_av_bwd_a(Prob p, int vec,
+__global__ __launch_bounds__(256) void k_av_bwd_a(Prob p, int vec, int split,
                                                   const T* __restrict__ dout, Lay ldo,
                                                   const T* __restrict__ v, Lay lv,
                                                   T* __restrict__ da, Lay lda) {
-    const long long qi = group_index(LPQ);
+    const long long qi = group_index(LPQ * split);
     if (qi >= static_cast<long long>(p.B) * p.nout * p.Hq) return;
-    const int d0 = (threadIdx.x % LPQ) * DPL;
+    using R = Run<T, DPL, LPQ>;
+    const int ln = threadIdx.x % LPQ;
+    const int sp = (threadIdx.x / LPQ) % split;
     const QPos Q = decode_query(p, qi);
     float dov[DPL];
-    load_run<T, DPL>(dout + ldo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), d0, p.Dv, vec, dov);
+    R::load(dout + ldo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), ln, p.Dv, vec, dov);
     T* row = da + lda.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h);
     if (vec) {
-        walk_neighbors_pipelined<pipe_depth<T, DPL, 1>()>(
-            p, Q.i0, Q.i1, Q.i2, 0, 1,
-            [&](int j0, int j1, int j2, int) { return fetch_run<T, DPL>(v + lv.at(Q.b, j0, j1, j2, Q.h), d0, p.Dv); },
-            [&](const Raw<T, DPL>& r, int e, bool ok) {
+        RowPut<T, LPQ, pipe_depth<T, DPL, 1>()> put{row};
+        walk_neighbors_pipelined<pipe_depth<T, DPL, 1>(), 1>(
+            p, Q.b, Q.h, Q.i0, Q.i1, Q.i2, sp, split, {lv},
+            [&](const Offsets<1>& at, int) { return R::fetch(v + at.o[0], ln, p.Dv); },
+            [&](const typename R::Raw& r, int e, bool ok, int u) {
                 float vv[DPL];
-                unpack_run<T, DPL>(r, d0, p.Dv, vv);
-                float acc = 0.f;
-#pragma unroll
-                for (int j = 0; j < DPL; ++j) acc = fmaf(dov[j], vv[j], acc);
-                const float g = ok ? group_sum<LPQ>(acc) : 0.f;
-                if (d0 == 0) row[e] = from_f<T>(g);
+                R::unpack(r, vv);
+                const float acc = R::dot(dov, vv, ln, p.Dv, vec);
+                const float g = ok ? lane_sum<LPQ>(acc) : 0.f;
+                put.add(ln, u, e, from_f<T>(g));
             });
+        put.flush();
         return;
     }
-    for_each_neighbor(p, Q.i0, Q.i1, Q.i2, [&](int j0, int j1, int j2, int e, bool ok) {
+    for_each_neighbor_split(p, Q.i0, Q.i1, Q.i2, sp, split, [&](int j0, int j1, int j2, int e, bool ok) {
         float g = 0.f;
         if (ok) {
             float vv[DPL];
-            load_run<T, DPL>(v + lv.at(Q.b, j0, j1, j2, Q.h), d0, p.Dv, vec, vv);
-            float acc = 0.f;
-#pragma unroll
-            for (int j = 0; j < DPL; ++j) acc = fmaf(dov[j], vv[j], acc);
-            g = group_sum<LPQ>(acc);
+            R::load(v + lv.at(Q.b, j0, j1, j2, Q.h), ln, p.Dv, vec, vv);
+            const float acc = R::dot(dov, vv, ln, p.Dv, vec);
+            g = lane_sum<LPQ>(acc);
         }
-        if (d0 == 0) row[e] = from_f<T>(g);
+        if (ln == 0) row[e] = from_f<T>(g);
     });
 }
 
 template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_av_bwd_v(Prob p, int vec,
+__global__ __launch_bounds__(256) void k_av_bwd_v(Prob p, int vec, int split,
                                                   const T* __restrict__ dout, Lay ldo,
                                                   const T* __restrict__ attn, Lay la,
                                                   T* __restrict__ dv, Lay ldv) {
-    const long long ki = group_index(LPQ);
+    const long long ki = group_index(LPQ * split);
     if (ki >= static_cast<long long>(p.B) * p.nkey * p.Hkv) return;
-    const int d0 = (threadIdx.x % LPQ) * DPL;
+    using R = Run<T, DPL, LPQ>;
+    const int ln = threadIdx.x % LPQ;
+    const int sp = (threadIdx.x / LPQ) % split;
     const KPos K = decode_key(p, ki, p.Hkv);
     using A = typename GatherAcc<T>::type;
     A acc[DPL];
 #pragma unroll
     for (int j = 0; j < DPL; ++j) acc[j] = 0;
-    for_each_query(p, K.m0, K.m1, K.m2, [&](int o0, int o1, int o2, int, int, int, int e) {
-        const float a = to_f(attn[la.at(K.b, o0, o1, o2, K.h) + e]);
-        float dov[DPL];
-        load_run<T, DPL>(dout + ldo.at(K.b, o0, o1, o2, K.h), d0, p.Dv, vec, dov);
+    if (vec && unit_strides(p)) {
+        struct Step {
+            typename R::Raw x;
+            T w;
+        };
+        walk_queries_pipelined<pipe_depth<T, DPL, 1>(), 2>(
+            p, K.b, K.h, K.m0, K.m1, K.m2, sp, split, {ldo, la},
+            [&](const Offsets<2>& at, int e) {
+                return Step{R::fetch(dout + at.o[0], ln, p.Dv), attn[at.o[1] + e]};
+            },
+            [&](const Step& st, int) {
+                const float w = to_f(st.w);
+                float xv[DPL];
+                R::unpack(st.x, xv);
 #pragma unroll
-        for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(a, dov[j], acc[j]);
-    });
+                for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(w, xv[j], acc[j]);
+            });
+    } else {
+        for_each_query_split(p, K.m0, K.m1, K.m2, sp, split, [&](int o0, int o1, int o2, int, int, int, int e) {
+            const float a = to_f(attn[la.at(K.b, o0, o1, o2, K.h) + e]);
+            float dov[DPL];
+            R::load(dout + ldo.at(K.b, o0, o1, o2, K.h), ln, p.Dv, vec, dov);
+#pragma unroll
+            for (int j = 0; j < DPL; ++j) acc[j] = gather_fma(a, dov[j], acc[j]);
+        });
+    }
     float res[DPL];
-    gather_out(acc, 1.f, res);
-    store_run<T, DPL>(dv + ldv.at(K.b, K.m0, K.m1, K.m2, K.h), d0, p.Dv, vec, res);
+    gather_out<LPQ>(acc, split, 1.f, res);
+    if (sp == 0) R::store(dv + ldv.at(K.b, K.m0, K.m1, K.m2, K.h), ln, p.Dv, vec, res);
 }
 
 // ---------------------------------------------------------------------------
@@ -754,20 +1026,25 @@ inline unsigned grid_for(long long groups, int lpq) {
     return static_cast<unsigned>((threads + 255) / 256);
 }
 
-// Lane groups per query (key) for the fused vector kernels.  Each group walks
-// its neighbours (attending queries) one after another, every step waiting
-// on its loads, so a small problem (few groups) is bound by that chain.
-// Splitting the walk over up to 8 groups, until the launch holds about 8
-// waves per SIMD of a 256-CU device, shortens the chain; groups stay within
-// one wave (lpq * split <= 64) and never outnumber the split axis's kernel
-// positions.  NATTEN_HIP_SPLIT=n fixes it (tuning).
+// Lane groups per query (key).  Each group walks its neighbours (attending
+// queries) one after another, so a small problem (few groups) is bound by that
+// chain.  Splitting the walk over up to 8 groups, until the launch holds about
+// 1.5 waves per SIMD of a 256-CU device, shortens the chain; past that the
+// walks are bound by issue and L1 and the groups' own overhead shows.  fp32,
+// all launches of one pass, us, split 1 / 2 / 4 / 8:
+//   split 2 x 20 x 28 x 4, dim 64, 7 x 7     560 waves  110 / 83 / 73 / -
+//   fused 2 x 28 x 28 x 4, dim 64, 11 x 11   784 waves  154 / 107 / - / 129
+//   split 4 x 45 x 61 x 4, dim 32, 7 x 7    2745 waves  159 / 161 / 181 / -
+//   split 4 x 2048 x 4, dim 64, 33          4096 waves  131 / 150 / - / -
+// Groups stay within one wave (lpq * split <= 64) and never outnumber the
+// split axis's kernel positions.  NATTEN_HIP_SPLIT=n fixes it (tuning).
 inline int choose_split(const Prob& p, long long groups, int lpq) {
     static const int forced = [] {
         const char* e = std::getenv("NATTEN_HIP_SPLIT");
         return e ? std::atoi(e) : 0;
     }();
     const int kmax = p.ax[split_axis(p)].k;
-    constexpr long long kTargetWaves = 256LL * 4 * 8;
+    constexpr long long kTargetWaves = 256LL * 4 * 3 / 2;
     int split = 1;
     if (forced > 0) {
         while (split * 2 <= forced && split * 2 * lpq <= 64) split *= 2;
@@ -796,7 +1073,8 @@ struct LQK {
     static hipError_t run(const Prob& p, int vec, const void* q, Lay lq, const void* k, Lay lk, void* a, Lay la,
                           hipStream_t s) {
         const long long n = static_cast<long long>(p.B) * p.nout * p.Hq;
-        NA_LAUNCH("na_qk", (k_qk<T, DPL, LPQ>), dim3(grid_for(n, LPQ)), dim3(256), 0, s, p, vec, (const T*)q, lq,
+        const int split = choose_split(p, n, LPQ);
+        NA_LAUNCH("na_qk", (k_qk<T, DPL, LPQ>), dim3(grid_for(n, LPQ * split)), dim3(256), 0, s, p, vec, split, (const T*)q, lq,
                            (const T*)k, lk, (T*)a, la);
         return hipGetLastError();
     }
@@ -807,7 +1085,8 @@ struct LAV {
     static hipError_t run(const Prob& p, int vec, const void* a, Lay la, const void* v, Lay lv, void* o, Lay lo,
                           hipStream_t s) {
         const long long n = static_cast<long long>(p.B) * p.nout * p.Hq;
-        NA_LAUNCH("na_av", (k_av<T, DPL, LPQ>), dim3(grid_for(n, LPQ)), dim3(256), 0, s, p, vec, (const T*)a, la,
+        const int split = choose_split(p, n, LPQ);
+        NA_LAUNCH("na_av", (k_av<T, DPL, LPQ>), dim3(grid_for(n, LPQ * split)), dim3(256), 0, s, p, vec, split, (const T*)a, la,
                            (const T*)v, lv, (T*)o, lo);
         return hipGetLastError();
     }
@@ -842,14 +1121,16 @@ struct LQKBwd {
                           Lay lk, void* dq, Lay ldq, void* dk, Lay ldk, int sides, hipStream_t s) {
         if (sides & kQuerySide) {
             const long long nq = static_cast<long long>(p.B) * p.nout * p.Hq;
-            NA_LAUNCH("na_qk_bwd_q", (k_qk_bwd_q<T, DPL, LPQ>), dim3(grid_for(nq, LPQ)), dim3(256), 0, s, p, vec,
+            const int split = choose_split(p, nq, LPQ);
+            NA_LAUNCH("na_qk_bwd_q", (k_qk_bwd_q<T, DPL, LPQ>), dim3(grid_for(nq, LPQ * split)), dim3(256), 0, s, p, vec, split,
                       (const T*)da, lda, (const T*)k, lk, (T*)dq, ldq);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
         }
         if (!(sides & kKeySide)) return hipSuccess;
         const long long nk = static_cast<long long>(p.B) * p.nkey * p.Hkv;
-        NA_LAUNCH("na_qk_bwd_k", (k_qk_bwd_k<T, DPL, LPQ>), dim3(grid_for(nk, LPQ)), dim3(256), 0, s, p, vec,
+        const int split = choose_split(p, nk, LPQ);
+        NA_LAUNCH("na_qk_bwd_k", (k_qk_bwd_k<T, DPL, LPQ>), dim3(grid_for(nk, LPQ * split)), dim3(256), 0, s, p, vec, split,
                            (const T*)da, lda, (const T*)q, lq, (T*)dk, ldk);
         return hipGetLastError();
     }
@@ -861,14 +1142,16 @@ struct LAVBwd {
                           Lay lv, void* da, Lay lda, void* dv, Lay ldv, int sides, hipStream_t s) {
         if (sides & kQuerySide) {
             const long long nq = static_cast<long long>(p.B) * p.nout * p.Hq;
-            NA_LAUNCH("na_av_bwd_a", (k_av_bwd_a<T, DPL, LPQ>), dim3(grid_for(nq, LPQ)), dim3(256), 0, s, p, vec,
+            const int split = choose_split(p, nq, LPQ);
+            NA_LAUNCH("na_av_bwd_a", (k_av_bwd_a<T, DPL, LPQ>), dim3(grid_for(nq, LPQ * split)), dim3(256), 0, s, p, vec, split,
                       (const T*)dout, ldo, (const T*)v, lv, (T*)da, lda);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
         }
         if (!(sides & kKeySide)) return hipSuccess;
         const long long nk = static_cast<long long>(p.B) * p.nkey * p.Hkv;
-        NA_LAUNCH("na_av_bwd_v", (k_av_bwd_v<T, DPL, LPQ>), dim3(grid_for(nk, LPQ)), dim3(256), 0, s, p, vec,
+        const int split = choose_split(p, nk, LPQ);
+        NA_LAUNCH("na_av_bwd_v", (k_av_bwd_v<T, DPL, LPQ>), dim3(grid_for(nk, LPQ * split)), dim3(256), 0, s, p, vec, split,
                            (const T*)dout, ldo, (const T*)a, la, (T*)dv, ldv);
         return hipGetLastError();
     }
