@@ -24,12 +24,13 @@
 // What bounds it: LDS reads (a chunk's 8 KB of K and V rows per 16 queries)
 // and the latency of a wave's score -> maximum -> exponential -> product
 // chain; 8 waves and bands of 4 rows measured as fast as 4 waves or bands of
-// 2 (16 waves: 28 % slower).  Measured, general tile (or vector) kernels ->
-// these: 13 x 13, head dim 64, fp16, 4 x 135 x 241, 8 heads, forward 2350 ->
-// 334 us; bf16 4 x 64 x 64, 8 heads, forward 275 -> 49, dQ 981 -> 124, dK/dV
-// 968 -> 105 us; head dim 128, 4 heads 501 / 1043 / 998 -> 53 / 139 / 107 us;
-// 11 x 11, head dim 32, 4 x 61 x 130, 8 heads 103 / 139 / 128 -> 57 / 128 /
-// 91 us.
+// 2 (16 waves: 28 % slower).  Measured, general tile (or, *, vector) kernels
+// -> these: 13 x 13, head dim 64, fp16, 4 x 135 x 241, 8 heads, forward 2350
+// -> 300 us; bf16 4 x 64 x 64, 8 heads, forward 275 -> 37, dQ 981* -> 71,
+// dK/dV 968* -> 99 us; head dim 128, 4 heads 501* / 1043* / 998* -> 42 / 83 /
+// 85 us; 11 x 11, head dim 32, 4 x 61 x 130, 8 heads 103 / 139 / 128 -> 50 /
+// 83 / 69 us.  (*: the two-term products of band_sides; one term takes 36 /
+// 61 / 78 in the first case.)
 //
 // The geometry is computed in the kernel (no tables): every call, captured
 // or not, runs the same code.  MFMA lane layouts, the swizzle and the masks
@@ -284,15 +285,39 @@ __device__ __forceinline__ void band_score(const unsigned char* X, const BandOff
     }
 }
 
-template <typename T, int D>
-__device__ __forceinline__ void band_accumulate(const unsigned char* X, const BandOff<D>& o, int c, uint4 packed,
-                                                f32x4_t (&acc)[D / 16]) {
+// What rounding v to `packed` left over, packed in turn.
+template <typename T>
+__device__ __forceinline__ uint4 pack_rest(const f32x4_t (&v)[2], uint4 packed) {
+    const uint32_t w[4] = {packed.x, packed.y, packed.z, packed.w};
+    f32x4_t r[2];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t h = w[i >> 1] >> (16 * (i & 1)) & 0xffffu;
+        float f;
+        if constexpr (std::is_same_v<T, bf16>)
+            f = __uint_as_float(h << 16);
+        else
+            f = static_cast<float>(__builtin_bit_cast(f16, static_cast<uint16_t>(h)));
+        r[i >> 2][i & 3] = v[i >> 2][i & 3] - f;
+    }
+    return pack8<T>(r);
+}
+
+// acc += X^T of chunk c times v, v as one 16-bit term or (TWO) as two.
+template <typename T, int D, bool TWO>
+__device__ __forceinline__ void band_accumulate(const unsigned char* X, const BandOff<D>& o, int c,
+                                                const f32x4_t (&v)[2], f32x4_t (&acc)[D / 16]) {
+    const uint4 packed = pack8<T>(v);
+    uint4 rest;
+    if constexpr (TWO) rest = pack_rest<T>(v, packed);
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) {
         const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(X + o.t[0][db] + c * 32 * D * 2));
         const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(X + o.t[1][db] + c * 32 * D * 2));
         const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-        acc[db] = Mma<T>::run(make_uint4(l2.x, l2.y, h2.x, h2.y), packed, acc[db]);
+        const uint4 x = make_uint4(l2.x, l2.y, h2.x, h2.y);
+        acc[db] = Mma<T>::run(x, packed, acc[db]);
+        if constexpr (TWO) acc[db] = Mma<T>::run(x, rest, acc[db]);
     }
 }
 
@@ -321,7 +346,7 @@ __device__ __forceinline__ void band_redo_fwd(const void* kargs, int b, int h, i
     if (grp == 0) bh_ptr(A.lse_out, A.ll, b, h)[vol_off(A.ll, pos)] = lse_v;
 }
 
-template <typename T, int D, int SL>
+template <typename T, int D, int SL, bool TWO>
 __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd(BandArgs<T> args) {
     constexpr int NC = kBandChunks<D>, RPC = 32 / SL, BUF = 2 * kBandOp<D>;
     const Prob& p = args.p;
@@ -404,9 +429,10 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd
                     for (int bb = 0; bb < 2; ++bb)
 #pragma unroll
                         for (int i = 0; i < 4; ++i) s[c][bb][i] = __builtin_amdgcn_exp2f(fmaf(s[c][bb][i], sc2, o));
+                    band_accumulate<T, D, TWO>(Vb, off, c, s[c], acc);
                     const uint4 pk = pack8<T>(s[c]);
-                    band_accumulate<T, D>(Vb, off, c, pk, acc);
                     lacc = Mma<T>::run(ones, pk, lacc);
+                    if constexpr (TWO) lacc = Mma<T>::run(ones, pack_rest<T>(s[c], pk), lacc);
                 }
             }
         }
@@ -446,7 +472,7 @@ __device__ __forceinline__ void band_redo_bwd_q(const void* kargs, int b, int h,
     store_rows<T, D>(bh_ptr(A.dq, A.ldq, b, h), vol_off(A.ldq, pos), grp, acc, A.p.scale);
 }
 
-template <typename T, int D, int SL>
+template <typename T, int D, int SL, bool TWO>
 __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_q(BandArgs<T> args) {
     constexpr int NC = kBandChunks<D>, RPC = 32 / SL, BUF = 2 * kBandOp<D>;
     const Prob& p = args.p;
@@ -516,7 +542,7 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         s[bb][i] = __builtin_amdgcn_exp2f(fmaf(s[bb][i], sc2, o)) * (dp[bb][i] - di);
-                band_accumulate<T, D>(Kb, off, c, pack8<T>(s), acc);
+                band_accumulate<T, D, TWO>(Kb, off, c, s, acc);
             }
         }
         if (pass == 1 && cpass == 0) {
@@ -567,7 +593,7 @@ __device__ __forceinline__ void band_redo_bwd_kv(const void* kargs, int b, int h
     store_rows<T, D>(bh_ptr(A.dk, A.ldk, b, hk), vol_off(A.ldk, pos), grp, g, A.p.scale);
 }
 
-template <typename T, int D, int SL>
+template <typename T, int D, int SL, bool TWO>
 __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_kv(BandArgs<T> args) {
     constexpr int NC = kBandChunks<D>, RPC = 32 / SL, BUF = 2 * kBandOp<D>, NS = NC * 32;
     const Prob& p = args.p;
@@ -670,8 +696,8 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
                         s[bb][i] = __builtin_amdgcn_exp2f(fmaf(s[bb][i], sc2, nl[bb][i]));
                         dp[bb][i] *= s[bb][i];
                     }
-                band_accumulate<T, D>(Gb, off, c, pack8<T>(s), gv);
-                band_accumulate<T, D>(Qb, off, c, pack8<T>(dp), gk);
+                band_accumulate<T, D, TWO>(Gb, off, c, s, gv);
+                band_accumulate<T, D, TWO>(Qb, off, c, dp, gk);
             }
         }
         return more;
@@ -724,9 +750,12 @@ constexpr size_t kBandLdsKv = kBandLds<T, D> + (4 * kBandChunks<D> * 32 + 8) * s
 
 template <typename T, int D>
 void band_audit_dim(LdsAudit& a) {
-    audit_one(k_band_fwd<T, D, 32>, "k_band_fwd", a);
-    audit_one(k_band_bwd_q<T, D, 32>, "k_band_bwd_q", a);
-    audit_one(k_band_bwd_kv<T, D, 32>, "k_band_bwd_kv", a);
+    audit_one(k_band_fwd<T, D, 32, false>, "k_band_fwd", a);
+    audit_one(k_band_fwd<T, D, 32, true>, "k_band_fwd", a);
+    audit_one(k_band_bwd_q<T, D, 32, false>, "k_band_bwd_q", a);
+    audit_one(k_band_bwd_q<T, D, 32, true>, "k_band_bwd_q", a);
+    audit_one(k_band_bwd_kv<T, D, 32, false>, "k_band_bwd_kv", a);
+    audit_one(k_band_bwd_kv<T, D, 32, true>, "k_band_bwd_kv", a);
 }
 
 // No static LDS in any instance (see lds_base): checked once per process.
@@ -754,7 +783,7 @@ bool band_switch() {
 
 template <typename T, int D>
 hipError_t band_fwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,
-                        Lay lo, float* lse, Lay ll, hipStream_t s) {
+                        Lay lo, float* lse, Lay ll, bool two, hipStream_t s) {
     BandArgs<T> a{};
     a.p = p;
     a.g = band_geo(p, band_columns(p.ax[2].k, false), p.Hq);
@@ -770,7 +799,7 @@ hipError_t band_fwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
     a.ll = to_k(ll);
     a.ab = band_plane(p, lk, D);
     a.bb = band_plane(p, lv, D);
-    auto kern = k_band_fwd<T, D, 32>;
+    auto kern = two ? k_band_fwd<T, D, 32, true> : k_band_fwd<T, D, 32, false>;
     const hipError_t e = allow_lds(kern, kBandLds<T, D>);
     if (e != hipSuccess) return e;
     NA_LAUNCH("na_fwd_band", kern, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
@@ -782,7 +811,7 @@ template <typename T, int D>
 hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                         const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll, const float* dlse,
                         Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv, float* delta, Lay lde,
-                        int sides, hipStream_t s) {
+                        int sides, bool two, hipStream_t s) {
     BandArgs<T> a{};
     a.p = p;
     a.g = band_geo(p, band_columns(p.ax[2].k, false), p.Hq);
@@ -813,7 +842,7 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
     a.bb = band_plane(p, lv, D);
     hipError_t e;
     if (sides & kQuerySide) {
-        auto kq = k_band_bwd_q<T, D, 32>;
+        auto kq = two ? k_band_bwd_q<T, D, 32, true> : k_band_bwd_q<T, D, 32, false>;
         if ((e = allow_lds(kq, kBandLds<T, D>)) != hipSuccess) return e;
         NA_LAUNCH("na_bwd_q_band", kq, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
                   (kBandLds<T, D>), s, a);
@@ -823,7 +852,7 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
     a.g = band_geo(p, band_columns(p.ax[2].k, true), p.Hkv);
     a.ab = band_plane(p, lq, D);
     a.bb = band_plane(p, ldo, D);
-    auto kk = k_band_bwd_kv<T, D, 32>;
+    auto kk = two ? k_band_bwd_kv<T, D, 32, true> : k_band_bwd_kv<T, D, 32, false>;
     if ((e = allow_lds(kk, kBandLdsKv<T, D>)) != hipSuccess) return e;
     NA_LAUNCH("na_bwd_kv_band", kk, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
               (kBandLdsKv<T, D>), s, a);
@@ -848,12 +877,17 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
 // * both sides for 10 to 16 columns (past the 8x8 tile kernels), and at head
 //   dim 128 from 8: there the general tiles' border unions cross 16 columns
 //   and their rows double (9 x 9, 8 x 64 x 64 x 4 heads: forward 97 -> 61
-//   us, the backward left the tiles, 995 + 950 -> 110 + 94 us; at 7 x 7 both
+//   us, the backward left the tiles, 995 + 950 -> 129 + 117 us; at 7 x 7 both
 //   are level, 57 + 76 + 90 against 58 + 99 + 87);
 // * the key side alone where the 8x8 tiles serve the query side but some key
 //   tile's union does not fit them (`lean`: they take the problem; 9 x 9, 8 x
 //   64 x 64 x 8: dK/dV 222 -> 56 us at head dim 32, 613 -> 111 at 64; 7 x 7
 //   on 32 x 22 x 22 x 8: 57 -> 37).
+// Where the general tiles cannot hold the problem either, the alternative is
+// the vector kernels, whose probabilities and their gradients stay in fp32:
+// there they enter the matrix products as two 16-bit terms (TWO; the rest
+// after rounding is the second), which keeps 16 (fp16: 22) of their bits.  The
+// callers ask for it (`two`).
 // `lays`: every 16-bit operand and fp32 row operand of the call.  The answer
 // depends on the problem alone, never on which tables exist.
 int band_sides(const Prob& p, int dtype, bool aligned, bool lean, std::initializer_list<Lay> lays) {
@@ -877,16 +911,16 @@ int band_sides(const Prob& p, int dtype, bool aligned, bool lean, std::initializ
 }
 
 hipError_t band_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,
-                        Lay lo, float* lse, Lay ll, int dtype, hipStream_t s) {
-    NA_BAND_DISPATCH(band_fwd_run, p, q, lq, k, lk, v, lv, o, lo, lse, ll, s);
+                        Lay lo, float* lse, Lay ll, int dtype, hipStream_t s, bool two) {
+    NA_BAND_DISPATCH(band_fwd_run, p, q, lq, k, lk, v, lv, o, lo, lse, ll, two, s);
 }
 
 hipError_t band_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                          const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll, const float* dlse,
                          Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv, float* delta, Lay lde,
-                         int dtype, hipStream_t s, int sides) {
+                         int dtype, hipStream_t s, int sides, bool two) {
     NA_BAND_DISPATCH(band_bwd_run, p, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
-                     ldv, delta, lde, sides, s);
+                     ldv, delta, lde, sides, two, s);
 }
 
 }  // namespace na

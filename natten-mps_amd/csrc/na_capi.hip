@@ -186,14 +186,15 @@ int natten_hip_forward(const natten_problem_t* p, const void* q, const natten_la
                                               to_lay(llse), p->dtype, s);
         if (e != hipErrorNotSupported) return launch_status(e, "forward");
     }
+    const bool mfma = use_mfma() && na::mfma_eligible(P, p->dtype, D, vec != 0, false) &&
+                      na::mfma_offsets_fit(P, {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)});
     if (use_mfma() && (na::band_sides(P, p->dtype, vec != 0, false,
                                       {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)}) &
                        na::kQuerySide))
         return launch_status(na::band_forward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), lse,
-                                              to_lay(llse), p->dtype, s),
+                                              to_lay(llse), p->dtype, s, !mfma),
                              "forward");
-    if (use_mfma() && na::mfma_eligible(P, p->dtype, D, vec != 0, false) &&
-        na::mfma_offsets_fit(P, {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)})) {
+    if (mfma) {
         return launch_status(na::mfma_forward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), lse,
                                               to_lay(llse), p->dtype, s),
                              "forward");
@@ -241,9 +242,11 @@ struct BackwardCall {
         return na::lean_backward(P, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
                                  ldv, delta, lde, dtype, s, sides);
     }
-    hipError_t band(int sides) const {
+    // two: probabilities in two 16-bit terms, for calls whose alternative is
+    // the vector kernels
+    hipError_t band(int sides, bool two) const {
         return na::band_backward(P, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
-                                 ldv, delta, lde, dtype, s, sides);
+                                 ldv, delta, lde, dtype, s, sides, two);
     }
     hipError_t mfma(int sides, const na::GlobalSet* g = nullptr) const {
         return na::mfma_backward(P, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
@@ -275,13 +278,14 @@ int backward_impl(const natten_problem_t* p, const na::Prob& P, const void* q, c
     // hold, then the general tiles
     const bool lean = c.lean_ok();
     const int band = c.band_sides(lean);
-    if (band == kBothSides) return launch_status(c.band(kBothSides), "backward");
-    if (band == na::kKeySide) {
+    if (band) {
+        const bool two = !c.mfma_ok(kBothSides);
+        if (two || band == kBothSides) return launch_status(c.band(kBothSides, two), "backward");
         // the query side as without the band kernels (the general tiles give
         // the lean ones' bits where no table of those exists)
         hipError_t e = c.lean(na::kQuerySide);
-        if (e == hipErrorNotSupported) e = c.mfma_ok(na::kQuerySide) ? c.mfma(na::kQuerySide) : c.band(na::kQuerySide);
-        return launch_status(e == hipSuccess ? c.band(na::kKeySide) : e, "backward");
+        if (e == hipErrorNotSupported) e = c.mfma(na::kQuerySide);
+        return launch_status(e == hipSuccess ? c.band(na::kKeySide, false) : e, "backward");
     }
     if (lean) {
         const hipError_t e = c.lean(kBothSides);
@@ -489,7 +493,7 @@ int natten_hip_backward_global(const natten_problem_t* p, const void* q, const n
     if (e == hipSuccess) {
         const bool lean = c.lean_ok();
         if (c.band_sides(lean) & na::kKeySide) {
-            e = c.band(na::kKeySide);
+            e = c.band(na::kKeySide, false);
         } else {
             e = lean ? c.lean(na::kKeySide) : hipErrorNotSupported;
             if (e == hipErrorNotSupported) e = c.mfma(na::kKeySide);

@@ -167,11 +167,11 @@ bool lean_key_tiles_fit(const Prob& p);
 // 8x8 tile kernels take the problem's query side.
 int band_sides(const Prob& p, int dtype, bool aligned, bool lean, std::initializer_list<Lay> lays);
 hipError_t band_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,
-                        Lay lo, float* lse, Lay ll, int dtype, hipStream_t s);
+                        Lay lo, float* lse, Lay ll, int dtype, hipStream_t s, bool two);
 hipError_t band_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,
                          const void* o, Lay lo, const void* dout, Lay ldo, const float* lse, Lay ll,
                          const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv, Lay ldv,
-                         float* delta, Lay lde, int dtype, hipStream_t s, int sides = kQuerySide | kKeySide);
+                         float* delta, Lay lde, int dtype, hipStream_t s, int sides, bool two);
 
 // Key side of the global keys' backward (na_global.hip): dk and dv of the
 // global keys (summed over every query of each q head of the group), from the

@@ -44,12 +44,12 @@ def _inputs(seed, shapes, dtype):
 # border, or of classes about twice the kernel, do not fit those.
 KEY_SIDE_CASES = [
     ((40, 64), 2, 2, 64, (9, 9), (1, 1), (False, False), False),
-    ((17, 30), 4, 2, 64, (9, 9), (1, 1), (False, False), False),
     ((40, 32), 2, 2, 32, (8, 8), (1, 1), (False, False), False),
     ((22, 22), 2, 2, 32, (7, 7), (1, 1), (False, False), True),
     ((48, 48), 2, 1, 32, (9, 9), (2, 2), (False, False), False),
 ]
-# Head dim 128 takes both sides from 8 columns.
+# Head dim 128 takes both sides from 8 columns; so does a backward whose key
+# side no other tile kernel holds.
 WIDE_CASES = [((21, 37), 2, 1, 128, (9, 9), (1, 1), (True, False), False),
               ((19, 40), 1, 1, 128, (5, 8), (1, 2), (False, False), True)]
 
@@ -100,6 +100,44 @@ def _check(case, dtype, names):
     for name, a, b in zip(("out", "lse", "dq", "dk", "dv"), (out, lse, *grads), (ref, ref_lse, *rgrads)):
         assert_parity(a.detach().cpu(), b.detach(), dtype, name)
     return launched
+
+
+# Calls whose alternative is the vector kernels (fp32 probabilities).
+TWO_TERM_CASES = [((24, 40), 64, (13, 13)), ((17, 30), 64, (9, 9)), ((24, 33), 128, (13, 15)),
+                  ((30, 21), 128, (9, 9)), ((80, 20), 32, (33, 13))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", TWO_TERM_CASES)
+def test_two_term_products_add_no_error(case, dtype):
+    """The gradients' error against float64 is that of rounding them once
+    (one-term probabilities, rounded as often as the result, add to that; two
+    terms leave 2^-17, a 256th of one rounding)."""
+    from natten_mps_amd import functional as F
+    from natten_mps_amd._core import _lib
+
+    sp, dim, ks = case
+    print(case, dtype, flush=True)
+    ts = _inputs(35, [(2, *sp, 2, dim)] * 4, dtype)
+    leaves = [t.to(DEV).requires_grad_(True) for t in ts[:3]]
+    _lib.profile_read(reset=True)
+    _lib.profile_enable(True)
+    try:
+        out = F.na2d(*leaves, kernel_size=ks)
+        grads = torch.autograd.grad(out, leaves, ts[3].to(DEV))
+        torch.cuda.synchronize()
+    finally:
+        _lib.profile_enable(False)
+    assert {"na_bwd_q_band", "na_bwd_kv_band"} <= set(_lib.profile_read(reset=True))
+    q, k, v = (t.double().requires_grad_(True) for t in ts[:3])
+    one = (1, 1)
+    w = torch.softmax(P.na2d_qk_forward(q, k, ks, one, one, (False, False), dim ** -0.5), dim=-1)
+    ref = P.na2d_av_forward(w, v, ks, one, one, (False, False))
+    rgrads = torch.autograd.grad(ref, (q, k, v), ts[3].double())
+    for name, a, b in zip(("dq", "dk", "dv"), grads, rgrads):
+        b = b.detach()
+        err = float((a.cpu().double() - b).norm())
+        assert err <= 1.03 * float((b.to(dtype).double() - b).norm()), (name, err)
 
 
 @pytest.mark.parametrize("tokens", [1, 7])
