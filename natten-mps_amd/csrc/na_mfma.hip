@@ -1316,10 +1316,28 @@ const int* forced_shape() {
 // waves): a depth window of K0 then stages K0 + 1 slices for two planes
 // instead of K0 for one. On config 5 (16 x 32 x 32, K 3 x 7 x 7, head dim
 // 64) that made both kernels about 11 % faster; the dK/dV kernel, limited by
-// its registers to one such workgroup per CU, keeps 64 items.
-bool deep_query_tile(const Prob& p, Kind kind, const int (&n)[3]) {
-    return (kind == kForward || kind == kBackwardQ) && fused_items() == kMaxItems && n[0] >= 2 &&
+// its registers to one such workgroup per CU, keeps 64 items.  At head dim 32
+// a slice is half as large and more workgroups fit: one plane measured faster
+// (2 x 16 x 32 x 32 x 8, 3 x 7 x 7: 55 / 57 -> 49 / 51 us).
+bool deep_query_tile(const Prob& p, Kind kind, int D, const int (&n)[3]) {
+    return (kind == kForward || kind == kBackwardQ) && D > 32 && fused_items() == kMaxItems && n[0] >= 2 &&
            p.ax[0].k > 1 && n[1] >= 8 && n[2] >= 8;
+}
+
+// Forward and dQ tiles whose 4-wide box has a union of at most 8 columns (K2
+// <= 5) take 8 rows of 4 (and two depth planes where the window has depth):
+// an 8-wide box's union crosses 8 columns and stages rows of 16, half of them
+// empty at K2 = 3 .. 5, and a wave's chunks hold as many.  Forward / dQ, us,
+// bfloat16: 2 x 16 x 32 x 32 x 4, 3 x 5 x 5, head dim 128 150 / 186 -> 54 / 62;
+// 16 x 64 x 64 x 8, 3 x 5 x 5, dim 32 96 / 101 -> 70 / 73, dim 64 (batch 2)
+// 254 / 301 -> 221 / 269; 8 x 64 x 64 x 4, 5 x 5, dim 128 68 / 89 -> 47 / 48,
+// dim 96 67 / 76 -> 37 / 39; level at 3 x 3.  (Key tiles' unions reach further
+// at the borders: 20 to 60 % slower.)  2-D problems at head dim 32 / 64 keep
+// the 8 x 8 box: without their tables the 8x8 tile kernels hand them over, and
+// the bits must not depend on that (with global keys both boxes are level).
+bool narrow_query_tile(const Prob& p, Kind kind, int D, const int (&n)[3]) {
+    return (kind == kForward || kind == kBackwardQ) && fused_items() == kMaxItems && n[1] >= 8 && n[2] >= 8 &&
+           p.ax[2].k <= 5 && (p.ax[0].len > 1 || D >= 96);
 }
 
 // LDS a forward / dQ workgroup adds for global keys: 32 key and 32 value rows.
@@ -1373,9 +1391,15 @@ bool choose_tile(const Prob& p, Kind kind, int D, TileShape& ts, size_t extra_ld
         int T[3];
         for (int a = 0; a < 3; ++a) T[a] = std::min(pow2_at_least(n[a]), forced[a]);
         if (fits(T, kLdsBudget)) return finish();
-    } else if (fused && deep_query_tile(p, kind, n)) {
-        const int T[3] = {2, 8, 8};
-        if (fits(T, kLdsBudget)) return finish();
+    } else {
+        if (narrow_query_tile(p, kind, D, n)) {
+            const int T[3] = {n[0] >= 2 && p.ax[0].k > 1 ? 2 : 1, 8, 4};
+            if (fits(T, kLdsBudget) && ts.rowshift == 3) return finish();
+        }
+        if (deep_query_tile(p, kind, D, n)) {
+            const int T[3] = {2, 8, 8};
+            if (fits(T, kLdsBudget)) return finish();
+        }
     }
     for (int pass = 0; pass < 2; ++pass) {
         const size_t budget = pass == 0 ? kLdsBudget : kLdsBudgetLarge;
