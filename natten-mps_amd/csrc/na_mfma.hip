@@ -1345,7 +1345,7 @@ size_t global_lds(int D) { return static_cast<size_t>(2 * 32) * (D == 96 ? 128 :
 
 // Workgroup box in class coordinates (query items on a strided axis): up to
 // 64 items (4 waves), power-of-two extents, innermost axis first (8 wide
-// unless the problem is 1-D); halved until the staged union fits the LDS
+// unless the problem is 1-D, or the narrow or deep box above); halved until the staged union fits the LDS
 // budget, kLdsBudget first, then kLdsBudgetLarge.
 bool choose_tile(const Prob& p, Kind kind, int D, TileShape& ts, size_t extra_lds = 0, bool varlen = false) {
     const bool key_tile = kind == kBackwardKV || kind == kSplitKey;
