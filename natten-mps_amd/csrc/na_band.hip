@@ -26,7 +26,7 @@
 // chain; 8 waves and bands of 4 rows measured as fast as 4 waves or bands of
 // 2 (16 waves: 28 % slower).  Measured, general tile (or, *, vector) kernels
 // -> these: 13 x 13, head dim 64, fp16, 4 x 135 x 241, 8 heads, forward 2350
-// -> 300 us; bf16 4 x 64 x 64, 8 heads, forward 275 -> 37, dQ 981* -> 71,
+// -> 250 us; bf16 4 x 64 x 64, 8 heads, forward 275 -> 37, dQ 981* -> 71,
 // dK/dV 968* -> 99 us; head dim 128, 4 heads 501* / 1043* / 998* -> 42 / 83 /
 // 85 us; 11 x 11, head dim 32, 4 x 61 x 130, 8 heads 103 / 139 / 128 -> 50 /
 // 83 / 69 us.  (*: the two-term products of band_sides; one term takes 36 /
