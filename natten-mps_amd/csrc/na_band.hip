@@ -303,6 +303,46 @@ __device__ __forceinline__ uint4 pack_rest(const f32x4_t (&v)[2], uint4 packed) 
     return pack8<T>(r);
 }
 
+// Two fp16 terms share fp16's exponents: their sum stops at 2^-25 absolute,
+// where bfloat16's keeps 16 bits of every value.  So fp16 pairs are scaled by
+// powers of two, exact to apply and to take out: P of the key side by 2^15 (P
+// <= 1 up to rounding), dS by a factor of its item's own.  Unscaled, dQ and dK
+// lost up to 7 times their rounding error at dO ~ 1e-3 (97 x 16, head dim
+// 32); scaled, none.  Time: 4 x 64 x 64 x 8, dim 64, 13 x 13, fp16 69 -> 74 us
+// (dQ) and 98 -> 105 us (dK/dV).
+template <typename T, bool TWO>
+constexpr bool kScaled = TWO && std::is_same_v<T, f16>;
+constexpr float kScaleP = 32768.f;
+// Values of a scaled item stay below this (their factor puts a new maximum
+// in [2^13, 2^14)).
+constexpr float kScaleLimit = 32768.f;
+
+// The power of two that moves m >= 0 into [2^13, 2^14); within 2^+-96, so
+// that it and its reciprocal are normal.
+__device__ __forceinline__ float scale_for(float m) {
+    const int e = static_cast<int>(__float_as_uint(m) >> 23 & 0xffu);
+    const int k = 140 - e < 96 ? 140 - e : 96;
+    return __uint_as_float(static_cast<uint32_t>(k < -96 ? 127 - 96 : 127 + k) << 23);
+}
+
+// 1 / x of a power of two from scale_for.
+__device__ __forceinline__ float inv_pow2(float x) { return __uint_as_float((254u << 23) - __float_as_uint(x)); }
+
+// Largest |v| of 8, at least m; NaNs (a masked slot's 0 times infinity) drop out.
+__device__ __forceinline__ float abs_max8(const f32x4_t (&v)[2], float m) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = fmaxf(m, __builtin_fabsf(v[i >> 2][i & 3]));
+    return m;
+}
+
+// Maximum over the four 16-lane rows of the wave, NaNs dropping out.
+__device__ __forceinline__ float max_rows_num(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 // acc += X^T of chunk c times v, v as one 16-bit term or (TWO) as two.
 template <typename T, int D, bool TWO>
 __device__ __forceinline__ void band_accumulate(const unsigned char* X, const BandOff<D>& o, int c,
@@ -382,7 +422,7 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd
     const uint4 ones = make_uint4(Mma<T>::kOnes, Mma<T>::kOnes, Mma<T>::kOnes, Mma<T>::kOnes);
 
     f32x4_t acc[D / 16], lacc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY;
+    float m = -INFINITY, lpart = 0.f;
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     int u0 = 0, bi = 0;
@@ -418,7 +458,8 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd
             const float mref = mnew == -INFINITY ? 0.f : mnew;
             const float corr = __builtin_amdgcn_exp2f(m - mref);
             m = mnew;
-            lacc *= corr;
+            if constexpr (TWO) lpart *= corr;
+            else lacc *= corr;
 #pragma unroll
             for (int db = 0; db < D / 16; ++db) acc[db] *= corr;
 #pragma unroll
@@ -430,9 +471,13 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd
 #pragma unroll
                         for (int i = 0; i < 4; ++i) s[c][bb][i] = __builtin_amdgcn_exp2f(fmaf(s[c][bb][i], sc2, o));
                     band_accumulate<T, D, TWO>(Vb, off, c, s[c], acc);
-                    const uint4 pk = pack8<T>(s[c]);
-                    lacc = Mma<T>::run(ones, pk, lacc);
-                    if constexpr (TWO) lacc = Mma<T>::run(ones, pack_rest<T>(s[c], pk), lacc);
+                    // the row sum: of the rounded values that the product took, or
+                    // (two terms, the rest far below the result's rounding) in fp32
+                    if constexpr (TWO)
+                        lpart += ((s[c][0][0] + s[c][0][1]) + (s[c][0][2] + s[c][0][3])) +
+                                 ((s[c][1][0] + s[c][1][1]) + (s[c][1][2] + s[c][1][3]));
+                    else
+                        lacc = Mma<T>::run(ones, pack8<T>(s[c]), lacc);
                 }
             }
         }
@@ -441,7 +486,7 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd
 #pragma unroll 1
     while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{})) {
     }
-    const float lsum = lacc[0];
+    const float lsum = TWO ? sum_rows(lpart) : lacc[0];
     const bool redo = ln.valid && item_nonfinite(lane_sum(acc, lsum));
     if (ln.valid) {
         store_rows<T, D>(bh_ptr(args.out, args.lo, t.b, t.h), vol_off(args.lo, ln.pos), grp, acc, 1.f / lsum);
@@ -512,6 +557,7 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     float part = 0.f, di = 0.f;
+    float pmax = 0.f, gs = 1.f;  // scaled: largest |P dP|, and dS's factor
     int bi = 0, pass = 0;
     const auto step = [&](auto BC) {
         constexpr int B = decltype(BC)::value;
@@ -535,13 +581,23 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
             band_score<T, D>(Kb, off, c, qf, cb, s);
             band_score<T, D>(Vb, off, c, gf, zero, dp);
             if (cpass == 0) {
-                part = delta_part(s, dp, sc2, o, part);
+                if constexpr (kScaled<T, TWO>) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const float e = __builtin_amdgcn_exp2f(fmaf(s[i >> 2][i & 3], sc2, o)), x = dp[i >> 2][i & 3];
+                        part = fmaf(e, x, part);
+                        pmax = fmaxf(pmax, __builtin_fabsf(e * x));
+                    }
+                } else {
+                    part = delta_part(s, dp, sc2, o, part);
+                }
             } else {
 #pragma unroll
                 for (int bb = 0; bb < 2; ++bb)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        s[bb][i] = __builtin_amdgcn_exp2f(fmaf(s[bb][i], sc2, o)) * (dp[bb][i] - di);
+                        s[bb][i] = __builtin_amdgcn_exp2f(fmaf(s[bb][i], sc2, o)) *
+                                   (kScaled<T, TWO> ? fmaf(dp[bb][i], gs, -gs * di) : dp[bb][i] - di);
                 band_accumulate<T, D, TWO>(Kb, off, c, s, acc);
             }
         }
@@ -552,6 +608,8 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
                                      bh_ptr(args.o, args.lo, t.b, t.h) + vol_off(args.lo, ln.pos)) -
                      dl;
             if (ln.valid && grp == 0) bh_ptr(args.delta_out, args.lde, t.b, t.h)[vol_off(args.lde, ln.pos)] = di;
+            // |dS| <= |P dP| + |delta|, as P <= 1
+            if constexpr (kScaled<T, TWO>) gs = scale_for(max_rows_num(pmax) + __builtin_fabsf(di));
         }
         return more;
     };
@@ -559,7 +617,9 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
     while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{})) {
     }
     const bool redo = ln.valid && item_nonfinite(lane_sum(acc, 0.f));
-    if (ln.valid) store_rows<T, D>(bh_ptr(args.dq, args.ldq, t.b, t.h), vol_off(args.ldq, ln.pos), grp, acc, p.scale);
+    if (ln.valid)
+        store_rows<T, D>(bh_ptr(args.dq, args.ldq, t.b, t.h), vol_off(args.ldq, ln.pos), grp, acc,
+                         kScaled<T, TWO> ? p.scale * inv_pow2(gs) : p.scale);
     if (redo)
         band_redo_bwd_q<T, D>(kernargs(), t.b, t.h, hk, opaque(ln.pos[0]), opaque(ln.pos[1]), opaque(ln.pos[2]), grp);
 }
@@ -608,9 +668,13 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
     f32x4_t gk[D / 16], gv[D / 16];
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) gk[db] = gv[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float gs = scale_for(0.f);  // scaled: the factor of P' dP' = 2^15 dS
     const auto store = [&]() {
-        store_rows<T, D>(bh_ptr(args.dk, args.ldk, t.b, t.h), vol_off(args.ldk, ln.pos), grp, gk, p.scale);
-        store_rows<T, D>(bh_ptr(args.dv, args.ldv, t.b, t.h), vol_off(args.ldv, ln.pos), grp, gv, 1.f);
+        constexpr bool S = kScaled<T, TWO>;
+        store_rows<T, D>(bh_ptr(args.dk, args.ldk, t.b, t.h), vol_off(args.ldk, ln.pos), grp, gk,
+                         S ? p.scale * (1.f / kScaleP) * inv_pow2(gs) : p.scale);
+        store_rows<T, D>(bh_ptr(args.dv, args.ldv, t.b, t.h), vol_off(args.ldv, ln.pos), grp, gv,
+                         S ? 1.f / kScaleP : 1.f);
     };
     if (U0 == 0 || U1 == 0 || U2 == 0) {  // no query attends these keys
         if (ln.valid) store();
@@ -694,8 +758,23 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         s[bb][i] = __builtin_amdgcn_exp2f(fmaf(s[bb][i], sc2, nl[bb][i]));
+                        if constexpr (kScaled<T, TWO>) s[bb][i] *= kScaleP;
                         dp[bb][i] *= s[bb][i];
                     }
+                if constexpr (kScaled<T, TWO>) {
+                    // a new maximum past the limit lowers the item's factor (and what
+                    // it has gathered), as the forward's online softmax does
+                    const float mx = abs_max8(dp, 0.f);
+                    if (__any(mx * gs >= kScaleLimit)) {
+                        const float m = max_rows_num(mx), ng = m * gs >= kScaleLimit ? scale_for(m) : gs;
+                        const float corr = ng * inv_pow2(gs);
+                        gs = ng;
+#pragma unroll
+                        for (int db = 0; db < D / 16; ++db) gk[db] *= corr;
+                    }
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) dp[i >> 2][i & 3] *= gs;
+                }
                 band_accumulate<T, D, TWO>(Gb, off, c, s, gv);
                 band_accumulate<T, D, TWO>(Qb, off, c, dp, gk);
             }
@@ -886,8 +965,8 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
 // Where the general tiles cannot hold the problem either, the alternative is
 // the vector kernels, whose probabilities and their gradients stay in fp32:
 // there they enter the matrix products as two 16-bit terms (TWO; the rest
-// after rounding is the second), which keeps 16 (fp16: 22) of their bits.  The
-// callers ask for it (`two`).
+// after rounding is the second), which keeps 16 (fp16, scaled: 22) of their
+// bits, and the row sums stay in fp32.  The callers ask for it (`two`).
 // `lays`: every 16-bit operand and fp32 row operand of the call.  The answer
 // depends on the problem alone, never on which tables exist.
 int band_sides(const Prob& p, int dtype, bool aligned, bool lean, std::initializer_list<Lay> lays) {

@@ -140,6 +140,34 @@ def test_two_term_products_add_no_error(case, dtype):
         assert err <= 1.03 * float((b.to(dtype).double() - b).norm()), (name, err)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("scales", [(1e-2, 1), (1e-3, 1), (1e-4, 1), (1e-3, 4), (100, 1)])  # of dO and k
+@pytest.mark.parametrize("case", [TWO_TERM_CASES[2], TWO_TERM_CASES[4], ((200, 19), 32, (97, 16))])
+def test_two_term_products_keep_small_gradients(case, scales, dtype):
+    """The bound of test_two_term_products_add_no_error where dS or P leaves
+    the range in which two unscaled fp16 terms hold it: a mean-reduced loss's
+    gradients, and windows of hundreds of keys.  (The forward takes two terms
+    in these cases: a one-term forward's log-sum-exp adds 4 % at 4 k.)"""
+    from natten_mps_amd import functional as F
+
+    sp, dim, ks = case
+    print(case, scales, dtype, flush=True)
+    q, k, v, do = _inputs(35, [(1, *sp, 2, dim)] * 4, torch.float32)
+    ts = [t.to(dtype) for t in (q, k * scales[1], v, do * scales[0])]
+    leaves = [t.to(DEV).requires_grad_(True) for t in ts[:3]]
+    out = F.na2d(*leaves, kernel_size=ks)
+    grads = torch.autograd.grad(out, leaves, ts[3].to(DEV))
+    one, no = (1, 1), (False, False)
+    q, k, v = (t.double().requires_grad_(True) for t in ts[:3])
+    logits = P.na2d_qk_forward(q, k, ks, one, one, no, dim ** -0.5)
+    ref = P.na2d_av_forward(torch.softmax(logits, dim=-1), v, ks, one, one, no)
+    rgrads = torch.autograd.grad(ref, (q, k, v), ts[3].double())
+    for name, a, b in zip(("dq", "dk", "dv"), grads, rgrads):
+        b = b.detach()
+        err = float((a.cpu().double() - b).norm())
+        assert err <= 1.03 * float((b.to(dtype).double() - b).norm()), (name, err)
+
+
 @pytest.mark.parametrize("tokens", [1, 7])
 @pytest.mark.parametrize("ks", [(9, 9), (7, 7)])  # key side on the band and on the lean tiles
 def test_window_key_side_under_global_keys(ks, tokens):
