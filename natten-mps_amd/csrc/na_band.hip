@@ -852,12 +852,11 @@ bool band_static_lds_ok() {
     return ok;
 }
 
-bool band_switch() {
-    static const bool on = [] {
-        const char* e = std::getenv("NATTEN_HIP_BAND");
-        return !(e && std::strcmp(e, "0") == 0);
-    }();
-    return on;
+// NATTEN_HIP_BAND: 0 keeps every call off these kernels, 1 puts every call
+// that they can serve on them (tuning, tests); else band_pays decides.
+int band_forced() {
+    const char* e = std::getenv("NATTEN_HIP_BAND");
+    return !e ? -1 : std::strcmp(e, "0") == 0 ? 0 : std::strcmp(e, "1") == 0 ? 1 : -1;
 }
 
 template <typename T, int D>
@@ -962,6 +961,7 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
 //   tile's union does not fit them (`lean`: they take the problem; 9 x 9, 8 x
 //   64 x 64 x 8: dK/dV 222 -> 56 us at head dim 32, 613 -> 111 at 64; 7 x 7
 //   on 32 x 22 x 22 x 8: 57 -> 37).
+// Where the general tiles hold the problem too, band_pays decides per kernel.
 // Where the general tiles cannot hold the problem either, the alternative is
 // the vector kernels, whose probabilities and their gradients stay in fp32:
 // there they enter the matrix products as two 16-bit terms (TWO; the rest
@@ -970,7 +970,7 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
 // `lays`: every 16-bit operand and fp32 row operand of the call.  The answer
 // depends on the problem alone, never on which tables exist.
 int band_sides(const Prob& p, int dtype, bool aligned, bool lean, std::initializer_list<Lay> lays) {
-    if (!band_switch() || !aligned || dtype == NATTEN_F32 || !(p.scale > 0.f)) return 0;
+    if (!aligned || dtype == NATTEN_F32 || !(p.scale > 0.f)) return 0;
     if (p.Dqk != p.Dv || (p.Dqk != 32 && p.Dqk != 64 && p.Dqk != 128)) return 0;
     if (p.ax[0].len != 1 || p.ax[0].k != 1) return 0;
     for (int a = 0; a < 3; ++a)
@@ -985,8 +985,39 @@ int band_sides(const Prob& p, int dtype, bool aligned, bool lean, std::initializ
         if (band_plane(p, l, p.Dqk) >= kBandOOR) return 0;
     const long long tiles = ((static_cast<long long>(p.ax[1].len) + 7) / 8 + p.ax[1].dil) *
                             ((static_cast<long long>(p.ax[2].len) + 7) / 8 + p.ax[2].dil);
-    if (tiles * p.B * p.Hq >= (1LL << 31) || !band_static_lds_ok()) return 0;
+    if (tiles * p.B * p.Hq >= (1LL << 31) || !band_static_lds_ok() || band_forced() == 0) return 0;
     return both ? kQuerySide | kKeySide : kKeySide;
+}
+
+// A workgroup here owns 128 items and walks rows of 32 slots, 16 of them idle
+// where a class is that narrow, so small grids, short windows and small
+// classes are faster on the general tiles.  The line, over 4080 timed pairs (a
+// kernel each; 16 x 16 to 128 x 128 at dilation 1 to 4, windows of 3 x 8 to
+// 16 x 16, 1 to 256 heads in all, bf16):
+// * the general tiles stage enough in all: below 300 / 150 / 130 thousand slots
+//   (head dim 32 / 64 / 128) both are bound by one workgroup's latency, which
+//   is longer here (one 64 x 64 image, 1 head, dim 64, 13 x 13 under dilation
+//   4: forward 6.8 against 11.1 us, backward 16 against 35);
+// * their tile is past 64 KB of LDS (one workgroup per CU, nothing overlaps)
+//   and they stage more slots than these kernels, or at dim 128 about as many
+//   (forward, 256 heads of 20 x 20, 9 x 9: 100 against 58 us at 0.94 of the
+//   slots), but not dQ, whose registers leave one workgroup per CU here too;
+// * or it has fallen to 32 items or fewer and they stage 1.5 times the slots
+//   (backward: 2.1 times).
+// Over those pairs the choice is within 0.9 % of the faster kernel's time on
+// average (kernel by kernel), and above the general tiles' by more than 5 %
+// in 8 of them (at most 23 %).
+bool band_pays(const Prob& p, FusedKernel kernel, const TileLoad& general) {
+    if (band_forced() == 1) return true;
+    const bool key = kernel == kFusedKey;
+    if (general.slots <= (p.Dqk == 32 ? 300000 : p.Dqk == 64 ? 150000 : 130000)) return false;
+    const BandGeo g = band_geo(p, band_columns(p.ax[2].k, key), key ? p.Hkv : p.Hq);
+    const long long slots = band_blocks(p, g) * 32 * union_extent(p.ax[1], 1 << g.sh1, key) * (key ? p.rep : 1);
+    if (general.lds > 64 * 1024) {
+        const bool wide = p.Dqk == 128 && kernel != kFusedQuery;
+        return 20 * general.slots > (wide ? 17 : 22) * slots;
+    }
+    return general.items <= 32 && 10 * general.slots > (kernel == kFusedForward ? 15 : 21) * slots;
 }
 
 hipError_t band_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,

@@ -186,11 +186,14 @@ int natten_hip_forward(const natten_problem_t* p, const void* q, const natten_la
                                               to_lay(llse), p->dtype, s);
         if (e != hipErrorNotSupported) return launch_status(e, "forward");
     }
-    const bool mfma = use_mfma() && na::mfma_eligible(P, p->dtype, D, vec != 0, false) &&
+    na::TileLoad general[3];
+    const bool mfma = use_mfma() && na::mfma_eligible(P, p->dtype, D, vec != 0, false, false, general) &&
                       na::mfma_offsets_fit(P, {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)});
-    if (use_mfma() && (na::band_sides(P, p->dtype, vec != 0, false,
-                                      {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)}) &
-                       na::kQuerySide))
+    if (use_mfma() &&
+        (na::band_sides(P, p->dtype, vec != 0, false,
+                        {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(llse)}) &
+         na::kQuerySide) &&
+        (!mfma || na::band_pays(P, na::kFusedForward, general[na::kFusedForward])))
         return launch_status(na::band_forward(P, q, to_lay(lq), k, to_lay(lk), v, to_lay(lv), out, to_lay(lo), lse,
                                               to_lay(llse), p->dtype, s, !mfma),
                              "forward");
@@ -233,10 +236,18 @@ struct BackwardCall {
                                            {lq, lk, lv, lo, ldo, ll, ldq, ldk, ldv, lde, dlse ? ldl : ll})
                           : 0;
     }
-    bool mfma_ok(int sides) const {
-        return use_mfma() && na::mfma_eligible(P, dtype, P.Dqk > P.Dv ? P.Dqk : P.Dv, vec != 0, true, false, sides) &&
+    bool mfma_ok(na::TileLoad* loads) const {
+        return use_mfma() &&
+               na::mfma_eligible(P, dtype, P.Dqk > P.Dv ? P.Dqk : P.Dv, vec != 0, true, false, loads) &&
                na::mfma_offsets_fit(P, {lq, lk, lv, lo, ldo, ll, ldq, ldk, ldv, lde}) &&
                (!dlse || na::mfma_offsets_fit(P, {ldl}));
+    }
+    // the sides of `band` on which the band kernels beat the general tiles
+    int band_gains(int band, const na::TileLoad* general) const {
+        if ((band & na::kQuerySide) && !na::band_pays(P, na::kFusedQuery, general[na::kFusedQuery]))
+            band &= ~na::kQuerySide;
+        if ((band & na::kKeySide) && !na::band_pays(P, na::kFusedKey, general[na::kFusedKey])) band &= ~na::kKeySide;
+        return band;
     }
     hipError_t lean(int sides) const {
         return na::lean_backward(P, q, lq, k, lk, v, lv, o, lo, dout, ldo, lse, ll, dlse, ldl, dq, ldq, dk, ldk, dv,
@@ -274,24 +285,27 @@ int backward_impl(const natten_problem_t* p, const na::Prob& P, const void* q, c
     const BackwardCall c{P, p->dtype, vec, q, k, v, out, dout, to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo),
                          to_lay(ldo), lse, to_lay(llse), dlse, to_lay(ldlse), dq, dk, dv, to_lay(ldq), to_lay(ldk),
                          to_lay(ldv), delta, to_lay(ldelta), static_cast<hipStream_t>(stream)};
-    // the lean tiles first, the band kernels for what their unions cannot
-    // hold, then the general tiles
+    // the lean tiles first; for what their unions cannot hold each side on
+    // the band kernels or the general tiles, whichever is the faster
     const bool lean = c.lean_ok();
-    const int band = c.band_sides(lean);
-    if (band) {
-        const bool two = !c.mfma_ok(kBothSides);
-        if (two || band == kBothSides) return launch_status(c.band(kBothSides, two), "backward");
-        // the query side as without the band kernels (the general tiles give
-        // the lean ones' bits where no table of those exists)
-        hipError_t e = c.lean(na::kQuerySide);
+    if (const int can = c.band_sides(lean)) {
+        na::TileLoad general[3];
+        if (!c.mfma_ok(general)) return launch_status(c.band(kBothSides, true), "backward");
+        const int band = c.band_gains(can, general);
+        if (band == kBothSides) return launch_status(c.band(kBothSides, false), "backward");
+        hipError_t e = hipErrorNotSupported;
+        // (the general tiles give the lean ones' bits where no table of those exists)
+        if (band & na::kQuerySide) e = c.band(na::kQuerySide, false);
+        else if (lean) e = c.lean(na::kQuerySide);
         if (e == hipErrorNotSupported) e = c.mfma(na::kQuerySide);
-        return launch_status(e == hipSuccess ? c.band(na::kKeySide, false) : e, "backward");
+        if (e == hipSuccess) e = band & na::kKeySide ? c.band(na::kKeySide, false) : c.mfma(na::kKeySide);
+        return launch_status(e, "backward");
     }
     if (lean) {
         const hipError_t e = c.lean(kBothSides);
         if (e != hipErrorNotSupported) return launch_status(e, "backward");
     }
-    if (c.mfma_ok(kBothSides)) return launch_status(c.mfma(kBothSides), "backward");
+    if (c.mfma_ok(nullptr)) return launch_status(c.mfma(kBothSides), "backward");
     return launch_status(
         na::generic_backward(P, vec, q, c.lq, k, c.lk, v, c.lv, out, c.lo, dout, c.ldo, lse, c.ll, dlse, c.ldl, dq,
                              c.ldq, dk, c.ldk, dv, c.ldv, delta, c.lde, p->dtype, c.s),
@@ -395,9 +409,10 @@ int make_global(const na::Prob& P, const void* gk, const natten_layout_t* lgk, c
 }
 
 // The global-key path: the MFMA tile kernels with global-key chunks.
-bool global_eligible(const na::Prob& P, int dtype, int vec, const na::GlobalSet& g, bool backward) {
+bool global_eligible(const na::Prob& P, int dtype, int vec, const na::GlobalSet& g, bool backward,
+                     na::TileLoad* loads = nullptr) {
     const int D = P.Dqk > P.Dv ? P.Dqk : P.Dv;
-    return use_mfma() && na::mfma_eligible(P, dtype, D, vec != 0, backward, true) &&
+    return use_mfma() && na::mfma_eligible(P, dtype, D, vec != 0, backward, true, loads) &&
            na::mfma_global_key_ok(P, dtype, g);
 }
 
@@ -476,7 +491,8 @@ int natten_hip_backward_global(const natten_problem_t* p, const void* q, const n
                         : 0;
     // every check of both launches before the first: an unsupported problem
     // is rejected with no output written
-    if (!global_eligible(P, p->dtype, vec, g, true) ||
+    na::TileLoad general[3];
+    if (!global_eligible(P, p->dtype, vec, g, true, general) ||
         !na::mfma_offsets_fit(P, {to_lay(lq), to_lay(lk), to_lay(lv), to_lay(lo), to_lay(ldo), to_lay(llse),
                                   to_lay(ldq), to_lay(ldk), to_lay(ldv), to_lay(ldelta)}) ||
         (dlse && !na::mfma_offsets_fit(P, {to_lay(ldlse)})) || !na::mfma_global_batch_fit(P, to_lay(lq), to_lay(ldo)))
@@ -492,8 +508,8 @@ int natten_hip_backward_global(const natten_problem_t* p, const void* q, const n
     hipError_t e = c.mfma(na::kQuerySide, &g);
     if (e == hipSuccess) {
         const bool lean = c.lean_ok();
-        if (c.band_sides(lean) & na::kKeySide) {
-            e = c.band(na::kKeySide, false);
+        if (const int can = c.band_sides(lean) & na::kKeySide) {
+            e = c.band_gains(can, general) ? c.band(na::kKeySide, false) : c.mfma(na::kKeySide);
         } else {
             e = lean ? c.lean(na::kKeySide) : hipErrorNotSupported;
             if (e == hipErrorNotSupported) e = c.mfma(na::kKeySide);

@@ -110,10 +110,18 @@ struct GlobalSet {
 // number of instances whose attributes were read.
 bool mfma_static_lds_ok();
 int mfma_lds_audit(int* checked);
-// `global`: with global keys (their LDS on top of the tiles'); `sides`: of
-// the backward.
+// What a fused kernel's tiles come to: items and LDS bytes of one, and the
+// slots that all of them stage (the key side: for every q head of a group).
+struct TileLoad {
+    int items;
+    size_t lds;
+    long long slots;
+};
+enum FusedKernel { kFusedForward = 0, kFusedQuery = 1, kFusedKey = 2 };
+// `global`: with global keys (their LDS on top of the tiles').  loads, if
+// given: of the kernels (FusedKernel) asked about.
 bool mfma_eligible(const Prob& p, int dtype, int D, bool aligned, bool backward, bool global = false,
-                   int sides = kQuerySide | kKeySide);
+                   TileLoad* loads = nullptr);
 bool mfma_offsets_fit(const Prob& p, std::initializer_list<Lay> lays);
 
 // Variable-length fused forward / backward on the MFMA tile kernels: the
@@ -166,6 +174,9 @@ bool lean_key_tiles_fit(const Prob& p);
 // run on them; no tables, so each has a launch in every call.  `lean`: the
 // 8x8 tile kernels take the problem's query side.
 int band_sides(const Prob& p, int dtype, bool aligned, bool lean, std::initializer_list<Lay> lays);
+// A kernel that both the band kernels and the general tiles (of this load)
+// serve is faster on the former.
+bool band_pays(const Prob& p, FusedKernel kernel, const TileLoad& general);
 hipError_t band_forward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv, void* o,
                         Lay lo, float* lse, Lay ll, int dtype, hipStream_t s, bool two);
 hipError_t band_backward(const Prob& p, const void* q, Lay lq, const void* k, Lay lk, const void* v, Lay lv,

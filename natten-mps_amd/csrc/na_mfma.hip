@@ -2216,24 +2216,25 @@ static Lay item_lay(const Prob& p, Lay l) {
     return l;
 }
 
-bool mfma_eligible(const Prob& p, int dtype, int D, bool aligned, bool backward, bool global, int sides) {
+bool mfma_eligible(const Prob& p, int dtype, int D, bool aligned, bool backward, bool global, TileLoad* loads) {
     if (dtype == NATTEN_F32 || !aligned || !(p.scale > 0.f) || !mfma_static_lds_ok()) return false;
     if (p.Dqk != p.Dv || !(D == 32 || D == 64 || D == 96 || D == 128)) return false;
     // a strided axis must be one residue class (its query items then sit at
     // class coordinates stride * t); global keys come at stride 1 only
     for (int a = 0; a < 3; ++a)
         if (p.ax[a].st != 1 && (p.ax[a].dil != 1 || global)) return false;
-    // tile indices (the launch grid) stay in 31 bits
     const size_t extra = global ? global_lds(D) : 0;
-    TileShape ts{};
-    if (!choose_tile(p, kForward, D, ts, extra) || grid_blocks(p, ts) >= (1LL << 31)) return false;
-    if (backward) {
-        if ((sides & kQuerySide) && (!choose_tile(p, kBackwardQ, D, ts, extra) || grid_blocks(p, ts) >= (1LL << 31)))
-            return false;
-        if ((sides & kKeySide) && (!choose_tile(p, kBackwardKV, D, ts) || grid_blocks(p, ts) >= (1LL << 31)))
-            return false;
-    }
-    return true;
+    const auto holds = [&](Kind kind, FusedKernel f, size_t more) {
+        TileShape ts{};
+        // tile indices (the launch grid) stay in 31 bits
+        if (!choose_tile(p, kind, D, ts, more) || grid_blocks(p, ts) >= (1LL << 31)) return false;
+        if (loads)
+            loads[f] = {ts.T[0] * ts.T[1] * ts.T[2], lds_bytes(kind, ts.slots, D),
+                        grid_blocks(p, ts) * ts.slots * (f == kFusedKey ? p.rep : 1)};
+        return true;
+    };
+    return holds(kForward, kFusedForward, extra) &&
+           (!backward || (holds(kBackwardQ, kFusedQuery, extra) && holds(kBackwardKV, kFusedKey, 0)));
 }
 
 bool mfma_offsets_fit(const Prob& p, std::initializer_list<Lay> lays) { return offsets_fit(p, lays); }

@@ -14,10 +14,12 @@ DEV = torch.device("cuda:0")
 
 
 @pytest.fixture(autouse=True)
-def _hip():
+def _hip(monkeypatch):
     import natten_mps_amd
 
     natten_mps_amd.set_backend("hip")
+    # small grids run on the general tiles where those hold the problem
+    monkeypatch.setenv("NATTEN_HIP_BAND", "1")
     yield
 
 
@@ -212,3 +214,52 @@ def test_band_kernels_recompute_non_finite_operands():
         assert torch.equal(torch.isfinite(a), torch.isfinite(b)), name
         fin = torch.isfinite(b)
         assert_parity(a[fin], b[fin], torch.bfloat16, name)
+
+
+# batch, spatial, heads, dim, kernel, dilation, and which of the forward, dQ
+# and dK/dV run on the band kernels by themselves
+ROUTE_CASES = [
+    (1, (20, 20), 1, 64, (3, 13), (1, 1), ""),          # a few workgroups
+    (4, (56, 56), 8, 64, (11, 11), (4, 4), ""),         # classes of 14: 64-query tiles in 64 KB
+    (4, (128, 128), 8, 64, (3, 13), (1, 1), "fq"),      # 32-query tiles
+    (8, (64, 64), 8, 32, (9, 9), (1, 1), "k"),          # key tiles of 16
+    (4, (64, 64), 8, 64, (8, 8), (1, 1), "k"),          # key tiles past 64 KB
+    (1, (64, 64), 1, 64, (9, 9), (1, 1), ""),           # the same, one image of one head
+    (2, (64, 64), 4, 64, (5, 11), (1, 1), "fqk"),       # past 64 KB, or 16-query tiles
+    (8, (28, 28), 8, 128, (8, 8), (2, 2), "fk"),        # dQ: its registers leave one workgroup per CU
+]
+
+
+@pytest.mark.parametrize("case", ROUTE_CASES)
+def test_each_side_takes_the_faster_kernels(case, monkeypatch):
+    """The route that the sizes give, and both routes' results beside each
+    other (bfloat16, probabilities rounded once on either)."""
+    from natten_mps_amd import functional as F
+    from natten_mps_amd._core import _lib
+
+    B, sp, heads, dim, ks, dil, want = case
+    print(case, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(41)
+    ts = [torch.randn(B, *sp, heads, dim, generator=g, device=DEV).bfloat16() for _ in range(4)]
+    leaves = [t.requires_grad_(True) for t in ts[:3]]
+
+    def run():
+        _lib.profile_read(reset=True)
+        _lib.profile_enable(True)
+        try:
+            out = F.na2d(*leaves, kernel_size=ks, dilation=dil)
+            res = (out.detach(), *torch.autograd.grad(out, leaves, ts[3]))
+            torch.cuda.synchronize()
+        finally:
+            _lib.profile_enable(False)
+        names = {"na_fwd_band": "f", "na_bwd_q_band": "q", "na_bwd_kv_band": "k"}
+        launched = _lib.profile_read(reset=True)
+        return res, "".join(v for n, v in names.items() if n in launched)
+
+    monkeypatch.setenv("NATTEN_HIP_BAND", "0")
+    general, none = run()
+    monkeypatch.delenv("NATTEN_HIP_BAND")
+    chosen, got = run()
+    assert none == "" and got == want, (none, got)
+    for name, a, b in zip(("out", "dq", "dk", "dv"), chosen, general):
+        assert_parity(a.cpu(), b.cpu().float(), torch.bfloat16, name)
