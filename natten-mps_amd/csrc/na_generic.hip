@@ -191,11 +191,17 @@ struct Run {
 // queries) waits on each step's loads; with `walk_*_pipelined` the loads of
 // the next U steps are already in flight.  `fetch` issues a step's loads and
 // returns the raw registers (no use of the loaded values, so no wait), `use`
-// consumes them, in the same order as the plain walk.  Only for 16-byte
-// aligned runs (`vec`); masked (causal) neighbours load from a clamped position
-// and are skipped by `use`.  fetch(j0, j1, j2, e) gets the neighbour's
-// position and index, use(step, e, valid, u) its registers (u: step within
-// its block of U).
+// consumes them, in the same order as the plain walk.  fetch(offsets, e) gets
+// the neighbour's offsets in the walk's operands and its index, use(step, e,
+// valid, u) its registers (u: step within its block of U); masked (causal)
+// neighbours load from a clamped position and are skipped by `use`.  Only for
+// 16-byte aligned runs and, on the key side, strides of 1 (`VEC` where a kernel
+// has an instance of its own for them: their registers would take up to half
+// of the waves from the plain walk's callers).  dK/dV, bfloat16, 8 x 8 heads,
+// us, one kernel for both walks -> two: 12 x 24 x 24, 3 x 3 x 3, dim 20 1011 ->
+// 610; 96 x 96, 3 x 3, stride 2, dim 72 762 -> 463; QK of 130 x 150, 5 x 5, dim
+// 44, 2 heads 59 -> 40.  (Forward, AV and dQ keep one: apart they were level,
+// or slower for more waves on the same L1.)
 // ---------------------------------------------------------------------------
 // Steps in flight: about 8 runs of 16 bytes per lane.
 template <typename T, int DPL, int RUNS>
@@ -355,7 +361,14 @@ __device__ __forceinline__ void walk_queries_pipelined(const Prob& p, int b, int
     }
 }
 
-__device__ __forceinline__ bool unit_strides(const Prob& p) {
+// Instances whose registers sit just past a step of the waves per SIMD (head
+// dims above 128) are built for the waves below it.
+template <typename T, int DPL>
+constexpr bool kWide16 = DPL == 16 && sizeof(T) == 2;
+template <typename T, int DPL>
+constexpr bool kWide32 = DPL == 16 && sizeof(T) == 4;
+
+__host__ __device__ inline bool unit_strides(const Prob& p) {
     return p.ax[0].st == 1 && p.ax[1].st == 1 && p.ax[2].st == 1;
 }
 
@@ -363,7 +376,7 @@ __device__ __forceinline__ bool unit_strides(const Prob& p) {
 // Fused forward with online softmax.
 // ---------------------------------------------------------------------------
 template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_forward(Prob p, int vec, int split, const int* __restrict__ lens,
+__global__ __launch_bounds__(256, (kWide16<T, DPL> ? 4 : 1)) void k_forward(Prob p, int vec, int split, const int* __restrict__ lens,
                                                  const T* __restrict__ q, Lay lq,
                                                  const T* __restrict__ k, Lay lk,
                                                  const T* __restrict__ v, Lay lv,
@@ -467,21 +480,22 @@ struct RowPut {
 // ---------------------------------------------------------------------------
 // Split QK: logits per neighbour (unscaled unless has_scale), -inf if invalid.
 // ---------------------------------------------------------------------------
-template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_qk(Prob p, int vec, int split,
+template <typename T, int DPL, int LPQ, bool VEC>
+__global__ __launch_bounds__(256) void k_qk(Prob p, int split,
                                             const T* __restrict__ q, Lay lq,
                                             const T* __restrict__ k, Lay lk,
                                             T* __restrict__ attn, Lay la) {
     const long long qi = group_index(LPQ * split);
     if (qi >= static_cast<long long>(p.B) * p.nout * p.Hq) return;
     using R = Run<T, DPL, LPQ>;
+    constexpr int vec = VEC;
     const int ln = threadIdx.x % LPQ;
     const int sp = (threadIdx.x / LPQ) % split;
     const QPos Q = decode_query(p, qi);
     float qv[DPL];
     R::load(q + lq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), ln, p.Dqk, vec, qv);
     T* row = attn + la.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h);
-    if (vec) {
+    if constexpr (VEC) {
         RowPut<T, LPQ, pipe_depth<T, DPL, 1>()> put{row};
         walk_neighbors_pipelined<pipe_depth<T, DPL, 1>(), 1>(
             p, Q.b, Q.h, Q.i0, Q.i1, Q.i2, sp, split, {lk},
@@ -530,7 +544,7 @@ __device__ __forceinline__ A gather_fma(float a, float b, A acc) {
     return static_cast<A>(a) * static_cast<A>(b) + acc;
 }
 
-// The groups' sum of acc (times mul) rounded to float for store_run.
+// The groups' sum of acc (times mul) rounded to float.
 template <int LPQ, typename A, int DPL>
 __device__ __forceinline__ void gather_out(const A (&acc)[DPL], int split, float mul, float (&out)[DPL]) {
 #pragma unroll
@@ -599,7 +613,7 @@ __global__ __launch_bounds__(256) void k_av(Prob p, int vec, int split,
 // dq = scale * sum_k P (dO.v_k - delta) k_k with P = exp(scale q.k - lse).
 // ---------------------------------------------------------------------------
 template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_bwd_dq(Prob p, int vec, int split, const int* __restrict__ lens,
+__global__ __launch_bounds__(256, (kWide32<T, DPL> ? 3 : 1)) void k_bwd_dq(Prob p, int vec, int split, const int* __restrict__ lens,
                                                 const T* __restrict__ q, Lay lq,
                                                 const T* __restrict__ k, Lay lk,
                                                 const T* __restrict__ v, Lay lv,
@@ -696,8 +710,8 @@ __global__ __launch_bounds__(256) void k_bwd_dq(Prob p, int vec, int split, cons
 // dv = sum P dO,  dk = scale * sum P (dO.v - delta) q.  Deterministic (no
 // atomics); recomputes P from q, k and lse.
 // ---------------------------------------------------------------------------
-template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_bwd_dkdv(Prob p, int vec, int split, const int* __restrict__ lens,
+template <typename T, int DPL, int LPQ, bool VEC>
+__global__ __launch_bounds__(256, (kWide32<T, DPL> ? 2 : 1)) void k_bwd_dkdv(Prob p, int aligned, int split, const int* __restrict__ lens,
                                                   const T* __restrict__ q, Lay lq,
                                                   const T* __restrict__ k, Lay lk,
                                                   const T* __restrict__ v, Lay lv,
@@ -709,6 +723,7 @@ __global__ __launch_bounds__(256) void k_bwd_dkdv(Prob p, int vec, int split, co
     const long long ki = group_index(LPQ * split);
     if (ki >= static_cast<long long>(p.B) * p.nkey * p.Hkv) return;
     using R = Run<T, DPL, LPQ>;
+    const int vec = VEC ? 1 : aligned;
     const int ln = threadIdx.x % LPQ;
     const int sp = (threadIdx.x / LPQ) % split;
     const KPos K = decode_key(p, ki, p.Hkv);
@@ -735,7 +750,7 @@ __global__ __launch_bounds__(256) void k_bwd_dkdv(Prob p, int vec, int split, co
             gk[j] = fmaf(ds, qv[j], gk[j]);
         }
     };
-    if (vec && unit_strides(p)) {
+    if constexpr (VEC) {
         struct Step {
             typename R::Raw q, g;
             float L, di;
@@ -828,14 +843,15 @@ __global__ __launch_bounds__(256) void k_qk_bwd_q(Prob p, int vec, int split,
     if (sp == 0) R::store(dq + ldq.at(Q.b, Q.i0, Q.i1, Q.i2, Q.h), ln, p.Dqk, vec, res);
 }
 
-template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_qk_bwd_k(Prob p, int vec, int split,
+template <typename T, int DPL, int LPQ, bool VEC>
+__global__ __launch_bounds__(256) void k_qk_bwd_k(Prob p, int aligned, int split,
                                                   const T* __restrict__ da, Lay lda,
                                                   const T* __restrict__ q, Lay lq,
                                                   T* __restrict__ dk, Lay ldk) {
     const long long ki = group_index(LPQ * split);
     if (ki >= static_cast<long long>(p.B) * p.nkey * p.Hkv) return;
     using R = Run<T, DPL, LPQ>;
+    const int vec = VEC ? 1 : aligned;
     const int ln = threadIdx.x % LPQ;
     const int sp = (threadIdx.x / LPQ) % split;
     const KPos K = decode_key(p, ki, p.Hkv);
@@ -843,7 +859,7 @@ __global__ __launch_bounds__(256) void k_qk_bwd_k(Prob p, int vec, int split,
     A acc[DPL];
 #pragma unroll
     for (int j = 0; j < DPL; ++j) acc[j] = 0;
-    if (vec && unit_strides(p)) {
+    if constexpr (VEC) {
         struct Step {
             typename R::Raw x;
             T w;
@@ -877,21 +893,22 @@ __global__ __launch_bounds__(256) void k_qk_bwd_k(Prob p, int vec, int split,
 // ---------------------------------------------------------------------------
 // Split AV backward: dattn (query side) and dv (key side).
 // ---------------------------------------------------------------------------
-template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_av_bwd_a(Prob p, int vec, int split,
+template <typename T, int DPL, int LPQ, bool VEC>
+__global__ __launch_bounds__(256) void k_av_bwd_a(Prob p, int split,
                                                   const T* __restrict__ dout, Lay ldo,
                                                   const T* __restrict__ v, Lay lv,
                                                   T* __restrict__ da, Lay lda) {
     const long long qi = group_index(LPQ * split);
     if (qi >= static_cast<long long>(p.B) * p.nout * p.Hq) return;
     using R = Run<T, DPL, LPQ>;
+    constexpr int vec = VEC;
     const int ln = threadIdx.x % LPQ;
     const int sp = (threadIdx.x / LPQ) % split;
     const QPos Q = decode_query(p, qi);
     float dov[DPL];
     R::load(dout + ldo.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h), ln, p.Dv, vec, dov);
     T* row = da + lda.at(Q.b, Q.o0, Q.o1, Q.o2, Q.h);
-    if (vec) {
+    if constexpr (VEC) {
         RowPut<T, LPQ, pipe_depth<T, DPL, 1>()> put{row};
         walk_neighbors_pipelined<pipe_depth<T, DPL, 1>(), 1>(
             p, Q.b, Q.h, Q.i0, Q.i1, Q.i2, sp, split, {lv},
@@ -918,14 +935,15 @@ __global__ __launch_bounds__(256) void k_av_bwd_a(Prob p, int vec, int split,
     });
 }
 
-template <typename T, int DPL, int LPQ>
-__global__ __launch_bounds__(256) void k_av_bwd_v(Prob p, int vec, int split,
+template <typename T, int DPL, int LPQ, bool VEC>
+__global__ __launch_bounds__(256) void k_av_bwd_v(Prob p, int aligned, int split,
                                                   const T* __restrict__ dout, Lay ldo,
                                                   const T* __restrict__ attn, Lay la,
                                                   T* __restrict__ dv, Lay ldv) {
     const long long ki = group_index(LPQ * split);
     if (ki >= static_cast<long long>(p.B) * p.nkey * p.Hkv) return;
     using R = Run<T, DPL, LPQ>;
+    const int vec = VEC ? 1 : aligned;
     const int ln = threadIdx.x % LPQ;
     const int sp = (threadIdx.x / LPQ) % split;
     const KPos K = decode_key(p, ki, p.Hkv);
@@ -933,7 +951,7 @@ __global__ __launch_bounds__(256) void k_av_bwd_v(Prob p, int vec, int split,
     A acc[DPL];
 #pragma unroll
     for (int j = 0; j < DPL; ++j) acc[j] = 0;
-    if (vec && unit_strides(p)) {
+    if constexpr (VEC) {
         struct Step {
             typename R::Raw x;
             T w;
@@ -1074,7 +1092,8 @@ struct LQK {
                           hipStream_t s) {
         const long long n = static_cast<long long>(p.B) * p.nout * p.Hq;
         const int split = choose_split(p, n, LPQ);
-        NA_LAUNCH("na_qk", (k_qk<T, DPL, LPQ>), dim3(grid_for(n, LPQ * split)), dim3(256), 0, s, p, vec, split, (const T*)q, lq,
+        const auto kern = vec ? k_qk<T, DPL, LPQ, true> : k_qk<T, DPL, LPQ, false>;
+        NA_LAUNCH("na_qk", kern, dim3(grid_for(n, LPQ * split)), dim3(256), 0, s, p, split, (const T*)q, lq,
                            (const T*)k, lk, (T*)a, la);
         return hipGetLastError();
     }
@@ -1107,7 +1126,8 @@ struct LBackward {
         if (e != hipSuccess) return e;
         const long long nk = static_cast<long long>(p.B) * p.nkey * p.Hkv;
         const int sk = choose_split(p, nk, LPQ);
-        NA_LAUNCH(lens ? "na_varlen_bwd_dkdv" : "na_bwd_dkdv", (k_bwd_dkdv<T, DPL, LPQ>),
+        const auto kern_k = vec && unit_strides(p) ? k_bwd_dkdv<T, DPL, LPQ, true> : k_bwd_dkdv<T, DPL, LPQ, false>;
+        NA_LAUNCH(lens ? "na_varlen_bwd_dkdv" : "na_bwd_dkdv", kern_k,
                   dim3(grid_for(nk, LPQ * sk)), dim3(256), 0, s, p, vec, sk, lens, (const T*)q, lq, (const T*)k, lk,
                   (const T*)v, lv, (const T*)dout, ldo, lse, ll, (const float*)delta, lde, (T*)dk, ldk, (T*)dv,
                   ldv);
@@ -1130,7 +1150,8 @@ struct LQKBwd {
         if (!(sides & kKeySide)) return hipSuccess;
         const long long nk = static_cast<long long>(p.B) * p.nkey * p.Hkv;
         const int split = choose_split(p, nk, LPQ);
-        NA_LAUNCH("na_qk_bwd_k", (k_qk_bwd_k<T, DPL, LPQ>), dim3(grid_for(nk, LPQ * split)), dim3(256), 0, s, p, vec, split,
+        const auto kern = vec && unit_strides(p) ? k_qk_bwd_k<T, DPL, LPQ, true> : k_qk_bwd_k<T, DPL, LPQ, false>;
+        NA_LAUNCH("na_qk_bwd_k", kern, dim3(grid_for(nk, LPQ * split)), dim3(256), 0, s, p, vec, split,
                            (const T*)da, lda, (const T*)q, lq, (T*)dk, ldk);
         return hipGetLastError();
     }
@@ -1143,7 +1164,8 @@ struct LAVBwd {
         if (sides & kQuerySide) {
             const long long nq = static_cast<long long>(p.B) * p.nout * p.Hq;
             const int split = choose_split(p, nq, LPQ);
-            NA_LAUNCH("na_av_bwd_a", (k_av_bwd_a<T, DPL, LPQ>), dim3(grid_for(nq, LPQ * split)), dim3(256), 0, s, p, vec, split,
+            const auto kern = vec ? k_av_bwd_a<T, DPL, LPQ, true> : k_av_bwd_a<T, DPL, LPQ, false>;
+            NA_LAUNCH("na_av_bwd_a", kern, dim3(grid_for(nq, LPQ * split)), dim3(256), 0, s, p, split,
                       (const T*)dout, ldo, (const T*)v, lv, (T*)da, lda);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
@@ -1151,7 +1173,8 @@ struct LAVBwd {
         if (!(sides & kKeySide)) return hipSuccess;
         const long long nk = static_cast<long long>(p.B) * p.nkey * p.Hkv;
         const int split = choose_split(p, nk, LPQ);
-        NA_LAUNCH("na_av_bwd_v", (k_av_bwd_v<T, DPL, LPQ>), dim3(grid_for(nk, LPQ * split)), dim3(256), 0, s, p, vec, split,
+        const auto kern = vec && unit_strides(p) ? k_av_bwd_v<T, DPL, LPQ, true> : k_av_bwd_v<T, DPL, LPQ, false>;
+        NA_LAUNCH("na_av_bwd_v", kern, dim3(grid_for(nk, LPQ * split)), dim3(256), 0, s, p, vec, split,
                            (const T*)dout, ldo, (const T*)a, la, (T*)dv, ldv);
         return hipGetLastError();
     }
