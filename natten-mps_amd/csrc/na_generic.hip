@@ -21,6 +21,7 @@
 // 260 -> 80 / 85 / 152 (forward / dQ / dK dV); bfloat16 2 x 12 x 20 x 24 x 4,
 // dim 48, 3 x 5 x 5: 130 / 239 / 262 -> 77 / 156 / 145; fp32 split ops 4 x 45
 // x 61 x 4, dim 32, 7 x 7: query side 25 each, key side 66 -> 22-25 and 33.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1046,30 +1047,33 @@ inline unsigned grid_for(long long groups, int lpq) {
 
 // Lane groups per query (key).  Each group walks its neighbours (attending
 // queries) one after another, so a small problem (few groups) is bound by that
-// chain.  Splitting the walk over up to 8 groups, until the launch holds about
-// 1.5 waves per SIMD of a 256-CU device, shortens the chain; past that the
-// walks are bound by issue and L1 and the groups' own overhead shows.  fp32,
-// all launches of one pass, us, split 1 / 2 / 4 / 8:
-//   split 2 x 20 x 28 x 4, dim 64, 7 x 7     560 waves  110 / 83 / 73 / -
-//   fused 2 x 28 x 28 x 4, dim 64, 11 x 11   784 waves  154 / 107 / - / 129
-//   split 4 x 45 x 61 x 4, dim 32, 7 x 7    2745 waves  159 / 161 / 181 / -
-//   split 4 x 2048 x 4, dim 64, 33          4096 waves  131 / 150 / - / -
-// Groups stay within one wave (lpq * split <= 64) and never outnumber the
-// split axis's kernel positions.  NATTEN_HIP_SPLIT=n fixes it (tuning).
-inline int choose_split(const Prob& p, long long groups, int lpq) {
+// chain.  Splitting the walk over up to 8 groups shortens it, until the launch
+// fills a 256-CU device: past that the walks are bound by issue and L1 and the
+// groups' own overhead shows.  Over 3500 timed kernels (1-D to 3-D, head dims 10
+// to 256, splits of 1 to 8 forced) the best split reaches about 1.5 waves per
+// SIMD on the query side, 2 for the key side's pipelined walk and 3 for its
+// plain one, which waits on every step's loads; a group of a pipelined walk
+// needs a block of loads (8 neighbours) of its own.  By this rule they take 0.5
+// to 3.4 % more than at their best split (at 1.5 waves throughout 1.2 to 6.4 %;
+// dK/dV, bfloat16, 8 x 6 x 12 x 14 x 8, 3 x 5 x 5, dim 12: 350 -> 213 us, AV of
+// 2 x 300 x 4, 7, dim 72: 7.5 -> 5.7).  Groups stay within one wave (lpq * split
+// <= 64) and never outnumber the split axis's kernel positions.
+// NATTEN_HIP_SPLIT=n fixes it (tuning).
+inline int choose_split(const Prob& p, long long groups, int lpq, bool piped, bool key) {
     static const int forced = [] {
         const char* e = std::getenv("NATTEN_HIP_SPLIT");
         return e ? std::atoi(e) : 0;
     }();
-    const int kmax = p.ax[split_axis(p)].k;
-    constexpr long long kTargetWaves = 256LL * 4 * 3 / 2;
+    int kmax = p.ax[split_axis(p)].k;
+    if (piped) kmax = std::min(kmax, p.kv / 8);
+    const long long target = 256LL * (!key ? 6 : piped ? 8 : 12);
     int split = 1;
     if (forced > 0) {
         while (split * 2 <= forced && split * 2 * lpq <= 64) split *= 2;
         return split;
     }
     const long long waves = (groups * lpq + 63) / 64;
-    while (split < 8 && split * 2 * lpq <= 64 && split * 2 <= kmax && waves * split < kTargetWaves) split *= 2;
+    while (split < 8 && split * 2 * lpq <= 64 && split * 2 <= kmax && waves * split < target) split *= 2;
     return split;
 }
 
@@ -1078,7 +1082,7 @@ struct LForward {
     static hipError_t run(const Prob& p, int vec, const int* lens, const void* q, Lay lq, const void* k, Lay lk,
                           const void* v, Lay lv, void* o, Lay lo, float* lse, Lay ll, hipStream_t s) {
         const long long n = static_cast<long long>(p.B) * p.nout * p.Hq;
-        const int split = choose_split(p, n, LPQ);
+        const int split = choose_split(p, n, LPQ, vec != 0, false);
         NA_LAUNCH(lens ? "na_varlen_forward" : "na_forward", (k_forward<T, DPL, LPQ>),
                   dim3(grid_for(n, LPQ * split)), dim3(256), 0, s, p, vec, split, lens, (const T*)q, lq, (const T*)k, lk, (const T*)v, lv, (T*)o, lo, lse,
                   ll);
@@ -1091,7 +1095,7 @@ struct LQK {
     static hipError_t run(const Prob& p, int vec, const void* q, Lay lq, const void* k, Lay lk, void* a, Lay la,
                           hipStream_t s) {
         const long long n = static_cast<long long>(p.B) * p.nout * p.Hq;
-        const int split = choose_split(p, n, LPQ);
+        const int split = choose_split(p, n, LPQ, vec != 0, false);
         const auto kern = vec ? k_qk<T, DPL, LPQ, true> : k_qk<T, DPL, LPQ, false>;
         NA_LAUNCH("na_qk", kern, dim3(grid_for(n, LPQ * split)), dim3(256), 0, s, p, split, (const T*)q, lq,
                            (const T*)k, lk, (T*)a, la);
@@ -1104,7 +1108,7 @@ struct LAV {
     static hipError_t run(const Prob& p, int vec, const void* a, Lay la, const void* v, Lay lv, void* o, Lay lo,
                           hipStream_t s) {
         const long long n = static_cast<long long>(p.B) * p.nout * p.Hq;
-        const int split = choose_split(p, n, LPQ);
+        const int split = choose_split(p, n, LPQ, vec != 0, false);
         NA_LAUNCH("na_av", (k_av<T, DPL, LPQ>), dim3(grid_for(n, LPQ * split)), dim3(256), 0, s, p, vec, split, (const T*)a, la,
                            (const T*)v, lv, (T*)o, lo);
         return hipGetLastError();
@@ -1118,14 +1122,14 @@ struct LBackward {
                           Lay ll, const float* dlse, Lay ldl, void* dq, Lay ldq, void* dk, Lay ldk, void* dv,
                           Lay ldv, float* delta, Lay lde, hipStream_t s) {
         const long long nq = static_cast<long long>(p.B) * p.nout * p.Hq;
-        const int sq = choose_split(p, nq, LPQ);
+        const int sq = choose_split(p, nq, LPQ, vec != 0, false);
         NA_LAUNCH(lens ? "na_varlen_bwd_dq" : "na_bwd_dq", (k_bwd_dq<T, DPL, LPQ>), dim3(grid_for(nq, LPQ * sq)),
                   dim3(256), 0, s, p, vec, sq, lens, (const T*)q, lq, (const T*)k, lk, (const T*)v, lv, (const T*)o, lo,
                   (const T*)dout, ldo, lse, ll, dlse, ldl, (T*)dq, ldq, delta, lde);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         const long long nk = static_cast<long long>(p.B) * p.nkey * p.Hkv;
-        const int sk = choose_split(p, nk, LPQ);
+        const int sk = choose_split(p, nk, LPQ, vec && unit_strides(p), true);
         const auto kern_k = vec && unit_strides(p) ? k_bwd_dkdv<T, DPL, LPQ, true> : k_bwd_dkdv<T, DPL, LPQ, false>;
         NA_LAUNCH(lens ? "na_varlen_bwd_dkdv" : "na_bwd_dkdv", kern_k,
                   dim3(grid_for(nk, LPQ * sk)), dim3(256), 0, s, p, vec, sk, lens, (const T*)q, lq, (const T*)k, lk,
@@ -1141,7 +1145,7 @@ struct LQKBwd {
                           Lay lk, void* dq, Lay ldq, void* dk, Lay ldk, int sides, hipStream_t s) {
         if (sides & kQuerySide) {
             const long long nq = static_cast<long long>(p.B) * p.nout * p.Hq;
-            const int split = choose_split(p, nq, LPQ);
+            const int split = choose_split(p, nq, LPQ, vec != 0, false);
             NA_LAUNCH("na_qk_bwd_q", (k_qk_bwd_q<T, DPL, LPQ>), dim3(grid_for(nq, LPQ * split)), dim3(256), 0, s, p, vec, split,
                       (const T*)da, lda, (const T*)k, lk, (T*)dq, ldq);
             const hipError_t e = hipGetLastError();
@@ -1149,7 +1153,7 @@ struct LQKBwd {
         }
         if (!(sides & kKeySide)) return hipSuccess;
         const long long nk = static_cast<long long>(p.B) * p.nkey * p.Hkv;
-        const int split = choose_split(p, nk, LPQ);
+        const int split = choose_split(p, nk, LPQ, vec && unit_strides(p), true);
         const auto kern = vec && unit_strides(p) ? k_qk_bwd_k<T, DPL, LPQ, true> : k_qk_bwd_k<T, DPL, LPQ, false>;
         NA_LAUNCH("na_qk_bwd_k", kern, dim3(grid_for(nk, LPQ * split)), dim3(256), 0, s, p, vec, split,
                            (const T*)da, lda, (const T*)q, lq, (T*)dk, ldk);
@@ -1163,7 +1167,7 @@ struct LAVBwd {
                           Lay lv, void* da, Lay lda, void* dv, Lay ldv, int sides, hipStream_t s) {
         if (sides & kQuerySide) {
             const long long nq = static_cast<long long>(p.B) * p.nout * p.Hq;
-            const int split = choose_split(p, nq, LPQ);
+            const int split = choose_split(p, nq, LPQ, vec != 0, false);
             const auto kern = vec ? k_av_bwd_a<T, DPL, LPQ, true> : k_av_bwd_a<T, DPL, LPQ, false>;
             NA_LAUNCH("na_av_bwd_a", kern, dim3(grid_for(nq, LPQ * split)), dim3(256), 0, s, p, split,
                       (const T*)dout, ldo, (const T*)v, lv, (T*)da, lda);
@@ -1172,7 +1176,7 @@ struct LAVBwd {
         }
         if (!(sides & kKeySide)) return hipSuccess;
         const long long nk = static_cast<long long>(p.B) * p.nkey * p.Hkv;
-        const int split = choose_split(p, nk, LPQ);
+        const int split = choose_split(p, nk, LPQ, vec && unit_strides(p), true);
         const auto kern = vec && unit_strides(p) ? k_av_bwd_v<T, DPL, LPQ, true> : k_av_bwd_v<T, DPL, LPQ, false>;
         NA_LAUNCH("na_av_bwd_v", kern, dim3(grid_for(nk, LPQ * split)), dim3(256), 0, s, p, vec, split,
                            (const T*)dout, ldo, (const T*)a, la, (T*)dv, ldv);
