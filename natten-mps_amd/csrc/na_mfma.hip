@@ -1332,12 +1332,22 @@ bool deep_query_tile(const Prob& p, Kind kind, int D, const int (&n)[3]) {
 // 16 x 64 x 64 x 8, 3 x 5 x 5, dim 32 96 / 101 -> 70 / 73, dim 64 (batch 2)
 // 254 / 301 -> 221 / 269; 8 x 64 x 64 x 4, 5 x 5, dim 128 68 / 89 -> 47 / 48,
 // dim 96 67 / 76 -> 37 / 39; level at 3 x 3.  (Key tiles' unions reach further
-// at the borders: 20 to 60 % slower.)  2-D problems at head dim 32 / 64 keep
+// at the borders: 20 to 60 % slower.)  3 x 3 x 3 at head dim 96 and up gains from
+// 512 tiles on (8 x 16 x 16, 16 heads, dim 128: forward 0.68 of the time; 4 heads:
+// 1.11) and where an 8-wide box would be half empty.  2-D problems at head dim 32 / 64 keep
 // the 8 x 8 box: without their tables the 8x8 tile kernels hand them over, and
 // the bits must not depend on that (with global keys both boxes are level).
 bool narrow_query_tile(const Prob& p, Kind kind, int D, const int (&n)[3]) {
-    return (kind == kForward || kind == kBackwardQ) && fused_items() == kMaxItems && n[1] >= 8 && n[2] >= 8 &&
-           p.ax[2].k <= 5 && (p.ax[0].len > 1 || D >= 96);
+    if (!((kind == kForward || kind == kBackwardQ) && fused_items() == kMaxItems && n[1] >= 8 && n[2] >= 8 &&
+          p.ax[2].k <= 5 && (p.ax[0].len > 1 || D >= 96)))
+        return false;
+    if (D < 96 || p.ax[2].k > 3 || p.ax[0].len == 1 || n[2] < 16) return true;
+    long long tiles = static_cast<long long>(p.B) * p.Hq;
+    for (int a = 0; a < 3; ++a) {
+        const int t = a == 1 ? 8 : a == 2 ? 4 : p.ax[0].k > 1 ? 2 : 1;
+        tiles *= static_cast<long long>(p.ax[a].dil) * ((n[a] + t - 1) / t);
+    }
+    return tiles >= 512;
 }
 
 // LDS a forward / dQ workgroup adds for global keys: 32 key and 32 value rows.
