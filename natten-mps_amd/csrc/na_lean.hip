@@ -1951,19 +1951,17 @@ hipError_t lean_bwd_run(const Prob& p, const LeanGeo* gq, const LeanGeo* gk, con
 // staged rows high, a wave's own rows within the widest instance.  The
 // borders widen a union: at K = 8 and 9 a tile next to one reaches 20
 // columns, at K = 7 a class of 22 makes one of 17.  The same conditions as
-// lean_geometry's, from the extents alone; kept per axis geometry.
+// lean_geometry's, from the extents alone.  Every 2-D backward asks: a table
+// per thread holds the answers of the axes seen last, so that a call neither
+// waits for another thread's nor looks through every shape of the process.
 bool lean_key_tiles_fit(const Prob& p) {
     struct Entry {
         int len, k, dil, causal, u, rows, nst;
     };
-    static std::mutex mu;
-    static std::vector<Entry> cache;
-    const auto axis = [](const Axis& A) {
-        {
-            std::lock_guard<std::mutex> g(mu);
-            for (const Entry& e : cache)
-                if (e.len == A.len && e.k == A.k && e.dil == A.dil && e.causal == A.causal) return e;
-        }
+    const auto axis = [](const Axis& A) -> Entry {
+        thread_local Entry table[64];
+        Entry& slot = table[(static_cast<unsigned>(A.len) * 13 + A.k * 5 + A.dil * 3 + A.causal) % 64];
+        if (slot.len == A.len && slot.k == A.k && slot.dil == A.dil && slot.causal == A.causal) return slot;
         Entry e{A.len, A.k, A.dil, A.causal, 0, 0, 0};
         for (int r = 0; r < A.dil; ++r) {
             const int n = (A.len - r + A.dil - 1) / A.dil;
@@ -1979,10 +1977,7 @@ bool lean_key_tiles_fit(const Prob& p) {
                 e.nst = std::max(e.nst, a.U);
             }
         }
-        std::lock_guard<std::mutex> g(mu);
-        if (cache.size() >= 512) cache.clear();
-        cache.push_back(e);
-        return e;
+        return slot = e;
     };
     const Entry a1 = axis(p.ax[1]), a2 = axis(p.ax[2]);
     return a2.u <= 16 && a1.rows <= 2 * kLeanMaxKeyChunks && a1.nst <= 32;
