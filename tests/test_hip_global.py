@@ -32,6 +32,9 @@ CASES = [
     (2, (12, 12), 2, 1, 32, 5, (1, 1), (False, False), 5, torch.float16),
     (1, (300,), 4, 4, 32, 33, (1,), (False,), 64, torch.bfloat16),
     (2, (10, 11), 2, 2, 96, 3, (1, 1), (False, False), 7, torch.bfloat16),
+    # the tokens' LDS on top of a 57 KB union: 73 KB a workgroup
+    (2, (20, 22), 2, 2, 64, 7, (1, 1), (False, False), 33, torch.bfloat16),
+    (2, (17, 19), 4, 2, 64, 7, (1, 1), (True, False), 16, torch.float16),
 ]
 
 
