@@ -6,7 +6,7 @@
 // kernels (na_mfma.hip) stage a whole plane of the union: at kernel 13 x 13
 // and head dim 64 only a 16-query tile fits, which stages 23 rows of K and V
 // per query and runs one wave per workgroup.  Here a workgroup of 8 waves
-// owns 128 queries (keys) of one class triple and one (batch, head) -- a box
+// owns 128 queries (keys) of one class pair and one (batch, head) -- a box
 // of 128 / T2 rows of T2 = 8 or 16 columns, 16 items per wave -- and walks
 // the union a band of NC chunks (32 slots each) at a time, so that LDS holds
 // two bands whatever the kernel size:
@@ -16,8 +16,8 @@
 //   overlap the products, with one barrier per band.  (Loads straight to
 //   LDS cannot be used that way: the compiler waits for all of them before
 //   any LDS read.)
-// * A union row takes SL slots: 32 (kernels over 9 in-plane: a 16-column
-//   tile's union spans up to 15 + K columns), one row per chunk.
+// * A union row takes one chunk: 32 slots, which every union's columns fit
+//   (band_columns in na_common.h).
 // * A wave computes only the chunks that its own items' windows reach; its
 //   online softmax rescales once per band.
 //
@@ -26,11 +26,10 @@
 // chain; 8 waves and bands of 4 rows measured as fast as 4 waves or bands of
 // 2 (16 waves: 28 % slower).  Measured, general tile (or, *, vector) kernels
 // -> these: 13 x 13, head dim 64, fp16, 4 x 135 x 241, 8 heads, forward 2350
-// -> 250 us; bf16 4 x 64 x 64, 8 heads, forward 275 -> 37, dQ 981* -> 71,
-// dK/dV 968* -> 99 us; head dim 128, 4 heads 501* / 1043* / 998* -> 42 / 83 /
-// 85 us; 11 x 11, head dim 32, 4 x 61 x 130, 8 heads 103 / 139 / 128 -> 50 /
-// 83 / 69 us.  (*: the two-term products of band_sides; one term takes 36 /
-// 61 / 78 in the first case.)
+// -> 252 us; bf16 4 x 64 x 64, 8 heads, forward 275 -> 35, dQ 981* -> 70,
+// dK/dV 968* -> 81 us; head dim 128, 4 heads 501* / 1043* / 998* -> 40 / 82 /
+// 82 us; 11 x 11, head dim 32, 4 x 61 x 130, 8 heads 103 / 139 / 128 -> 46 /
+// 81 / 62 us.  (*: the two-term products of band_sides.)
 //
 // The geometry is computed in the kernel (no tables): every call, captured
 // or not, runs the same code.  MFMA lane layouts, the swizzle and the masks
@@ -65,7 +64,7 @@ constexpr int kBandOp = kBandChunks<D> * 32 * D * 2;
 // and the divisors that decode a workgroup's index.
 struct BandGeo {
     int sh1, sh2;
-    int lenmod[3];
+    int lenmod[3];                            // (axes 1 and 2, as the next two)
     FastDiv heads, tiles, rep, nt[3], dil[3];
 };
 
@@ -82,10 +81,12 @@ struct BandArgs {
 };
 
 // A workgroup's tile: batch, head (kv head on the key side), the tile's
-// geometry per axis (with this wave's box), residues.
+// geometry on axes 1 and 2 (with this wave's box), residues.
 struct BandTile {
     int b, h, r[3];
     AxisGeo a[3];
+    __device__ __forceinline__ bool tile_ok() const { return a[1].tile_ok && a[2].tile_ok; }
+    __device__ __forceinline__ bool wave_ok() const { return a[1].wave_ok && a[2].wave_ok; }
 };
 
 template <bool KEY>
@@ -98,7 +99,7 @@ __device__ __forceinline__ BandTile band_tile(const Prob& p, const BandGeo& g, i
     int s = bt - t.b * static_cast<int>(g.tiles.d);
     int tt[3];
 #pragma unroll
-    for (int a = 2; a >= 0; --a) {
+    for (int a = 2; a >= 1; --a) {
         int q = fdiv(s, g.nt[a]);
         tt[a] = s - q * static_cast<int>(g.nt[a].d);
         s = q;
@@ -106,14 +107,12 @@ __device__ __forceinline__ BandTile band_tile(const Prob& p, const BandGeo& g, i
         t.r[a] = s - q * static_cast<int>(g.dil[a].d);
         s = q;
     }
-    const int T[3] = {(kBandWaves * 16) >> (g.sh1 + g.sh2), 1 << g.sh1, 1 << g.sh2};
-    // the wave's items 16 w .. 16 w + 15 in row-major order: whole rows of
-    // one depth (T2 <= 16)
-    const int f0 = wave * 16;
-    const int e0 = f0 >> (g.sh1 + g.sh2), e1 = (f0 >> g.sh2) & (T[1] - 1);
-    const int wl[3] = {e0, e1, 0}, wh[3] = {e0, e1 + (16 >> g.sh2) - 1, T[2] - 1};
+    const int T[3] = {1, 1 << g.sh1, 1 << g.sh2};
+    // the wave's items 16 w .. 16 w + 15 in row-major order: whole rows (T2 <= 16)
+    const int e1 = wave * 16 >> g.sh2;
+    const int wl[3] = {0, e1, 0}, wh[3] = {0, e1 + (16 >> g.sh2) - 1, T[2] - 1};
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
+    for (int a = 1; a < 3; ++a) {
         const Axis& A = p.ax[a];
         t.a[a] = axis_geometry(A.len, A.k, A.dil, A.causal, g.lenmod[a], 1, A.len, T[a], tt[a], t.r[a], wl[a], wh[a],
                                KEY, g.dil[a]);
@@ -136,12 +135,13 @@ struct BandLane {
 template <bool KEY>
 __device__ __forceinline__ BandLane band_lane(const Prob& p, const BandGeo& g, const BandTile& t, int wave, int col) {
     const int f = wave * 16 + col;
-    const int e[3] = {f >> (g.sh1 + g.sh2), (f >> g.sh2) & ((1 << g.sh1) - 1), f & ((1 << g.sh2) - 1)};
+    const int e[3] = {0, f >> g.sh2, f & ((1 << g.sh2) - 1)};
     BandLane l;
-    l.valid = e[0] < t.a[0].E && e[1] < t.a[1].E && e[2] < t.a[2].E;
+    l.valid = e[1] < t.a[1].E && e[2] < t.a[2].E;
+    l.pos[0] = 0;
     int lo[3], hi[3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
+    for (int a = 1; a < 3; ++a) {
         const int j = t.a[a].J + (l.valid ? e[a] : 0);
         l.pos[a] = t.r[a] + j * p.ax[a].dil;
         item_box(band_class(p.ax[a], t.a[a]), j, KEY, lo[a], hi[a]);
@@ -155,9 +155,8 @@ __device__ __forceinline__ BandLane band_lane(const Prob& p, const BandGeo& g, c
 
 // Column mask of the lane's 8 slots of a chunk, as the score product's
 // accumulator input.
-template <int SL>
 __device__ __forceinline__ void band_colbias(const BandLane& l, int grp, f32x4_t (&bias)[2]) {
-    const int c0 = 8 * (grp & (SL / 8 - 1)) - l.clo;
+    const int c0 = 8 * grp - l.clo;
 #pragma unroll
     for (int e = 0; e < 8; ++e)
         bias[e >> 2][e & 3] = static_cast<unsigned>(c0 + e) < static_cast<unsigned>(l.cn) ? 0.f : -INFINITY;
@@ -178,8 +177,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t band_rsrc(const T* p, uint32_t
 // the next, and a transposing pass x = 0, 1 or x = 2, 3 of all y, two
 // neighbouring pieces each: both are free of conflicts when the swizzle's
 // bits above 0 take every value over (x % 2, y) and bit 0 stays clear.  With
-// swz (na_tile.h) the transposing reads take two passes more: 2 to 4 % of
-// these kernels' time (13 x 13, head dim 64, dK/dV 103 -> 100 us).
+// swz (na_tile.h) the transposing reads take two passes more, which shows
+// little: dK/dV 11 x 11, head dim 32, 63.5 -> 61.9 us, 13 x 13, head dim 128,
+// 82.3 -> 81.6, but 9 x 9, head dim 64, 106 -> 107 us.
 template <int D>
 __host__ __device__ constexpr int band_swz(int row) {
     if constexpr (D == 32) return ((row >> 3) & 1) << 1;
@@ -188,34 +188,26 @@ __host__ __device__ constexpr int band_swz(int row) {
 }
 
 // Staging of two operands' bands: thread t moves 16-byte piece t % P of
-// slots t / P + j * SPT, j < NP, of each operand (SPT slots per round of the
-// workgroup).  Columns past the union and rows past it load from outside the
-// buffer (zeros).  A round covers whole union rows, or 1 / CPR of one.
-template <typename T, int D, int SL>
+// slots t / P + j * SPT, j < NP, of each operand (SPT slots, whole union rows,
+// per round of the workgroup).  Columns past the union and rows past it load
+// from outside the buffer (zeros).
+template <typename T, int D>
 struct BandStage {
     static constexpr int P = D / 8, NP = kBandChunks<D> * 32 * P / kBandThreads, SPT = kBandThreads / P;
-    static constexpr int CPR = SPT >= SL ? 1 : SL / SPT;            // rounds per union row
-    static constexpr int RB = kBandChunks<D> * 32 / SL;             // union rows per band
-    static_assert(SPT % SL == 0 || SL % SPT == 0, "rounds of whole rows or equal parts of one");
-    static_assert((P * (SPT < SL ? SPT : SL)) % 64 == 0, "a wave stays in one union row");
-    static_assert(SPT % 16 == 0 && (SPT % 32 == 0 || CPR == 2), "the swizzle repeats every 32 slots");
-    int row0, dst[CPR];           // first union row (wave-uniform); LDS byte offset of rounds 0 .. CPR - 1
-    uint32_t ca[CPR], cb[CPR];    // lane part of the global offsets
+    static_assert(SPT % 32 == 0, "rounds of whole rows; the swizzle repeats every 32 slots");
+    int row0, dst;                // first union row (wave-uniform); LDS byte offset of round 0
+    uint32_t ca, cb;              // lane part of the global offsets
     int base_a, base_b, step_a, step_b;
     uint4 ra[NP], rb[NP];
 
     __device__ __forceinline__ void init(const Prob& p, const BandTile& t, const LayK& la, const LayK& lb) {
-        const int tid = threadIdx.x, pp = tid % P, slot0 = tid / P;
-        row0 = __builtin_amdgcn_readfirstlane(slot0 / SL);
+        const int tid = threadIdx.x, pp = tid % P, slot = tid / P, c = slot % 32;
+        row0 = __builtin_amdgcn_readfirstlane(slot / 32);
         const int d1 = p.ax[1].dil, d2 = p.ax[2].dil;
-#pragma unroll
-        for (int r = 0; r < CPR; ++r) {
-            const int slot = slot0 + r * SPT, c = slot % SL;
-            dst[r] = slot * D * 2 + ((pp ^ band_swz<D>(slot)) << 4);
-            const bool in = c < t.a[2].U;
-            ca[r] = in ? static_cast<uint32_t>(c * d2 * la.s2 * 2 + pp * 16) : kBandOOR;
-            cb[r] = in ? static_cast<uint32_t>(c * d2 * lb.s2 * 2 + pp * 16) : kBandOOR;
-        }
+        dst = slot * D * 2 + ((pp ^ band_swz<D>(slot)) << 4);
+        const bool in = c < t.a[2].U;
+        ca = in ? static_cast<uint32_t>(c * d2 * la.s2 * 2 + pp * 16) : kBandOOR;
+        cb = in ? static_cast<uint32_t>(c * d2 * lb.s2 * 2 + pp * 16) : kBandOOR;
         const int p1 = t.r[1] + t.a[1].lo * d1, p2 = t.r[2] + t.a[2].lo * d2;
         base_a = (p1 * la.s1 + p2 * la.s2) * 2;
         base_b = (p1 * lb.s1 + p2 * lb.s2) * 2;
@@ -227,11 +219,11 @@ struct BandStage {
     __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t pa, __amdgpu_buffer_rsrc_t pb, int bi, int U1) {
 #pragma unroll
         for (int j = 0; j < NP; ++j) {
-            const int row = bi * RB + row0 + j * SPT / SL, r = j % CPR;
+            const int row = bi * kBandChunks<D> + row0 + j * (SPT / 32);
             const uint32_t oa = row < U1 ? static_cast<uint32_t>(base_a + row * step_a) : kBandOOR;
             const uint32_t ob = row < U1 ? static_cast<uint32_t>(base_b + row * step_b) : kBandOOR;
-            ra[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(pa, ca[r] + oa, 0, 0));
-            rb[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(pb, cb[r] + ob, 0, 0));
+            ra[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(pa, ca + oa, 0, 0));
+            rb[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(pb, cb + ob, 0, 0));
         }
     }
 
@@ -239,7 +231,7 @@ struct BandStage {
     __device__ __forceinline__ void store(unsigned char* buf) const {
 #pragma unroll
         for (int j = 0; j < NP; ++j) {
-            unsigned char* x = buf + dst[j % CPR] + j / CPR * (CPR * kBandThreads * 16);
+            unsigned char* x = buf + dst + j * (kBandThreads * 16);
             *reinterpret_cast<uint4*>(x) = ra[j];
             *reinterpret_cast<uint4*>(x + kBandOp<D>) = rb[j];
         }
@@ -308,8 +300,8 @@ __device__ __forceinline__ uint4 pack_rest(const f32x4_t (&v)[2], uint4 packed) 
 // powers of two, exact to apply and to take out: P of the key side by 2^15 (P
 // <= 1 up to rounding), dS by a factor of its item's own.  Unscaled, dQ and dK
 // lost up to 7 times their rounding error at dO ~ 1e-3 (97 x 16, head dim
-// 32); scaled, none.  Time: 4 x 64 x 64 x 8, dim 64, 13 x 13, fp16 69 -> 74 us
-// (dQ) and 98 -> 105 us (dK/dV).
+// 32); scaled, none.  Time: 4 x 64 x 64 x 8, dim 64, 13 x 13, fp16 68 -> 71 us
+// (dQ) and 80 -> 88 us (dK/dV).
 template <typename T, bool TWO>
 constexpr bool kScaled = TWO && std::is_same_v<T, f16>;
 constexpr float kScaleP = 32768.f;
@@ -361,11 +353,12 @@ __device__ __forceinline__ void band_accumulate(const unsigned char* X, const Ba
     }
 }
 
-// Walk over the union: bands of a plane, then the next plane (and, key
-// side, the next q head).
-struct BandWalk {
-    int bi, u0, h;
-};
+// Chunks of a band whose code the backward kernels lay side by side.  With two
+// terms at head dim 64 that spilled 12 to 47 registers; one after another, 0
+// to 12 (13 x 13, 4 x 135 x 241 x 8, bfloat16, dQ 586 -> 546, dK/dV 1040 -> 685
+// us).
+template <int D, bool TWO>
+constexpr int kBandUnroll = TWO && D == 64 ? 1 : kBandChunks<D>;
 
 // Waves per SIMD the kernels are built for: two workgroups of 8 waves fit a
 // CU's LDS; at head dim 128 the backward kernels need the registers of one.
@@ -373,7 +366,8 @@ constexpr int band_waves(int D, bool backward) { return D == 128 && backward ? 2
 #define NA_BAND_OCC(D, BWD) __attribute__((amdgpu_waves_per_eu(band_waves(D, BWD))))
 
 template <typename T, int D>
-__device__ __forceinline__ void band_redo_fwd(const void* kargs, int b, int h, int hk, int p0, int p1, int p2, int grp) {
+__device__ __forceinline__ void band_redo_fwd(const void* kargs, int b, int h, int hk, int p0, int p1, int p2,
+                                              int grp) {
     const BandArgs<T>& A = *static_cast<const BandArgs<T>*>(kargs);
     const int pos[3] = {p0, p1, p2};
     ExactAxis x[3];
@@ -386,60 +380,50 @@ __device__ __forceinline__ void band_redo_fwd(const void* kargs, int b, int h, i
     if (grp == 0) bh_ptr(A.lse_out, A.ll, b, h)[vol_off(A.ll, pos)] = lse_v;
 }
 
-template <typename T, int D, int SL, bool TWO>
+template <typename T, int D, bool TWO>
 __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd(BandArgs<T> args) {
-    constexpr int NC = kBandChunks<D>, RPC = 32 / SL, BUF = 2 * kBandOp<D>;
+    constexpr int NC = kBandChunks<D>, BUF = 2 * kBandOp<D>;
     const Prob& p = args.p;
     unsigned char* smem = lds_base();
     const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const BandTile t = band_tile<false>(p, args.g, wave);
-    if (!(t.a[0].tile_ok && t.a[1].tile_ok && t.a[2].tile_ok)) return;
+    if (!t.tile_ok()) return;
     const int hk = args.g.rep.d == 1 ? t.h : fdiv(t.h, args.g.rep);
     const T* kb = bh_ptr(args.k, args.lk, t.b, hk);
     const T* vb = bh_ptr(args.v, args.lv, t.b, hk);
-    BandStage<T, D, SL> st;
+    BandStage<T, D> st;
     st.init(p, t, args.lk, args.lv);
-    const int U0 = t.a[0].U, U1 = t.a[1].U, nb = (U1 + st.RB - 1) / st.RB;
-    const auto load = [&](int u0, int bi) {
-        const int p0 = t.r[0] + (t.a[0].lo + u0) * p.ax[0].dil;
-        st.load(band_rsrc(kb + p0 * args.lk.s0, args.ab), band_rsrc(vb + p0 * args.lv.s0, args.bb), bi, U1);
-    };
-    load(0, 0);
+    const int U1 = t.a[1].U, nb = (U1 + NC - 1) / NC;
+    const auto load = [&](int bi) { st.load(band_rsrc(kb, args.ab), band_rsrc(vb, args.bb), bi, U1); };
+    load(0);
 
     const BandLane ln = band_lane<false>(p, args.g, t, wave, col);
     uint4 qf[D / 32];
     load_frags<T, D>(bh_ptr(args.q, args.lq, t.b, t.h), vol_off(args.lq, ln.pos), ln.valid, grp, qf);
     f32x4_t cb[2];
-    band_colbias<SL>(ln, grp, cb);
+    band_colbias(ln, grp, cb);
     BandOff<D> off;
     off.init(lane);
     const float sc2 = p.scale * kLog2e;
-    const bool wave_ok = t.a[0].wave_ok && t.a[1].wave_ok && t.a[2].wave_ok;
-    // the wave's chunks of a plane, and its planes
-    const int wc0 = t.a[1].glo / RPC, wc1 = wave_ok ? t.a[1].ghi / RPC : -1;
-    const int w0 = t.a[0].glo, w1 = t.a[0].ghi;
+    // the wave's chunks
+    const int wc0 = t.a[1].glo, wc1 = t.wave_ok() ? t.a[1].ghi : -1;
     const uint4 ones = make_uint4(Mma<T>::kOnes, Mma<T>::kOnes, Mma<T>::kOnes, Mma<T>::kOnes);
 
     f32x4_t acc[D / 16], lacc = f32x4_t{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, lpart = 0.f;
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    int u0 = 0, bi = 0;
+    int bi = 0;
     // one band: publish it in buffer B, request the next one, compute
     const auto step = [&](auto BC) {
         constexpr int B = decltype(BC)::value;
         st.store(smem + B * BUF);
         lds_publish_barrier();
-        const int cu = u0, cbi = bi;
-        if (++bi == nb) {
-            bi = 0;
-            ++u0;
-        }
-        const bool more = u0 < U0;
-        if (more) load(u0, bi);
-        const int c0 = cbi * NC;
-        if (cu >= w0 && cu <= w1 && c0 + NC - 1 >= wc0 && c0 <= wc1) {
+        const int c0 = bi * NC;
+        const bool more = ++bi < nb;
+        if (more) load(bi);
+        if (c0 + NC - 1 >= wc0 && c0 <= wc1) {
             const unsigned char* Kb = smem + B * BUF;
             const unsigned char* Vb = Kb + kBandOp<D>;
             f32x4_t s[NC][2];
@@ -448,7 +432,7 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
                 if (c0 + c >= wc0 && c0 + c <= wc1) {
-                    const int row = (c0 + c) * RPC + (RPC == 2 ? grp >> 1 : 0) - ln.rlo;
+                    const int row = c0 + c - ln.rlo;
                     rv[c] = static_cast<unsigned>(row) < static_cast<unsigned>(ln.rn);
                     band_score<T, D>(Kb, off, c, qf, cb, s[c]);
                     cm = fmaxp(cm, rv[c] ? max8(s[c]) : -INFINITY);
@@ -496,7 +480,7 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, false) void k_band_fwd
         band_redo_fwd<T, D>(kernargs(), t.b, t.h, hk, opaque(ln.pos[0]), opaque(ln.pos[1]), opaque(ln.pos[2]), grp);
 }
 
-// Backward, query side: as k_bwd_q_mfma.  2-D: a first walk takes delta =
+// Backward, query side: as k_bwd_q_mfma.  A first walk takes delta =
 // sum over the window of P dP (= dO . O) from the kernel's own products
 // (where that is not finite, dO . O from the rows), a second one forms dS =
 // P (dP - delta) and dq.
@@ -517,25 +501,22 @@ __device__ __forceinline__ void band_redo_bwd_q(const void* kargs, int b, int h,
     store_rows<T, D>(bh_ptr(A.dq, A.ldq, b, h), vol_off(A.ldq, pos), grp, acc, A.p.scale);
 }
 
-template <typename T, int D, int SL, bool TWO>
+template <typename T, int D, bool TWO>
 __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_q(BandArgs<T> args) {
-    constexpr int NC = kBandChunks<D>, RPC = 32 / SL, BUF = 2 * kBandOp<D>;
+    constexpr int NC = kBandChunks<D>, BUF = 2 * kBandOp<D>;
     const Prob& p = args.p;
     unsigned char* smem = lds_base();
     const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const BandTile t = band_tile<false>(p, args.g, wave);
-    if (!(t.a[0].tile_ok && t.a[1].tile_ok && t.a[2].tile_ok)) return;
+    if (!t.tile_ok()) return;
     const int hk = args.g.rep.d == 1 ? t.h : fdiv(t.h, args.g.rep);
     const T* kb = bh_ptr(args.k, args.lk, t.b, hk);
     const T* vb = bh_ptr(args.v, args.lv, t.b, hk);
-    BandStage<T, D, SL> st;
+    BandStage<T, D> st;
     st.init(p, t, args.lk, args.lv);
-    const int U1 = t.a[1].U, nb = (U1 + st.RB - 1) / st.RB;
-    const int p0 = t.r[0] + t.a[0].lo * p.ax[0].dil;
-    const auto load = [&](int bi) {
-        st.load(band_rsrc(kb + p0 * args.lk.s0, args.ab), band_rsrc(vb + p0 * args.lv.s0, args.bb), bi, U1);
-    };
+    const int U1 = t.a[1].U, nb = (U1 + NC - 1) / NC;
+    const auto load = [&](int bi) { st.load(band_rsrc(kb, args.ab), band_rsrc(vb, args.bb), bi, U1); };
     load(0);
 
     const BandLane ln = band_lane<false>(p, args.g, t, wave, col);
@@ -545,12 +526,11 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
     const float L2 = ln.valid ? bh_ptr(args.lse, args.ll, t.b, t.h)[vol_off(args.ll, ln.pos)] * kLog2e : 0.f;
     const float dl = ln.valid && args.dlse ? bh_ptr(args.dlse, args.ldl, t.b, t.h)[vol_off(args.ldl, ln.pos)] : 0.f;
     f32x4_t cb[2];
-    band_colbias<SL>(ln, grp, cb);
+    band_colbias(ln, grp, cb);
     BandOff<D> off;
     off.init(lane);
     const float sc2 = p.scale * kLog2e;
-    const bool wave_ok = t.a[0].wave_ok && t.a[1].wave_ok && t.a[2].wave_ok;
-    const int wc0 = t.a[1].glo / RPC, wc1 = wave_ok ? t.a[1].ghi / RPC : -1;
+    const int wc0 = t.a[1].glo, wc1 = t.wave_ok() ? t.a[1].ghi : -1;
     const f32x4_t zero[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
 
     f32x4_t acc[D / 16];
@@ -572,10 +552,10 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
         if (more) load(bi);
         const unsigned char* Kb = smem + B * BUF;
         const unsigned char* Vb = Kb + kBandOp<D>;
-#pragma unroll
+#pragma unroll kBandUnroll<D, TWO>
         for (int c = 0; c < NC; ++c) {
             if (c0 + c < wc0 || c0 + c > wc1) continue;
-            const int row = (c0 + c) * RPC + (RPC == 2 ? grp >> 1 : 0) - ln.rlo;
+            const int row = c0 + c - ln.rlo;
             const float o = static_cast<unsigned>(row) < static_cast<unsigned>(ln.rn) ? -L2 : -INFINITY;
             f32x4_t s[2], dp[2];
             band_score<T, D>(Kb, off, c, qf, cb, s);
@@ -653,18 +633,18 @@ __device__ __forceinline__ void band_redo_bwd_kv(const void* kargs, int b, int h
     store_rows<T, D>(bh_ptr(A.dk, A.ldk, b, hk), vol_off(A.ldk, pos), grp, g, A.p.scale);
 }
 
-template <typename T, int D, int SL, bool TWO>
+template <typename T, int D, bool TWO>
 __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_kv(BandArgs<T> args) {
-    constexpr int NC = kBandChunks<D>, RPC = 32 / SL, BUF = 2 * kBandOp<D>, NS = NC * 32;
+    constexpr int NC = kBandChunks<D>, BUF = 2 * kBandOp<D>, NS = NC * 32;
     const Prob& p = args.p;
     unsigned char* smem = lds_base();
     float* scal = reinterpret_cast<float*>(smem + 2 * BUF);  // per buffer NS (-lse), NS (-delta); then 8 x -inf
     const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const BandTile t = band_tile<true>(p, args.g, wave);
-    if (!(t.a[0].tile_ok && t.a[1].tile_ok && t.a[2].tile_ok)) return;
+    if (!t.tile_ok()) return;
     const BandLane ln = band_lane<true>(p, args.g, t, wave, col);
-    const int U0 = t.a[0].U, U1 = t.a[1].U, U2 = t.a[2].U;
+    const int U1 = t.a[1].U, U2 = t.a[2].U;
     f32x4_t gk[D / 16], gv[D / 16];
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) gk[db] = gv[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -676,32 +656,31 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
         store_rows<T, D>(bh_ptr(args.dv, args.ldv, t.b, t.h), vol_off(args.ldv, ln.pos), grp, gv,
                          S ? 1.f / kScaleP : 1.f);
     };
-    if (U0 == 0 || U1 == 0 || U2 == 0) {  // no query attends these keys
+    if (U1 == 0 || U2 == 0) {  // no query attends these keys
         if (ln.valid) store();
         return;
     }
     const int rep = static_cast<int>(args.g.rep.d);
-    BandStage<T, D, SL> st;
+    BandStage<T, D> st;
     st.init(p, t, args.lq, args.ldo);
-    const int nb = (U1 + st.RB - 1) / st.RB;
+    const int nb = (U1 + NC - 1) / NC;
     // the thread's slot of a band (threads past NS load slot 0's scalars and drop them)
     const int sslot = threadIdx.x < NS ? static_cast<int>(threadIdx.x) : 0;
-    const int srow = sslot / SL, scol = sslot % SL;
+    const int srow = sslot / 32, scol = sslot % 32;
     const bool sin = scol < U2;
     const int q2 = t.r[2] + (t.a[2].lo + (sin ? scol : 0)) * p.ax[2].dil;
     const int sl2 = q2 * args.ll.s2, sd2 = q2 * args.lde.s2;
     float pl, pd;
     bool pin;
-    int h = t.h * rep, u0 = 0, bi = 0;
+    int h = t.h * rep, bi = 0;
     const auto load = [&]() {
-        const int p0 = t.r[0] + (t.a[0].lo + u0) * p.ax[0].dil;
-        const int row = bi * st.RB + srow;
+        const int row = bi * NC + srow;
         pin = sin && row < U1;
         const int p1 = t.r[1] + (t.a[1].lo + (pin ? row : 0)) * p.ax[1].dil;
-        pl = (bh_ptr(args.lse, args.ll, t.b, h) + p0 * args.ll.s0)[p1 * args.ll.s1 + sl2];
-        pd = (bh_ptr(args.delta, args.lde, t.b, h) + p0 * args.lde.s0)[p1 * args.lde.s1 + sd2];
-        st.load(band_rsrc(bh_ptr(args.q, args.lq, t.b, h) + p0 * args.lq.s0, args.ab),
-                band_rsrc(bh_ptr(args.dout, args.ldo, t.b, h) + p0 * args.ldo.s0, args.bb), bi, U1);
+        pl = bh_ptr(args.lse, args.ll, t.b, h)[p1 * args.ll.s1 + sl2];
+        pd = bh_ptr(args.delta, args.lde, t.b, h)[p1 * args.lde.s1 + sd2];
+        st.load(band_rsrc(bh_ptr(args.q, args.lq, t.b, h), args.ab),
+                band_rsrc(bh_ptr(args.dout, args.ldo, t.b, h), args.bb), bi, U1);
     };
     load();
 
@@ -710,13 +689,11 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
     load_frags<T, D>(bh_ptr(args.v, args.lv, t.b, t.h), vol_off(args.lv, ln.pos), ln.valid, grp, vf);
     if (threadIdx.x < 8) scal[4 * NS + threadIdx.x] = -INFINITY;
     f32x4_t cb[2];
-    band_colbias<SL>(ln, grp, cb);
+    band_colbias(ln, grp, cb);
     BandOff<D> off;
     off.init(lane);
     const float sc2 = p.scale * kLog2e;
-    const bool wave_ok = t.a[0].wave_ok && t.a[1].wave_ok && t.a[2].wave_ok;
-    const int wc0 = t.a[1].glo / RPC, wc1 = wave_ok ? t.a[1].ghi / RPC : -1;
-    const int w0 = t.a[0].glo, w1 = t.a[0].ghi;
+    const int wc0 = t.a[1].glo, wc1 = t.wave_ok() ? t.a[1].ghi : -1;
     const int hend = (t.h + 1) * rep;
     const float* ninf = scal + 4 * NS;
     const auto step = [&](auto BC) {
@@ -727,57 +704,52 @@ __global__ __launch_bounds__(kBandThreads) NA_BAND_OCC(D, true) void k_band_bwd_
             scal[B * 2 * NS + NS + threadIdx.x] = pin ? -pd : 0.f;
         }
         lds_publish_barrier();
-        const int c0 = bi * NC, cu = u0;
+        const int c0 = bi * NC;
         if (++bi == nb) {
             bi = 0;
-            if (++u0 == U0) {
-                u0 = 0;
-                ++h;
-            }
+            ++h;
         }
         const bool more = h < hend;
         if (more) load();
         const unsigned char* Qb = smem + B * BUF;
         const unsigned char* Gb = Qb + kBandOp<D>;
-        if (cu >= w0 && cu <= w1) {
+#pragma unroll kBandUnroll<D, TWO>
+        for (int c = 0; c < NC; ++c) {
+            if (c0 + c < wc0 || c0 + c > wc1) continue;
+            const int row = c0 + c - ln.rlo;
+            const float* sc = scal + B * 2 * NS + 32 * c + 8 * grp;
+            const float* nlc = static_cast<unsigned>(row) < static_cast<unsigned>(ln.rn) ? sc : ninf;
+            const f32x4_t nl[2] = {*reinterpret_cast<const f32x4_t*>(nlc),
+                                   *reinterpret_cast<const f32x4_t*>(nlc + 4)};
+            const f32x4_t nd[2] = {*reinterpret_cast<const f32x4_t*>(sc + NS),
+                                   *reinterpret_cast<const f32x4_t*>(sc + NS + 4)};
+            f32x4_t s[2], dp[2];
+            band_score<T, D>(Qb, off, c, kf, cb, s);
+            band_score<T, D>(Gb, off, c, vf, nd, dp);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                if (c0 + c < wc0 || c0 + c > wc1) continue;
-                const int row = (c0 + c) * RPC + (RPC == 2 ? grp >> 1 : 0) - ln.rlo;
-                const float* sc = scal + B * 2 * NS + 32 * c + 8 * grp;
-                const float* nlc = static_cast<unsigned>(row) < static_cast<unsigned>(ln.rn) ? sc : ninf;
-                const f32x4_t nl[2] = {*reinterpret_cast<const f32x4_t*>(nlc),
-                                       *reinterpret_cast<const f32x4_t*>(nlc + 4)};
-                const f32x4_t nd[2] = {*reinterpret_cast<const f32x4_t*>(sc + NS),
-                                       *reinterpret_cast<const f32x4_t*>(sc + NS + 4)};
-                f32x4_t s[2], dp[2];
-                band_score<T, D>(Qb, off, c, kf, cb, s);
-                band_score<T, D>(Gb, off, c, vf, nd, dp);
+            for (int bb = 0; bb < 2; ++bb)
 #pragma unroll
-                for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        s[bb][i] = __builtin_amdgcn_exp2f(fmaf(s[bb][i], sc2, nl[bb][i]));
-                        if constexpr (kScaled<T, TWO>) s[bb][i] *= kScaleP;
-                        dp[bb][i] *= s[bb][i];
-                    }
-                if constexpr (kScaled<T, TWO>) {
-                    // a new maximum past the limit lowers the item's factor (and what
-                    // it has gathered), as the forward's online softmax does
-                    const float mx = abs_max8(dp, 0.f);
-                    if (__any(mx * gs >= kScaleLimit)) {
-                        const float m = max_rows_num(mx), ng = m * gs >= kScaleLimit ? scale_for(m) : gs;
-                        const float corr = ng * inv_pow2(gs);
-                        gs = ng;
-#pragma unroll
-                        for (int db = 0; db < D / 16; ++db) gk[db] *= corr;
-                    }
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) dp[i >> 2][i & 3] *= gs;
+                for (int i = 0; i < 4; ++i) {
+                    s[bb][i] = __builtin_amdgcn_exp2f(fmaf(s[bb][i], sc2, nl[bb][i]));
+                    if constexpr (kScaled<T, TWO>) s[bb][i] *= kScaleP;
+                    dp[bb][i] *= s[bb][i];
                 }
-                band_accumulate<T, D, TWO>(Gb, off, c, s, gv);
-                band_accumulate<T, D, TWO>(Qb, off, c, dp, gk);
+            if constexpr (kScaled<T, TWO>) {
+                // a new maximum past the limit lowers the item's factor (and what
+                // it has gathered), as the forward's online softmax does
+                const float mx = abs_max8(dp, 0.f);
+                if (__any(mx * gs >= kScaleLimit)) {
+                    const float m = max_rows_num(mx), ng = m * gs >= kScaleLimit ? scale_for(m) : gs;
+                    const float corr = ng * inv_pow2(gs);
+                    gs = ng;
+#pragma unroll
+                    for (int db = 0; db < D / 16; ++db) gk[db] *= corr;
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) dp[i >> 2][i & 3] *= gs;
             }
+            band_accumulate<T, D, TWO>(Gb, off, c, s, gv);
+            band_accumulate<T, D, TWO>(Qb, off, c, dp, gk);
         }
         return more;
     };
@@ -800,7 +772,7 @@ BandGeo band_geo(const Prob& p, int sh2, int heads) {
     g.sh1 = log2_of(kBandWaves * 16) - sh2;
     const int T[3] = {1, 1 << g.sh1, 1 << g.sh2};
     long long tiles = 1;
-    for (int a = 0; a < 3; ++a) {
+    for (int a = 1; a < 3; ++a) {
         const int n = (n_class_h(p.ax[a], 0) + T[a] - 1) / T[a];
         g.lenmod[a] = p.ax[a].len % p.ax[a].dil;
         g.nt[a] = make_fastdiv(static_cast<uint32_t>(n));
@@ -829,12 +801,12 @@ constexpr size_t kBandLdsKv = kBandLds<T, D> + (4 * kBandChunks<D> * 32 + 8) * s
 
 template <typename T, int D>
 void band_audit_dim(LdsAudit& a) {
-    audit_one(k_band_fwd<T, D, 32, false>, "k_band_fwd", a);
-    audit_one(k_band_fwd<T, D, 32, true>, "k_band_fwd", a);
-    audit_one(k_band_bwd_q<T, D, 32, false>, "k_band_bwd_q", a);
-    audit_one(k_band_bwd_q<T, D, 32, true>, "k_band_bwd_q", a);
-    audit_one(k_band_bwd_kv<T, D, 32, false>, "k_band_bwd_kv", a);
-    audit_one(k_band_bwd_kv<T, D, 32, true>, "k_band_bwd_kv", a);
+    audit_one(k_band_fwd<T, D, false>, "k_band_fwd", a);
+    audit_one(k_band_fwd<T, D, true>, "k_band_fwd", a);
+    audit_one(k_band_bwd_q<T, D, false>, "k_band_bwd_q", a);
+    audit_one(k_band_bwd_q<T, D, true>, "k_band_bwd_q", a);
+    audit_one(k_band_bwd_kv<T, D, false>, "k_band_bwd_kv", a);
+    audit_one(k_band_bwd_kv<T, D, true>, "k_band_bwd_kv", a);
 }
 
 // No static LDS in any instance (see lds_base): checked once per process.
@@ -877,7 +849,7 @@ hipError_t band_fwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
     a.ll = to_k(ll);
     a.ab = band_plane(p, lk, D);
     a.bb = band_plane(p, lv, D);
-    auto kern = two ? k_band_fwd<T, D, 32, true> : k_band_fwd<T, D, 32, false>;
+    auto kern = two ? k_band_fwd<T, D, true> : k_band_fwd<T, D, false>;
     const hipError_t e = allow_lds(kern, kBandLds<T, D>);
     if (e != hipSuccess) return e;
     NA_LAUNCH("na_fwd_band", kern, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
@@ -920,7 +892,7 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
     a.bb = band_plane(p, lv, D);
     hipError_t e;
     if (sides & kQuerySide) {
-        auto kq = two ? k_band_bwd_q<T, D, 32, true> : k_band_bwd_q<T, D, 32, false>;
+        auto kq = two ? k_band_bwd_q<T, D, true> : k_band_bwd_q<T, D, false>;
         if ((e = allow_lds(kq, kBandLds<T, D>)) != hipSuccess) return e;
         NA_LAUNCH("na_bwd_q_band", kq, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
                   (kBandLds<T, D>), s, a);
@@ -930,7 +902,7 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
     a.g = band_geo(p, band_columns(p.ax[2].k, true), p.Hkv);
     a.ab = band_plane(p, lq, D);
     a.bb = band_plane(p, ldo, D);
-    auto kk = two ? k_band_bwd_kv<T, D, 32, true> : k_band_bwd_kv<T, D, 32, false>;
+    auto kk = two ? k_band_bwd_kv<T, D, true> : k_band_bwd_kv<T, D, false>;
     if ((e = allow_lds(kk, kBandLdsKv<T, D>)) != hipSuccess) return e;
     NA_LAUNCH("na_bwd_kv_band", kk, dim3(static_cast<unsigned>(band_blocks(p, a.g))), dim3(kBandThreads),
               (kBandLdsKv<T, D>), s, a);
