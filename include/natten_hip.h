@@ -255,6 +255,14 @@ int natten_hip_neighborhood_map(const natten_problem_t *p,
                                 int64_t *flat, uint8_t *valid,
                                 void *stream);
 
+/* The lens array of the variable-length entry points below from host memory:
+ * writes the device int32 [batch][3] at lens from sizes, host int32
+ * [batch][rank] (rank 1, 2 or 3; the padded leading axes become 1).  The
+ * values travel as kernel arguments: the host copy may be reused at once, and
+ * nothing waits. */
+int natten_hip_varlen_extents(const int32_t *sizes, int32_t batch, int32_t rank,
+                              int32_t *lens, void *stream);
+
 /* Variable-length fused forward / backward.  The problem describes the
  * padded (maximum) extents, stride 1; lens (device memory, int32 [batch][3],
  * padded axes first as in `length`) holds each sample's own extent per axis,
@@ -264,13 +272,6 @@ int natten_hip_neighborhood_map(const natten_problem_t *p,
  * A sample whose extents are out of range (or an even kernel equal to its
  * extent, non-causal, dilation 1) comes out all zero.  Other arguments as for
  * natten_hip_forward / natten_hip_backward. */
-/* The lens array of these entry points from host memory: writes the device
- * int32 [batch][3] at lens from sizes, host int32 [batch][rank] (rank 1, 2
- * or 3; the padded leading axes become 1).  The values travel as kernel
- * arguments: the host copy may be reused at once, and nothing waits. */
-int natten_hip_varlen_extents(const int32_t *sizes, int32_t batch, int32_t rank,
-                              int32_t *lens, void *stream);
-
 int natten_hip_varlen_forward(const natten_problem_t *p, const int32_t *lens,
                               const void *q, const natten_layout_t *lq,
                               const void *k, const natten_layout_t *lk,
