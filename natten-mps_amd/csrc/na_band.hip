@@ -926,12 +926,12 @@ hipError_t band_bwd_run(const Prob& p, const void* q, Lay lq, const void* k, Lay
 // kernel of 2 to 16 columns (so that a tile's union fits 32), and
 // * both sides for 10 to 16 columns (past the 8x8 tile kernels), and at head
 //   dim 128 from 8: there the general tiles' border unions cross 16 columns
-//   and their rows double (9 x 9, 8 x 64 x 64 x 4 heads: forward 97 -> 61
-//   us, the backward left the tiles, 995 + 950 -> 129 + 117 us; at 7 x 7 both
+//   and their rows double (9 x 9, 8 x 64 x 64 x 4 heads: forward 97 -> 54
+//   us, the backward left the tiles, 995 + 950 -> 124 + 111 us; at 7 x 7 both
 //   are level, 57 + 76 + 90 against 58 + 99 + 87);
 // * the key side alone where the 8x8 tiles serve the query side but some key
 //   tile's union does not fit them (`lean`: they take the problem; 9 x 9, 8 x
-//   64 x 64 x 8: dK/dV 222 -> 56 us at head dim 32, 613 -> 111 at 64; 7 x 7
+//   64 x 64 x 8: dK/dV 222 -> 49 us at head dim 32, 613 -> 107 at 64; 7 x 7
 //   on 32 x 22 x 22 x 8: 57 -> 37).
 // Where the general tiles hold the problem too, band_pays decides per kernel.
 // Where the general tiles cannot hold the problem either, the alternative is
